@@ -1,7 +1,6 @@
-// Grouped routed-expert FFN for many tokens (prefill) on native MXFP4 MFMA: every routed
-// (token, slot) pair is grouped by expert and each expert runs as a GEMM with M = its token
-// count, so each expert's MXFP4 weights stream from HBM once per 64-row tile instead of
-// once per token.
+// Grouped routed-expert FFN for many tokens (prefill): every routed (token, slot) pair is
+// grouped by expert and each expert runs as a GEMM with M = its token count on the bf16
+// matrix cores, so each expert's MXFP4 weights stream from HBM once.
 //
 // Reference: LatentMoE.__call__ (air_llm/models/kimi_k3/moe.py:110-132; k3ref
 // k3ref/layers.py:241-261): for each distinct routed expert, gather its tokens, run
@@ -10,38 +9,18 @@
 //
 //   count    block e counts the pairs routed to expert e                      -> counts[E]
 //   plan     one block: exclusive scan of the counts (segment bases) and the list of
-//            64-row tiles (expert, first row) of every non-empty expert
+//            64-row tiles of every non-empty expert
 //   place    block e writes its pairs, in (token, slot) order, into perm[base_e ...]
-//   quant_x  x -> E4M3 terms, one E8M0 scale per 32 elements per term: bf16 x as two,
-//            x = 2^e1 t1 + 2^e2 t2, exact for every element within 2^13 of its block's max;
-//            fp32 x as three (about 12 bits, as act)
-//   gateup   block (tile, 128 intermediate indices): v_mfma_scale_f32_16x16x128_f8f6f4 with
-//            the expert's MXFP4 rows as the FP4 A operand and their E8M0 bytes as the A
-//            scales (no decode), the x terms as the FP8 B operand; act = f(gate, up) in
-//            fp32, split in registers into three E4M3 terms per 32 (about 12 bits)
-//   down     block (tile, 256 output rows): the same MFMA over the three act terms
+//   split_x  (fp32 x only) x -> two bf16 terms, hi + lo, about 16 significant bits
+//   gateup   block (tile, 128 intermediate indices): gate and up rows against the tile's
+//            tokens; act = f(gate, up) in fp32, stored as two bf16 terms (16 bits)
+//   down     block (tile, 256 output rows): the same against the two act terms
 //            -> fp32 rows per (token, slot) pair
 //   combine  y[t] = sum_slot w[t, slot] * y_pair[t, slot], slots in order
 //
-// Deterministic: no atomics, fixed summation orders everywhere.
-//
-// Operand layout of v_mfma_scale_f32_16x16x128_f8f6f4 with FP4 A (cbsz 4) and FP8 E4M3 B
-// (blgp 0), as measured on gfx950:
-//   A   lane l: weight row l%16, the 32 elements of K block l/16 (of the instruction's 128),
-//       element j in nibble j, low nibble first -- the MXFP4 byte order, loaded verbatim
-//   B   lane l: column l%16; with g = l/16, bytes 0-15 hold elements 16(g%2)..16(g%2)+15 of
-//       K block g/2 and bytes 16-31 the same elements of K block 2+g/2
-//   scale_a / scale_b of lane l: row / column l%16, K block l/16; op_sel picks the byte
-//   C   lane l, register v: row 4(l/16)+v, column l%16
-// The 128-element dot is accumulated about 12 bits below its largest product (unbiased
-// rounding, measured), then added into the fp32 C.
-//
-// K runs in super-steps of 256: a lane's 32-byte A load covers blocks 2q, 2q+1 (q = l/16)
-// and MFMA m in {0, 1} uses block 2q+m, so MFMA m's K block q' is super-step block 2q'+m.
-// B rows are therefore stored in "MX-B" order: per super-step, sixteen 16-byte pieces
-// p = (m*2 + h)*4 + g, piece p holding elements 16(g%2)..+15 of block 4h + 2(g/2) + m.  The
-// B operand of (m, lane) is then pieces (m, h=0, g) and (m, h=1, g) of its row, and its
-// scale is byte 2g+m of the row's eight block scales (natural order).
+// Numerics: an E2M1 code times its E8M0 scale is a bf16 value, so the weights enter the
+// bf16 MFMA exactly; bf16 x is exact, and fp32 operands keep 16 bits in two terms.  Products
+// are exact and accumulate in fp32.  Deterministic: no atomics, fixed summation orders.
 #include <algorithm>
 
 #include "k3_common.h"
@@ -50,11 +29,7 @@
 namespace k3 {
 namespace {
 
-constexpr int kTM = 64;        // grouped rows (tokens) per tile: four 16-column B tiles
-constexpr int kSS = 256;       // K elements per super-step
-constexpr int kThreads = 256;  // 4 waves
-
-typedef int i32x8 __attribute__((ext_vector_type(8)));
+constexpr int kTM = 64;        // grouped rows (tokens) per tile: four 16-column MFMA tiles
 
 struct GroupArgs {
     const int32_t *idx;    // [P] expert id of pair p = t * k + slot
@@ -62,8 +37,7 @@ struct GroupArgs {
     int32_t *counts;       // [E]
     int32_t *base;         // [E]
     int32_t *perm;         // [P]: pairs grouped by expert
-    int32_t *tile_e;       // [max_tiles]
-    int32_t *tile_m0;      // [max_tiles]
+    int4 *tiles;           // [max_tiles]: (expert, its first tile, its pairs, its first grouped row)
     int32_t *n_tiles;      // [1]
     int max_tiles;
 };
@@ -142,440 +116,361 @@ __global__ __launch_bounds__(1024) void group_plan_kernel(GroupArgs g) {
     if (e < g.E) {
         g.base[e] = sc[e] - c;
         const int t0 = st[e] - (c + kTM - 1) / kTM;
-        for (int j = 0; j * kTM < c; ++j) {
-            if (t0 + j < g.max_tiles) {
-                g.tile_e[t0 + j] = e;
-                g.tile_m0[t0 + j] = j * kTM;
-            }
-        }
+        for (int j = 0; j * kTM < c; ++j)
+            if (t0 + j < g.max_tiles) g.tiles[t0 + j] = make_int4(e, t0, c, sc[e] - c);
     }
     if (e == 1023) *g.n_tiles = min(st[1023], g.max_tiles);
 }
 
-// ------------------------------------------------------------------ E4M3 / E8M0 terms
-// Exponent e of the block scale 2^e for a block whose largest magnitude is amax, chosen so
-// amax / 2^e lies in [128, 256) (below E4M3's 448); clamped to the E8M0 range.
-__device__ __forceinline__ int block_exp(float amax) {
-    const int ea = static_cast<int>((__float_as_uint(amax) >> 23) & 0xffu) - 127;
-    return max(ea - 7, -127);
+// ------------------------------------------------------------------ bf16 terms
+// hi + lo of an fp32 value: hi rounded to nearest, lo the rounded remainder (zero where hi
+// is not finite, so an infinity stays one).
+__device__ __forceinline__ void bf16_split2(float v, uint16_t &hi, uint16_t &lo) {
+    hi = f32_to_bf16(v);
+    const float h = bf16_to_f32(hi);
+    lo = (hi & 0x7f80u) == 0x7f80u ? 0 : f32_to_bf16(v - h);
 }
 
-// E4M3 (OCP, bias 7) code of x, |x| < 256, rounded to nearest even; q receives its value.
-__device__ __forceinline__ uint32_t e4m3_rne(float x, float &q) {
-    const float a = fabsf(x);
-    uint32_t code;
-    float v;
-    if (a < 0.015625f) {  // subnormals: multiples of 2^-9 (rounding up to 8 gives 2^-6, code 8)
-        const float m = rintf(a * 512.f);
-        code = static_cast<uint32_t>(m);
-        v = m * 0.001953125f;
-    } else {              // normals: keep 3 mantissa bits, the carry runs into the exponent
-        uint32_t b = __float_as_uint(a);
-        b += 0x7ffffu + ((b >> 20) & 1u);
-        b &= 0xfff00000u;
-        v = __uint_as_float(b);
-        code = (b >> 20) - 960u;  // ((exp - 127 + 7) << 3) | mantissa
-    }
-    const uint32_t s = __float_as_uint(x) >> 31;
-    q = s ? -v : v;
-    return code | (s << 7);
-}
+// A two-term row: per 128 elements, 128 hi values then 128 lo values (512 bytes), so one
+// staging step of the GEMM reads 512 contiguous bytes per row in either form.
+constexpr int kBlk = 128;
 
-// Byte offset, inside one row in MX-B order, of the 16-element half `half` of K block b.
-__device__ __forceinline__ uint32_t mxb_offset(uint32_t b, uint32_t half) {
-    const uint32_t bb = b & 7u, m = bb & 1u, h = bb >> 2, g = ((bb >> 1) & 1u) * 2u + half;
-    return (b >> 3) * kSS + ((m * 2u + h) * 4u + g) * 16u;
-}
-
-__device__ __forceinline__ float shfl_xor_f(float v, int m) { return __shfl_xor(v, m, 64); }
-
-// ------------------------------------------------------------------ quant_x
-struct QxArgs {
-    const void *x;        // [T, H] bf16 (two terms) or fp32 (three terms)
-    uint8_t *x8;          // [TERMS][T][Hpad] E4M3 codes, MX-B order
-    uint8_t *xs;          // [TERMS][T][Hpad / 32] E8M0
-    int T, H, Hpad;
-    uint32_t term, sterm; // bytes per term of x8 / xs
+struct SplitArgs {
+    const float *x;      // [T, H]
+    uint16_t *xt;        // [T][Hblk][2][128]
+    int T, H, Hblk;
 };
 
-// One thread per 16-element half block; the two halves of a block are adjacent lanes.
-// bf16 x is the exact sum of its two terms; fp32 x keeps about 12 bits in three (as act).
-template <bool F32>
-__global__ __launch_bounds__(256) void quant_x_kernel(QxArgs a) {
-    constexpr int TERMS = F32 ? 3 : 2;
-    const int halves = a.H >> 4;
-    const int idx = blockIdx.x * 256 + threadIdx.x;
-    const bool ok = idx < a.T * halves;
-    const int t = ok ? idx / halves : 0, hh = ok ? idx % halves : 0;
-    float v[16];
-    if (ok && F32) {
-        const float4 *src = reinterpret_cast<const float4 *>(static_cast<const float *>(a.x) +
-                                                             static_cast<int64_t>(t) * a.H + hh * 16);
+__global__ __launch_bounds__(256) void split_x_kernel(SplitArgs a) {
+    const int eighths = a.H >> 3;
+    const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (idx >= static_cast<int64_t>(a.T) * eighths) return;
+    const int64_t t = idx / eighths;
+    const int k = static_cast<int>(idx % eighths) * 8;
+    const float4 *src = reinterpret_cast<const float4 *>(a.x + t * a.H + k);
+    const float4 f0 = src[0], f1 = src[1];
+    const float v[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
+    uint32_t hi[4], lo[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float4 f = src[i];
-            v[4 * i] = f.x, v[4 * i + 1] = f.y, v[4 * i + 2] = f.z, v[4 * i + 3] = f.w;
-        }
-    } else if (ok) {
-        const uint4 *src = reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(a.x) +
-                                                           static_cast<int64_t>(t) * a.H + hh * 16);
-        const uint4 u0 = src[0], u1 = src[1];
-        const uint32_t w[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            v[2 * i] = __uint_as_float(w[i] << 16);
-            v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = 0.f;
+    for (int i = 0; i < 4; ++i) {
+        uint16_t h0, l0, h1, l1;
+        bf16_split2(v[2 * i], h0, l0);
+        bf16_split2(v[2 * i + 1], h1, l1);
+        hi[i] = h0 | (static_cast<uint32_t>(h1) << 16);
+        lo[i] = l0 | (static_cast<uint32_t>(l1) << 16);
     }
-    const uint32_t row8 = static_cast<uint32_t>(t) * a.Hpad + mxb_offset(hh >> 1, hh & 1);
-    const uint32_t rows = static_cast<uint32_t>(t) * (a.Hpad >> 5) + (hh >> 1);
-#pragma unroll
-    for (int term = 0; term < TERMS; ++term) {
-        float amax = 0.f;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(v[i]));
-        amax = fmaxf(amax, shfl_xor_f(amax, 1));
-        const int e = block_exp(amax);
-        uint32_t c[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            float q;
-            c[i >> 2] |= e4m3_rne(ldexpf(v[i], -e), q) << (8 * (i & 3));
-            v[i] -= ldexpf(q, e);
-        }
-        if (ok) {
-            *reinterpret_cast<uint4 *>(a.x8 + term * a.term + row8) = make_uint4(c[0], c[1], c[2], c[3]);
-            if ((hh & 1) == 0) a.xs[term * a.sterm + rows] = static_cast<uint8_t>(e + 127);
-        }
-    }
+    uint16_t *dst = a.xt + (t * a.Hblk + (k >> 7)) * (2 * kBlk) + (k & 127);
+    *reinterpret_cast<uint4 *>(dst) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+    *reinterpret_cast<uint4 *>(dst + kBlk) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
 }
 
-// ------------------------------------------------------------------ grouped MFMA GEMMs
-struct MxArgs {
-    const uint8_t *b8;       // B terms [TERMS][rows][Kpad], MX-B order
-    const uint8_t *bs;       // B scales [TERMS][rows][Kpad / 32]
-    uint32_t b_term, bs_term;
+// ------------------------------------------------------------------ grouped GEMMs
+struct GemmArgs {
+    const void *b;           // B rows: bf16 x [T, K], or two-term rows [., Kblk, 2, 128]
+    uint32_t b_bytes;        // size of all B rows (gate/up)
+    uint32_t brow;           // bytes per B row
     const uint64_t *table;   // [E][6] expert pointers
-    const int32_t *counts, *base, *perm, *tile_e, *tile_m0, *n_tiles;
-    uint8_t *a8, *as;        // gate/up output: act terms [3][P][Ipad], scales [3][P][Ipad / 32]
-    uint32_t a_term, as_term;
-    int Ipad;
-    float *ypair;            // down output [P, H]: row = pair id
-    int K, Kpad, N;          // reduction length, its padded row length, weight rows of one projection
-    int NT, tile_major;      // weight-row blocks; block order (see mx_gemm_kernel)
-    int top_k, max_tiles, act_kind;
+    const int32_t *perm, *n_tiles;
+    const int4 *tiles;
+    uint16_t *act;           // gate/up output: two-term rows [P, Iblk, 2, 128]
+    uint32_t act_row;        // bytes per act row
+    float *ypair;            // down output [P, N]: row = pair id
+    int K, N, NT;            // reduction length, weight rows of one projection, row blocks
+    int top_k, act_kind;
     float beta, lbeta;
 };
 
-template <int M>
-__device__ __forceinline__ f32x4 mfma_fp4_fp8(const uint4 &a, const uint4 &b0, const uint4 &b1, f32x4 c,
-                                              uint32_t sa, uint32_t sb) {
-    const i32x8 av = {static_cast<int>(a.x), static_cast<int>(a.y), static_cast<int>(a.z), static_cast<int>(a.w),
-                      0, 0, 0, 0};
-    const i32x8 bv = {static_cast<int>(b0.x), static_cast<int>(b0.y), static_cast<int>(b0.z), static_cast<int>(b0.w),
-                      static_cast<int>(b1.x), static_cast<int>(b1.y), static_cast<int>(b1.z), static_cast<int>(b1.w)};
-    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, c, 4, 0, M, static_cast<int>(sa), M,
-                                                            static_cast<int>(sb));
+// The GEMM streams weights, so it is bound by HBM as long as the operands reach the matrix
+// cores without extra traffic.  What decides that on this chip is the lane order of the
+// loads: adjacent lanes on one 128-byte line reach 48 B/clk per CU from L2, while the MFMA
+// operand order loaded straight from memory (adjacent lanes on different rows) makes one
+// L1 request per lane and stops at 16 B/clk per CU.  So every operand is loaded
+// line-contiguous into registers, two steps ahead, and turned into operand order through
+// LDS, in 16-byte chunks XOR-swizzled by the row so neither the stores nor the operand
+// reads meet bank conflicts:
+//   A  256 weight rows x 256 elements (128 bytes a row: one line), double buffered
+//   B  64 token rows x 512 bytes (256 elements, or 128 of two terms), double buffered
+//   S  256 rows x 32 scale bytes, one load per four steps, double buffered
+// 144 KB of LDS, one block of eight waves per CU.  Waves w and w + 4 own the same 64 weight
+// rows and split the reduction (their sums meet in LDS at the end), so no wave converts or
+// reads what another one does.  Weights become bf16 in registers (4 v_cvt per 8 values of
+// a row, reused by the tile's column groups and both terms).
+// Measured (2048 tokens, 896 experts top-16, latent 3584 / 3072): @@GU@@
+constexpr int kThreads = 512;
+constexpr uint32_t kOob = 0xf0000000u;      // past every buffer size the host lets through
+constexpr int kABuf = 256 * 128, kBBuf = 64 * 512, kSBuf = 256 * 32;
+constexpr int kLdsB = 2 * kABuf, kLdsS = kLdsB + 2 * kBBuf;
+constexpr int kLds = kLdsS + 2 * kSBuf;
+
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ bf16x8 fp4x8_bf16(uint32_t w, float s) {
+    const uint4 v = make_uint4(__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, s, 0)),
+                               __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, s, 1)),
+                               __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, s, 2)),
+                               __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, s, 3)));
+    return __builtin_bit_cast(bf16x8, v);
 }
 
-// DOWN == false: gate/up + activation.  Wave w owns the 32 intermediate indices
-// [i0 + 32 w, +32): A tiles j = 0, 1 are their gate rows and j = 2, 3 their up rows, so the
+// DOWN == false: gate/up + activation; A rows 0..127 of the block are gate rows, 128..255
+// the up rows of the same intermediate indices, and wave w % 4 owns 32 of both, so the
 // activation of a (token, index) pair meets both products in one lane.
-// DOWN == true: wave w owns 64 output rows [n0 + 64 w, +64) of W_down, B = the act terms.
-// TERMS: E4M3 terms of B (x: 2 for bf16, 3 for fp32; act: 3).
-template <bool DOWN, int TERMS>
-__global__ __launch_bounds__(kThreads, 1) void mx_gemm_kernel(MxArgs a) {
-    // two LDS tiles of B: [buffer][ct][term][piece][column] 16-byte pieces, then
-    // [buffer][ct][term][column][block pair] scale pairs
-    extern __shared__ uint4 smem[];
-    constexpr int kXT = 4 * TERMS * 16 * 16;  // uint4 per tile
-    constexpr int kST = 4 * TERMS * 16 * 4;   // uint16 per scale tile
-    uint16_t *const ssm = reinterpret_cast<uint16_t *>(smem + 2 * kXT);
-
+// DOWN == true: 256 rows of W_down, 64 per wave.
+// TERMS: bf16 terms of B (bf16 x: 1; fp32 x and act: 2).  NCT: 16-column groups in use.
+template <bool DOWN, int TERMS, int NCT>
+__device__ __forceinline__ void grouped_tile(const GemmArgs &a, char *lds, int nt, int rows, int pos0,
+                                             const uint64_t *ptr) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // Block order (block b runs on XCD b % 8).  Row-block major (gate/up): consecutive blocks
-    // on one XCD take consecutive tiles of one weight-row block, so the tiles of a hot expert
-    // stream the same weight rows together and share them in L2.  Tile major (down): XCD x
-    // owns tiles x, x + 8, ... and runs all row blocks of one tile together, so they share
-    // that tile's B rows (its act terms) in L2.  Measured on the 2048-token Zipf prefill:
-    // tile major is 8% faster for down and 5-12% slower for gate/up, where a hot expert's
-    // weight rows then stream once per XCD; groups of several tiles x row blocks per XCD were
-    // slower for both.
-    int tile, nt;
-    if (a.tile_major) {
-        const int li = blockIdx.x >> 3;
-        tile = (blockIdx.x & 7) + 8 * (li / a.NT), nt = li % a.NT;
-    } else {
-        const int nb = static_cast<int>(gridDim.x);
-        const int w = (nb & 7) == 0 ? (blockIdx.x & 7) * (nb >> 3) + (blockIdx.x >> 3) : blockIdx.x;
-        tile = w % a.max_tiles, nt = w / a.max_tiles;
-    }
-    if (tile >= *a.n_tiles || nt >= a.NT) return;
-    const int e = a.tile_e[tile], m0 = a.tile_m0[tile];
-    const int rows = min(kTM, a.counts[e] - m0);
-    const int pos0 = a.base[e] + m0;  // grouped row of the tile's first token
-    const int nct = (rows + 15) >> 4;
-    const uint64_t *ptr = a.table + static_cast<int64_t>(e) * 6;
-    const int KB = a.K >> 5;
-    const int NS = a.Kpad / kSS;
+    const int wr = wave & 3, kg = wave >> 2;
     const int r16 = lane & 15, q = lane >> 4;
+    const int KB = a.K >> 5;                     // 32-element groups per weight row
+    const int NS = (a.K + 255) >> 8;
 
-    // ---- A: four 16-row tiles per wave, 32 bytes + 2 scale bytes per lane per super-step,
-    // in a ring of four super-steps (loads run three super-steps ahead of their MFMAs)
+    // ---- loads: A and S by wave w for block rows 32 w .. + 31, B for token rows 8 w .. + 7
+    const int proj = DOWN ? 4 : (wave < 4 ? 0 : 2);
     const uint32_t rowA = static_cast<uint32_t>(a.K >> 1);
-    __amdgpu_buffer_rsrc_t ra[2], rsa[2];
-    {
-        const int p0 = DOWN ? 4 : 0;
-        ra[0] = make_rsrc(reinterpret_cast<const void *>(ptr[p0]), static_cast<uint32_t>(a.N) * rowA);
-        rsa[0] = make_rsrc(reinterpret_cast<const void *>(ptr[p0 + 1]), static_cast<uint32_t>(a.N * KB));
-        ra[1] = DOWN ? ra[0] : make_rsrc(reinterpret_cast<const void *>(ptr[2]), static_cast<uint32_t>(a.N) * rowA);
-        rsa[1] = DOWN ? rsa[0] : make_rsrc(reinterpret_cast<const void *>(ptr[3]), static_cast<uint32_t>(a.N * KB));
-    }
-    uint32_t aoff[4], asoff[4];
+    const auto ra = make_rsrc(uniform_ptr(ptr[proj]), static_cast<uint32_t>(a.N) * rowA);
+    const void *sbase = uniform_ptr(ptr[proj + 1]);
+    const auto rs = make_rsrc(sbase, static_cast<uint32_t>(a.N * KB));
+    const bool s_al = ((reinterpret_cast<uintptr_t>(sbase) | static_cast<uintptr_t>(KB)) & 3u) == 0;
+    const int grow0 = DOWN ? nt * 256 + wave * 32 : nt * 128 + (wave & 3) * 32;  // weight row of block row 32 w
+    const int ac = lane & 7;                     // 16-byte chunk of the 128-byte line
+    uint32_t aoff[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int row = DOWN ? nt * 256 + wave * 64 + j * 16 + r16 : nt * 128 + wave * 32 + (j & 1) * 16 + r16;
-        const bool ok = row < a.N;
-        aoff[j] = ok ? static_cast<uint32_t>(row) * rowA + 32u * q : kOobOffset;
-        asoff[j] = ok ? static_cast<uint32_t>(row * KB + 2 * q) : kOobOffset;
+    for (int n = 0; n < 4; ++n) {
+        const int row = grow0 + 8 * n + (lane >> 3);
+        aoff[n] = row < a.N ? static_cast<uint32_t>(row) * rowA + ac * 16u : kOob;
     }
-    constexpr int kRing = 4;
-    uint4 A[kRing][4][2];
-    uint16_t SA[kRing][4];  // widened only where used, so no VALU op waits on the load early
-    // Super-steps past the end load as zeros (block index >= KB), so every step issues the
-    // same loads and the waits stay exact.  Invalid offsets keep bit 31 set (every valid
-    // offset is below 2^31), OR-ed in without branches.
-    auto load_a = [&](int S, int slot) {
-        const uint32_t oob = S * 8 + 2 * q < KB ? 0u : kOobOffset;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t off = (aoff[j] + S * 128u) | oob;
-            A[slot][j][0] = buf_load16(ra[j >> 1], off);
-            A[slot][j][1] = buf_load16(ra[j >> 1], off + 16u);
-            SA[slot][j] = __builtin_amdgcn_raw_buffer_load_b16(rsa[j >> 1], (asoff[j] + S * 8u) | oob, 0, 0);
-        }
-    };
-
-    // ---- B staging.  Gate/up (x terms, gathered from memory): thread (column c = tid >> 4,
-    // piece p = tid & 15) copies piece p of tile row c of every 16-column tile and term, so
-    // one wave instruction reads four whole rows' 256-byte super-step runs (whole 128-byte
-    // lines; the loads of 16 rows x 64 bytes they replace measured 5% slower), and the LDS
-    // tile keeps [piece][column] order for the operand reads with the column XOR-ed by the
-    // piece, so neither the stores nor the reads meet bank conflicts.  Down (act terms, just
-    // written and in cache): thread (c = tid & 15, p = tid >> 4), plain order (the line-wise
-    // form measured 3-7% slower there).  (c = tid & 15, block pair g = (tid >> 4) & 3, tile
-    // tid >> 6) copies one scale pair per term.  Two register sets: loads run two super-steps
-    // ahead of their LDS stores.
-    constexpr bool kLines = !DOWN;
-    const auto rb = make_rsrc(a.b8, a.b_term * TERMS);
-    const auto rbs = make_rsrc(a.bs, a.bs_term * TERMS);
-    const int dc = kLines ? tid >> 4 : tid & 15, dp = kLines ? tid & 15 : tid >> 4;
-    // LDS unit (16 bytes) of piece pc of column c within one tile and term
-    auto bunit = [](int pc, int c) { return pc * 16 + (kLines ? c ^ pc : c); };
-    const int dp_bb = 4 * ((dp >> 2) & 1) + 2 * ((dp & 3) >> 1) + (dp >> 3);  // block of piece dp
+    const int srow = grow0 + (lane >> 1);
+    const uint32_t soff = srow < a.N ? static_cast<uint32_t>(srow * KB) + (lane & 1) * 16u : kOob;
+    const auto rb = DOWN ? make_rsrc(static_cast<const char *>(a.b) + static_cast<int64_t>(pos0) * a.brow,
+                                     static_cast<uint32_t>(rows) * a.brow)
+                         : make_rsrc(a.b, a.b_bytes);
+    const int bc = lane & 31;                    // 16-byte chunk of the 512 bytes
     uint32_t boff[4];
 #pragma unroll
-    for (int ct = 0; ct < 4; ++ct) {
-        const int rr = ct * 16 + dc;
-        int brow = -1;
-        if (rr < rows) brow = DOWN ? pos0 + rr : a.perm[pos0 + rr] / a.top_k;
-        boff[ct] = brow >= 0 ? static_cast<uint32_t>(brow) * a.Kpad + dp * 16u : kOobOffset;
+    for (int n = 0; n < 4; ++n) {
+        const int rr = wave * 8 + 2 * n + (lane >> 5);
+        boff[n] = kOob;
+        if (rr < rows) boff[n] = static_cast<uint32_t>(DOWN ? rr : a.perm[pos0 + rr] / a.top_k) * a.brow + bc * 16u;
     }
-    const int sc_c = tid & 15, sg = (tid >> 4) & 3, sct = tid >> 6;
-    uint32_t bsoff;
-    {
-        const int rr = sct * 16 + sc_c;
-        int brow = -1;
-        if (rr < rows) brow = DOWN ? pos0 + rr : a.perm[pos0 + rr] / a.top_k;
-        bsoff = brow >= 0 ? static_cast<uint32_t>(brow) * (a.Kpad >> 5) + 2u * sg : kOobOffset;
-    }
-    // gate/up stages bf16 x's two terms two super-steps ahead (gathered token rows); down,
-    // whose act terms were written just before and sit in cache, and gate/up over fp32 x's
-    // three terms, one step ahead, to stay in registers
-    constexpr int XD = (DOWN || TERMS == 3) ? 1 : 2;
-    uint4 XR[XD][4][TERMS];
-    uint16_t XS[XD][TERMS];
-    auto load_x = [&](int S, int xs) {
-        const uint32_t poob = S >= 0 && S * 8 + dp_bb < KB ? 0u : kOobOffset;
-        const uint32_t soob = S >= 0 && S * 8 + 2 * sg < KB ? 0u : kOobOffset;
+    uint4 RA[2][4], RB[2][4], RS;
+    auto load_a = [&](int S, int set) {
+        const bool ok = S * 8 + ac < KB;
 #pragma unroll
-        for (int ct = 0; ct < 4; ++ct)
-#pragma unroll
-            for (int t = 0; t < TERMS; ++t)
-                XR[xs][ct][t] = buf_load16(rb, (boff[ct] + t * a.b_term + S * kSS) | poob);
-#pragma unroll
-        for (int t = 0; t < TERMS; ++t)
-            XS[xs][t] = __builtin_amdgcn_raw_buffer_load_b16(rbs, (bsoff + t * a.bs_term + S * 8u) | soob, 0, 0);
+        for (int n = 0; n < 4; ++n) RA[set][n] = buf_load16(ra, ok ? aoff[n] + S * 128u : kOob);
     };
-    auto store_x = [&](int xs, int buf) {
-        uint4 *xt = smem + buf * kXT;
-        uint16_t *st = ssm + buf * kST;
+    auto load_b = [&](int u, int set) {
+        const bool ok = TERMS == 1 ? u * 32 + bc < (a.K >> 3) : u * 16 + (bc & 15) < (a.K >> 3);
 #pragma unroll
-        for (int ct = 0; ct < 4; ++ct)
-#pragma unroll
-            for (int t = 0; t < TERMS; ++t) xt[(ct * TERMS + t) * 256 + bunit(dp, dc)] = XR[xs][ct][t];
-#pragma unroll
-        for (int t = 0; t < TERMS; ++t) st[((sct * TERMS + t) * 16 + sc_c) * 4 + sg] = XS[xs][t];
+        for (int n = 0; n < 4; ++n) RB[set][n] = buf_load16(rb, ok ? boff[n] + u * 512u : kOob);
     };
+    auto load_s = [&](int G) {
+        const uint32_t off = soff + G * 32u;
+        if (s_al) {
+            RS = buf_load16(rs, off);
+        } else {  // scale rows of any alignment, byte by byte
+            uint32_t w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                w[i >> 2] |= static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b8(rs, off + i, 0, 0)) << (8 * (i & 3));
+            RS = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+    };
+    auto store_a = [&](int set, int buf) {
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            const int R = wave * 32 + 8 * n + (lane >> 3);
+            *reinterpret_cast<uint4 *>(lds + buf * kABuf + R * 128 + ((ac ^ (R & 7)) << 4)) = RA[set][n];
+        }
+    };
+    auto store_b = [&](int set, int buf) {
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            const int rr = wave * 8 + 2 * n + (lane >> 5);
+            if (NCT == 4 || rr < NCT * 16)
+                *reinterpret_cast<uint4 *>(lds + kLdsB + buf * kBBuf + rr * 512 + ((bc ^ (rr & 7)) << 4)) = RB[set][n];
+        }
+    };
+    auto store_s = [&](int buf) { *reinterpret_cast<uint4 *>(lds + kLdsS + buf * kSBuf + tid * 16) = RS; };
 
-    f32x4 acc[4][4];  // [A tile j][B tile ct]
+    f32x4 acc[4][NCT];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int ct = 0; ct < 4; ++ct) acc[j][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int ct = 0; ct < NCT; ++ct) acc[j][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+    int arow[4];                                 // block row of this lane in each 16-row tile
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        arow[j] = (DOWN ? wr * 64 + j * 16 : (j >> 1) * 128 + wr * 32 + (j & 1) * 16) + r16;
 
-    // MFMAs of one super-step.  B fragments are read from LDS one 16-column tile ahead of
-    // their MFMAs, two sets live; the scheduling fences keep the compiler from hoisting all
-    // four tiles' fragments at once (which costs ~128 registers and forces reuse of
-    // registers whose loads are still in flight).
-    auto compute = [&](int slot, int buf) {
-        const uint4 *xt = smem + buf * kXT;
-        const uint16_t *st = ssm + buf * kST;
+    // Lane (r16, q) holds weight row r16's 32-element group 4h + q of the step; MFMA i takes
+    // its elements 8i .. 8i + 7 (one dword), against the same elements of the tokens.  Wave
+    // group kg takes i = 2kg, 2kg + 1 in both forms, so bf16 x gives the sums that fp32 x
+    // with the same values gives.
+    auto compute = [&](int S, int h, int abuf, int bbuf) {
+        const char *A = lds + abuf * kABuf, *B = lds + kLdsB + bbuf * kBBuf;
+        const char *Sc = lds + kLdsS + ((S >> 2) & 1) * kSBuf + (S & 3) * 8 + 4 * h + q;
+        const bool live = S * 8 + 4 * h + q < KB;
+        constexpr int NI = 2;
+        uint32_t w[4][NI];
+        float sc[4];
 #pragma unroll
-        for (int ct = 0; ct < 4; ++ct) {
-            if (ct < nct) {
+        for (int j = 0; j < 4; ++j) {
+            const uint2 v = *reinterpret_cast<const uint2 *>(A + arow[j] * 128 + (((4 * h + q) ^ (arow[j] & 7)) << 4) + 8 * kg);
+            w[j][0] = v.x, w[j][1] = v.y;
+            const uint32_t b = *reinterpret_cast<const uint8_t *>(Sc + arow[j] * 32);
+            sc[j] = e8m0_to_f32(live ? b : 0u);
+        }
 #pragma unroll
-                for (int t = 0; t < TERMS; ++t) {
-                    const uint4 *xb = xt + (ct * TERMS + t) * 256;
-                    const uint32_t sb = st[((ct * TERMS + t) * 16 + r16) * 4 + q];
-                    const uint4 b00 = xb[bunit(q, r16)], b01 = xb[bunit(4 + q, r16)];
-                    const uint4 b10 = xb[bunit(8 + q, r16)], b11 = xb[bunit(12 + q, r16)];
+        for (int i = 0; i < NI; ++i) {
+            bf16x8 av[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) av[j] = fp4x8_bf16(w[j][i], sc[j]);
+#pragma unroll
+            for (int t = 0; t < TERMS; ++t) {
+                const int chunk = 16 * (TERMS == 1 ? h : t) + 4 * q + 2 * kg + i;
+#pragma unroll
+                for (int ct = 0; ct < NCT; ++ct) {
+                    const bf16x8 bv = *reinterpret_cast<const bf16x8 *>(B + (ct * 16 + r16) * 512 +
+                                                                        ((chunk ^ (r16 & 7)) << 4));
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
-                        acc[j][ct] = mfma_fp4_fp8<0>(A[slot][j][0], b00, b01, acc[j][ct], SA[slot][j], sb);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        acc[j][ct] = mfma_fp4_fp8<1>(A[slot][j][1], b10, b11, acc[j][ct], SA[slot][j], sb);
+                        acc[j][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[j], bv, acc[j][ct], 0, 0, 0);
                 }
             }
         }
     };
-    // Super-step S: MFMAs on LDS tile S % 2 and A slot S % 4; then A(S + 4) into the freed
-    // slot, B(S + 1) from registers into the other LDS tile, B(S + 1 + XD) into the freed
-    // registers.  The loop starts at S = -4 with the MFMAs skipped, so the pipeline fills
-    // through the same instruction stream as the steady state (a separate prologue leaves
-    // the loop entry with a different set of loads in flight, and the compiler's waits at the
-    // loop head then cover the worse of the two).
-    auto step = [&](int S, int slot, int par) {
-        __syncthreads();  // tile S is stored and every wave is done with tile S - 1
-        if (S >= 0) compute(slot, par);
-        load_a(S + kRing, slot);
-        store_x((par ^ 1) % XD, par ^ 1);
-        load_x(S + 1 + XD, (par ^ 1) % XD);
+
+    // ---- pipeline: step S computes on buffers S % 2 while step S + 1 is stored and steps
+    // S + 2, S + 3 are in flight
+    load_a(0, 0);
+    load_b(0, 0);
+    load_s(0);
+    load_a(1, 1);
+    load_b(1, 1);
+    store_a(0, 0);
+    store_b(0, 0);
+    store_s(0);
+    load_a(2, 0);
+    load_b(2, 0);
+    auto step = [&](int S, int P) {
+        const int nx = (P + 1) & 1;
+        if constexpr (TERMS == 1) {
+            __syncthreads();
+            store_a(nx, nx);
+            store_b(nx, nx);
+            if (P == 3) store_s(((S >> 2) + 1) & 1);
+            load_a(S + 3, nx);
+            load_b(S + 3, nx);
+            if (P == 0) load_s((S >> 2) + 1);
+            compute(S, 0, P & 1, P & 1);
+            compute(S, 1, P & 1, P & 1);
+        } else {
+            __syncthreads();
+            store_b(1, 1);
+            load_b(2 * S + 3, 1);
+            if (P == 0) load_s((S >> 2) + 1);
+            compute(S, 0, P & 1, 0);
+            __syncthreads();
+            store_a(nx, nx);
+            store_b(0, 0);
+            if (P == 3) store_s(((S >> 2) + 1) & 1);
+            load_a(S + 3, nx);
+            load_b(2 * S + 4, 0);
+            compute(S, 1, P & 1, 1);
+        }
     };
-#pragma unroll
-    for (int xs = 0; xs < XD; ++xs) {
-#pragma unroll
-        for (int ct = 0; ct < 4; ++ct)
-#pragma unroll
-            for (int t = 0; t < TERMS; ++t) XR[xs][ct][t] = make_uint4(0u, 0u, 0u, 0u);
-#pragma unroll
-        for (int t = 0; t < TERMS; ++t) XS[xs][t] = 0;
-    }
-    // Unrolled over the four ring slots, so slot and LDS-tile indices are compile-time.
-    static_assert(kRing == 4, "the loop below is unrolled over the four ring slots");
-    for (int S = -kRing; S < NS; S += 4) {
-        step(S, 0, 0);
-        if (S + 1 < NS) step(S + 1, 1, 1);
-        if (S + 2 < NS) step(S + 2, 2, 0);
-        if (S + 3 < NS) step(S + 3, 3, 1);
+    for (int S = 0; S < NS; S += 4) {
+        step(S, 0);
+        if (S + 1 < NS) step(S + 1, 1);
+        if (S + 2 < NS) step(S + 2, 2);
+        if (S + 3 < NS) step(S + 3, 3);
     }
 
-    // ---- epilogues (C: lane holds weight rows 4q + v of each A tile, column r16 of each B tile)
-    if constexpr (DOWN) {
+    // ---- the two wave groups' sums meet: group kg finishes column groups ct % 2 == kg and
+    // hands the others over through LDS
+    __syncthreads();
+    f32x4 *xch = reinterpret_cast<f32x4 *>(lds);
 #pragma unroll
-        for (int ct = 0; ct < 4; ++ct) {
-            const int rr = ct * 16 + r16;
-            if (ct < nct && rr < rows) {
-                const int pair = a.perm[pos0 + rr];
-                float *yrow = a.ypair + static_cast<int64_t>(pair) * a.N;
+    for (int ct = 0; ct < NCT; ++ct)
+        if ((ct & 1) != kg) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) xch[((wr * NCT + ct) * 4 + j) * 64 + lane] = acc[j][ct];
+        }
+    __syncthreads();
+    // (C: lane holds weight rows 4q + v of each A tile, column r16 of each column group)
+#pragma unroll
+    for (int ct = 0; ct < NCT; ++ct) {
+        const int rr = ct * 16 + r16;
+        if ((ct & 1) == kg && rr < rows) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[j][ct] += xch[((wr * NCT + ct) * 4 + j) * 64 + lane];
+            if constexpr (DOWN) {
+                float *yrow = a.ypair + static_cast<int64_t>(a.perm[pos0 + rr]) * a.N;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const int row = nt * 256 + wave * 64 + j * 16 + 4 * q;
+                    const int row = nt * 256 + wr * 64 + j * 16 + 4 * q;
                     if (row < a.N) *reinterpret_cast<float4 *>(yrow + row) = __builtin_bit_cast(float4, acc[j][ct]);
                 }
-            }
-        }
-    } else {
-        const int ib = nt * 128 + wave * 32;  // the wave's intermediate block
-        if (ib < a.N) {
-            const int blk = ib >> 5;
-            const uint32_t pbase = mxb_offset(blk, 0) + 4u * q;  // half 0; half 1 is 16 bytes on
+            } else if (nt * 128 + wr * 32 < a.N) {
+                uint16_t *dst = reinterpret_cast<uint16_t *>(reinterpret_cast<char *>(a.act) +
+                                                             static_cast<int64_t>(pos0 + rr) * a.act_row) +
+                                nt * (2 * kBlk) + wr * 32 + 4 * q;
 #pragma unroll
-            for (int ct = 0; ct < 4; ++ct) {
-                if (ct < nct) {
-                    const int rr = ct * 16 + r16;
-                    const bool ok = rr < rows;
-                    float v[2][4];
-                    float amax = 0.f;
+                for (int j = 0; j < 2; ++j) {
+                    uint16_t hi[4], lo[4];
 #pragma unroll
-                    for (int j = 0; j < 2; ++j)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            v[j][i] = act_fn(acc[j][ct][i], acc[j + 2][ct][i], a.act_kind, a.beta, a.lbeta);
-                            amax = fmaxf(amax, fabsf(v[j][i]));
-                        }
-                    const uint32_t pos = static_cast<uint32_t>(pos0 + rr);
-#pragma unroll
-                    for (int tt = 0; tt < 3; ++tt) {
-                        amax = fmaxf(amax, shfl_xor_f(amax, 16));
-                        amax = fmaxf(amax, shfl_xor_f(amax, 32));
-                        const int ex = block_exp(amax);
-                        uint32_t c[2] = {0u, 0u};
-                        amax = 0.f;
-#pragma unroll
-                        for (int j = 0; j < 2; ++j)
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) {
-                                float qv;
-                                c[j] |= e4m3_rne(ldexpf(v[j][i], -ex), qv) << (8 * i);
-                                v[j][i] -= ldexpf(qv, ex);
-                                amax = fmaxf(amax, fabsf(v[j][i]));
-                            }
-                        if (ok) {
-                            uint8_t *dst = a.a8 + tt * a.a_term + pos * static_cast<uint32_t>(a.Ipad) + pbase;
-                            *reinterpret_cast<uint32_t *>(dst) = c[0];
-                            *reinterpret_cast<uint32_t *>(dst + 16) = c[1];
-                            if (q == 0)
-                                a.as[tt * a.as_term + pos * static_cast<uint32_t>(a.Ipad >> 5) + blk] =
-                                    static_cast<uint8_t>(ex + 127);
-                        }
-                    }
+                    for (int i = 0; i < 4; ++i)
+                        bf16_split2(act_fn(acc[j][ct][i], acc[j + 2][ct][i], a.act_kind, a.beta, a.lbeta), hi[i], lo[i]);
+                    *reinterpret_cast<uint2 *>(dst + 16 * j) =
+                        make_uint2(hi[0] | (static_cast<uint32_t>(hi[1]) << 16), hi[2] | (static_cast<uint32_t>(hi[3]) << 16));
+                    *reinterpret_cast<uint2 *>(dst + kBlk + 16 * j) =
+                        make_uint2(lo[0] | (static_cast<uint32_t>(lo[1]) << 16), lo[2] | (static_cast<uint32_t>(lo[3]) << 16));
                 }
             }
         }
     }
 }
 
-// LDS of mx_gemm_kernel: two B tiles and their scale pairs
-constexpr size_t mx_lds_bytes(int terms) {
-    return 2 * (static_cast<size_t>(4 * terms * 16 * 16) * 16 + static_cast<size_t>(4 * terms * 16 * 4) * 2);
+// Block order: the work list is (expert, row block, token tile of the expert), and XCD x
+// (blocks b % 8 == x) walks the x-th eighth of it, so the CUs of one XCD read one or two
+// experts at a time: neighbouring rows of one weight matrix, the same token rows, and for
+// an expert of several tiles the same weight rows, which its L2 then holds.
+template <bool DOWN, int TERMS>
+__global__ __launch_bounds__(kThreads, 2) void grouped_gemm_kernel(GemmArgs a) {
+    extern __shared__ char lds[];
+    const int total = *a.n_tiles * a.NT;
+    const int per = (total + 7) >> 3, li = blockIdx.x >> 3;
+    const int w = (blockIdx.x & 7) * per + li;
+    if (li >= per || w >= total) return;
+    const int4 rec = a.tiles[w / a.NT];
+    const int ne = (rec.z + kTM - 1) / kTM, off = w - rec.y * a.NT;
+    const int nt = off / ne, m0 = (off % ne) * kTM;
+    const int rows = min(kTM, rec.z - m0), pos0 = rec.w + m0;
+    const uint64_t *ptr = a.table + static_cast<int64_t>(rec.x) * 6;
+    if (rows > 48)
+        grouped_tile<DOWN, TERMS, 4>(a, lds, nt, rows, pos0, ptr);
+    else if (rows > 32)
+        grouped_tile<DOWN, TERMS, 3>(a, lds, nt, rows, pos0, ptr);
+    else if (rows > 16)
+        grouped_tile<DOWN, TERMS, 2>(a, lds, nt, rows, pos0, ptr);
+    else
+        grouped_tile<DOWN, TERMS, 1>(a, lds, nt, rows, pos0, ptr);
 }
 
-// Grid of mx_gemm_kernel: every (tile, row block) pair; tile major rounds the tiles up to a
-// multiple of the 8 XCDs.
-unsigned mx_grid(const MxArgs &m) {
-    const int64_t tiles = m.tile_major ? 8 * cdiv(m.max_tiles, 8) : m.max_tiles;
-    return static_cast<unsigned>(tiles * m.NT);
-}
-
-// Both GEMMs take more than the default 64 KB of dynamic LDS (gfx950 has 160 KB per CU).
-int mx_prepare() {
+// More than the default 64 KB of dynamic LDS (gfx950 has 160 KB per CU).
+int grouped_prepare() {
     static const hipError_t rc = [] {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&mx_gemm_kernel<false, 2>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           static_cast<int>(mx_lds_bytes(2)));
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void *>(&mx_gemm_kernel<false, 3>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(mx_lds_bytes(3)));
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void *>(&mx_gemm_kernel<true, 3>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(mx_lds_bytes(3)));
-        return e;
+        const void *k[3] = {reinterpret_cast<const void *>(&grouped_gemm_kernel<false, 1>),
+                            reinterpret_cast<const void *>(&grouped_gemm_kernel<false, 2>),
+                            reinterpret_cast<const void *>(&grouped_gemm_kernel<true, 2>)};
+        for (const void *f : k) {
+            const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
     }();
     return check_hip(rc, "moe grouped: LDS size attribute");
 }
@@ -617,29 +512,27 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a) {
 
 // ------------------------------------------------------------------ host side
 struct GroupedWs {
-    size_t counts, base, perm, tile_e, tile_m0, n_tiles, x8, xs, a8, as, ypair, total;
+    size_t counts, base, perm, tiles, n_tiles, xt, act, ypair, total;
     int max_tiles;
-    int64_t Hpad, Ipad;
+    int64_t Hblk, Iblk;   // 128-element blocks of a two-term row
 };
 
 GroupedWs grouped_ws_layout(int64_t T, int64_t k, int64_t E, int64_t H, int64_t I) {
     GroupedWs L{};
     auto up = [](size_t v) { return (v + 255) & ~size_t(255); };
     const int64_t P = T * k;
-    L.Hpad = cdiv(H, kSS) * kSS;
-    L.Ipad = cdiv(I, kSS) * kSS;
-    L.max_tiles = static_cast<int>(cdiv(P, kTM) + E);
+    L.Hblk = cdiv(H, kBlk);
+    L.Iblk = cdiv(I, kBlk);
+    // every expert in use has at least one pair, and all its tiles but one are full
+    L.max_tiles = static_cast<int>(cdiv(P, kTM) + std::min(P, E));
     size_t o = 0;
     L.counts = o, o += up(E * 4);
     L.base = o, o += up(E * 4);
     L.perm = o, o += up(P * 4);
-    L.tile_e = o, o += up(static_cast<size_t>(L.max_tiles) * 4);
-    L.tile_m0 = o, o += up(static_cast<size_t>(L.max_tiles) * 4);
+    L.tiles = o, o += up(static_cast<size_t>(L.max_tiles) * sizeof(int4));
     L.n_tiles = o, o += up(4);
-    L.x8 = o, o += up(static_cast<size_t>(3) * T * L.Hpad);
-    L.xs = o, o += up(static_cast<size_t>(3) * T * (L.Hpad / 32));
-    L.a8 = o, o += up(static_cast<size_t>(3) * P * L.Ipad);
-    L.as = o, o += up(static_cast<size_t>(3) * P * (L.Ipad / 32));
+    L.xt = o, o += up(static_cast<size_t>(T) * L.Hblk * kBlk * 4);
+    L.act = o, o += up(static_cast<size_t>(P) * L.Iblk * kBlk * 4);
     L.ypair = o, o += up(static_cast<size_t>(P) * H * 4);
     L.total = o;
     return L;
@@ -672,8 +565,8 @@ extern "C" int k3_moe_grouped_ffn(const void *x, int x_dtype, const int32_t *exp
                          (long long)H, (long long)I);
     const GroupedWs L = grouped_ws_layout(T, top_k, n_experts, H, I);
     const int64_t P = T * top_k;
-    if (P >= (1ll << 30) || H * I / 2 >= (1ll << 31) || 3 * P * L.Ipad >= (1ll << 31) ||
-        3 * T * L.Hpad >= (1ll << 31))
+    const int64_t Hpad = cdiv(H, 256) * 256, Ipad = cdiv(I, 256) * 256;
+    if (P >= (1ll << 30) || H * I / 2 >= (1ll << 31) || 3 * P * Ipad >= (1ll << 31) || 3 * T * Hpad >= (1ll << 31))
         return set_error(K3_ERR_SHAPE, "moe grouped: problem too large");
     if (workspace_bytes < static_cast<int64_t>(L.total))
         return set_error(K3_ERR_WORKSPACE, "moe grouped: workspace %lld < %zu bytes", (long long)workspace_bytes,
@@ -690,8 +583,7 @@ extern "C" int k3_moe_grouped_ffn(const void *x, int x_dtype, const int32_t *exp
     g.counts = reinterpret_cast<int32_t *>(ws + L.counts);
     g.base = reinterpret_cast<int32_t *>(ws + L.base);
     g.perm = reinterpret_cast<int32_t *>(ws + L.perm);
-    g.tile_e = reinterpret_cast<int32_t *>(ws + L.tile_e);
-    g.tile_m0 = reinterpret_cast<int32_t *>(ws + L.tile_m0);
+    g.tiles = reinterpret_cast<int4 *>(ws + L.tiles);
     g.n_tiles = reinterpret_cast<int32_t *>(ws + L.n_tiles);
     g.max_tiles = L.max_tiles;
     group_count_kernel<<<dim3(g.E), kScanThreads, 0, st>>>(g);
@@ -700,72 +592,51 @@ extern "C" int k3_moe_grouped_ffn(const void *x, int x_dtype, const int32_t *exp
     int rc = check_hip(hipGetLastError(), "moe grouped: grouping launches");
     if (rc) return rc;
 
-    QxArgs qa{};
-    qa.x = x;
-    qa.x8 = reinterpret_cast<uint8_t *>(ws + L.x8);
-    qa.xs = reinterpret_cast<uint8_t *>(ws + L.xs);
-    qa.T = static_cast<int>(T);
-    qa.H = static_cast<int>(H);
-    qa.Hpad = static_cast<int>(L.Hpad);
-    qa.term = static_cast<uint32_t>(T * L.Hpad);
-    qa.sterm = static_cast<uint32_t>(T * (L.Hpad / 32));
+    rc = grouped_prepare();
+    if (rc) return rc;
     const bool xf32 = x_dtype == K3_F32;
-    if (xf32)
-        quant_x_kernel<true><<<dim3(static_cast<unsigned>(cdiv(T * (H / 16), 256))), 256, 0, st>>>(qa);
-    else
-        quant_x_kernel<false><<<dim3(static_cast<unsigned>(cdiv(T * (H / 16), 256))), 256, 0, st>>>(qa);
-    rc = check_hip(hipGetLastError(), "moe grouped: x quantization launch");
-    if (rc) return rc;
-
-    rc = mx_prepare();
-    if (rc) return rc;
-    MxArgs ma{};
+    if (xf32) {
+        SplitArgs sa{};
+        sa.x = static_cast<const float *>(x);
+        sa.xt = reinterpret_cast<uint16_t *>(ws + L.xt);
+        sa.T = static_cast<int>(T), sa.H = static_cast<int>(H), sa.Hblk = static_cast<int>(L.Hblk);
+        split_x_kernel<<<dim3(static_cast<unsigned>(cdiv(T * (H / 8), 256))), 256, 0, st>>>(sa);
+        rc = check_hip(hipGetLastError(), "moe grouped: x split launch");
+        if (rc) return rc;
+    }
+    GemmArgs ma{};
     ma.table = static_cast<const uint64_t *>(expert_table);
-    ma.counts = g.counts;
-    ma.base = g.base;
     ma.perm = g.perm;
-    ma.tile_e = g.tile_e;
-    ma.tile_m0 = g.tile_m0;
+    ma.tiles = g.tiles;
     ma.n_tiles = g.n_tiles;
-    ma.a8 = reinterpret_cast<uint8_t *>(ws + L.a8);
-    ma.as = reinterpret_cast<uint8_t *>(ws + L.as);
-    ma.a_term = static_cast<uint32_t>(P * L.Ipad);
-    ma.as_term = static_cast<uint32_t>(P * (L.Ipad / 32));
-    ma.Ipad = static_cast<int>(L.Ipad);
+    ma.act = reinterpret_cast<uint16_t *>(ws + L.act);
+    ma.act_row = static_cast<uint32_t>(L.Iblk * kBlk * 4);
     ma.ypair = reinterpret_cast<float *>(ws + L.ypair);
     ma.top_k = static_cast<int>(top_k);
-    ma.max_tiles = L.max_tiles;
     ma.act_kind = act_kind;
     ma.beta = beta;
     ma.lbeta = linear_beta;
     // gate/up: K = H, weight rows N = I, 128 intermediate indices per block
-    ma.b8 = qa.x8;
-    ma.bs = qa.xs;
-    ma.b_term = qa.term;
-    ma.bs_term = qa.sterm;
+    ma.b = xf32 ? static_cast<const void *>(ws + L.xt) : x;
+    ma.brow = static_cast<uint32_t>(xf32 ? L.Hblk * kBlk * 4 : H * 2);
+    ma.b_bytes = static_cast<uint32_t>(T * ma.brow);   // below kOob: 3 T Hpad < 2^31
     ma.K = static_cast<int>(H);
-    ma.Kpad = static_cast<int>(L.Hpad);
     ma.N = static_cast<int>(I);
     ma.NT = static_cast<int>(cdiv(I, 128));
-    ma.tile_major = 0;
-    const dim3 gu_grid(mx_grid(ma));
+    auto grid = [&](int NT) { return dim3(static_cast<unsigned>(8 * cdiv(static_cast<int64_t>(L.max_tiles) * NT, 8))); };
     if (xf32)
-        mx_gemm_kernel<false, 3><<<gu_grid, kThreads, mx_lds_bytes(3), st>>>(ma);
+        grouped_gemm_kernel<false, 2><<<grid(ma.NT), kThreads, kLds, st>>>(ma);
     else
-        mx_gemm_kernel<false, 2><<<gu_grid, kThreads, mx_lds_bytes(2), st>>>(ma);
+        grouped_gemm_kernel<false, 1><<<grid(ma.NT), kThreads, kLds, st>>>(ma);
     rc = check_hip(hipGetLastError(), "moe grouped: gate/up launch");
     if (rc) return rc;
     // down: K = I, weight rows N = H, 256 output rows per block, B = the act terms
-    ma.b8 = ma.a8;
-    ma.bs = ma.as;
-    ma.b_term = ma.a_term;
-    ma.bs_term = ma.as_term;
+    ma.b = ma.act;
+    ma.brow = ma.act_row;
     ma.K = static_cast<int>(I);
-    ma.Kpad = static_cast<int>(L.Ipad);
     ma.N = static_cast<int>(H);
     ma.NT = static_cast<int>(cdiv(H, 256));
-    ma.tile_major = 1;
-    mx_gemm_kernel<true, 3><<<dim3(mx_grid(ma)), kThreads, mx_lds_bytes(3), st>>>(ma);
+    grouped_gemm_kernel<true, 2><<<grid(ma.NT), kThreads, kLds, st>>>(ma);
     rc = check_hip(hipGetLastError(), "moe grouped: down launch");
     if (rc) return rc;
 
