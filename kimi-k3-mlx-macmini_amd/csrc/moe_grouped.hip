@@ -202,8 +202,6 @@ constexpr int kABuf = 256 * 128, kBBuf = 64 * 512, kSBuf = 256 * 32;
 constexpr int kLdsB = 2 * kABuf, kLdsS = kLdsB + 2 * kBBuf;
 constexpr int kLds = kLdsS + 2 * kSBuf;
 
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-
 __device__ __forceinline__ bf16x8 fp4x8_bf16(uint32_t w, float s) {
     const uint4 v = make_uint4(__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, s, 0)),
                                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, s, 1)),
@@ -231,9 +229,11 @@ __device__ __forceinline__ void grouped_tile(const GemmArgs &a, char *lds, int n
     const int proj = DOWN ? 4 : (wave < 4 ? 0 : 2);
     const uint32_t rowA = static_cast<uint32_t>(a.K >> 1);
     const auto ra = make_rsrc(uniform_ptr(ptr[proj]), static_cast<uint32_t>(a.N) * rowA);
-    const void *sbase = uniform_ptr(ptr[proj + 1]);
-    const auto rs = make_rsrc(sbase, static_cast<uint32_t>(a.N * KB));
-    const bool s_al = ((reinterpret_cast<uintptr_t>(sbase) | static_cast<uintptr_t>(KB)) & 3u) == 0;
+    // scale rows have any alignment: five aligned dwords hold the 16 bytes at any byte offset
+    const uintptr_t sbase = reinterpret_cast<uintptr_t>(uniform_ptr(ptr[proj + 1]));
+    const uint32_t sdelta = static_cast<uint32_t>(sbase & 3u);
+    const auto rs = make_rsrc(reinterpret_cast<const void *>(sbase - sdelta),
+                              (static_cast<uint32_t>(a.N * KB) + sdelta + 3u) & ~3u);
     const int grow0 = DOWN ? nt * 256 + wave * 32 : nt * 128 + (wave & 3) * 32;  // weight row of block row 32 w
     const int ac = lane & 7;                     // 16-byte chunk of the 128-byte line
     uint32_t aoff[4];
@@ -243,19 +243,24 @@ __device__ __forceinline__ void grouped_tile(const GemmArgs &a, char *lds, int n
         aoff[n] = row < a.N ? static_cast<uint32_t>(row) * rowA + ac * 16u : kOob;
     }
     const int srow = grow0 + (lane >> 1);
-    const uint32_t soff = srow < a.N ? static_cast<uint32_t>(srow * KB) + (lane & 1) * 16u : kOob;
+    const uint32_t soff = srow < a.N ? static_cast<uint32_t>(srow * KB) + (lane & 1) * 16u + sdelta : kOob;
     const auto rb = DOWN ? make_rsrc(static_cast<const char *>(a.b) + static_cast<int64_t>(pos0) * a.brow,
                                      static_cast<uint32_t>(rows) * a.brow)
                          : make_rsrc(a.b, a.b_bytes);
     const int bc = lane & 31;                    // 16-byte chunk of the 512 bytes
-    uint32_t boff[4];
+    const int brow0 = wave * 2 * NCT + (lane >> 5);  // NCT row pairs per wave
+    uint32_t boff[NCT];
 #pragma unroll
-    for (int n = 0; n < 4; ++n) {
-        const int rr = wave * 8 + 2 * n + (lane >> 5);
-        boff[n] = kOob;
-        if (rr < rows) boff[n] = static_cast<uint32_t>(DOWN ? rr : a.perm[pos0 + rr] / a.top_k) * a.brow + bc * 16u;
+    for (int n = 0; n < NCT; ++n) {
+        const int rr = brow0 + 2 * n;
+        const int src = DOWN ? rr : a.perm[pos0 + min(rr, rows - 1)] / a.top_k;
+        boff[n] = rr < rows ? static_cast<uint32_t>(src) * a.brow + bc * 16u : kOob;
     }
-    uint4 RA[2][4], RB[2][4], RS;
+    // register sets: loads run one or two steps ahead of their stores; a step of three or four
+    // column groups computes longer than a load takes, and its sums need the registers
+    constexpr int D = NCT >= 3 ? 1 : 2;
+    uint4 RA[D][4], RB[D][NCT], RS;
+    uint32_t RS4;
     auto load_a = [&](int S, int set) {
         const bool ok = S * 8 + ac < KB;
 #pragma unroll
@@ -264,36 +269,53 @@ __device__ __forceinline__ void grouped_tile(const GemmArgs &a, char *lds, int n
     auto load_b = [&](int u, int set) {
         const bool ok = TERMS == 1 ? u * 32 + bc < (a.K >> 3) : u * 16 + (bc & 15) < (a.K >> 3);
 #pragma unroll
-        for (int n = 0; n < 4; ++n) RB[set][n] = buf_load16(rb, ok ? boff[n] + u * 512u : kOob);
+        for (int n = 0; n < NCT; ++n) RB[set][n] = buf_load16(rb, ok ? boff[n] + u * 512u : kOob);
     };
     auto load_s = [&](int G) {
-        const uint32_t off = soff + G * 32u;
-        if (s_al) {
-            RS = buf_load16(rs, off);
-        } else {  // scale rows of any alignment, byte by byte
-            uint32_t w[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-            for (int i = 0; i < 16; ++i)
-                w[i >> 2] |= static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b8(rs, off + i, 0, 0)) << (8 * (i & 3));
-            RS = make_uint4(w[0], w[1], w[2], w[3]);
-        }
+        const uint32_t off = (soff + G * 32u) & ~3u;
+        RS = buf_load16(rs, off);
+        RS4 = buf_load4(rs, off + 16u);
     };
+    // LDS row of A: 16-byte unit p = 4 kg + q holds what lane (., q) of wave group kg takes in
+    // the step, dwords 2kg, 2kg + 1 of groups q and 4 + q
     auto store_a = [&](int set, int buf) {
 #pragma unroll
         for (int n = 0; n < 4; ++n) {
             const int R = wave * 32 + 8 * n + (lane >> 3);
-            *reinterpret_cast<uint4 *>(lds + buf * kABuf + R * 128 + ((ac ^ (R & 7)) << 4)) = RA[set][n];
+            char *row = lds + buf * kABuf + R * 128 + (ac >> 2) * 8;
+            *reinterpret_cast<uint2 *>(row + (((ac & 3) ^ (R & 7)) << 4)) = make_uint2(RA[set][n].x, RA[set][n].y);
+            *reinterpret_cast<uint2 *>(row + (((4 + (ac & 3)) ^ (R & 7)) << 4)) = make_uint2(RA[set][n].z, RA[set][n].w);
         }
     };
     auto store_b = [&](int set, int buf) {
 #pragma unroll
-        for (int n = 0; n < 4; ++n) {
-            const int rr = wave * 8 + 2 * n + (lane >> 5);
-            if (NCT == 4 || rr < NCT * 16)
-                *reinterpret_cast<uint4 *>(lds + kLdsB + buf * kBBuf + rr * 512 + ((bc ^ (rr & 7)) << 4)) = RB[set][n];
+        for (int n = 0; n < NCT; ++n) {
+            const int rr = brow0 + 2 * n;
+            *reinterpret_cast<uint4 *>(lds + kLdsB + buf * kBBuf + rr * 512 + ((bc ^ (rr & 7)) << 4)) = RB[set][n];
         }
     };
-    auto store_s = [&](int buf) { *reinterpret_cast<uint4 *>(lds + kLdsS + buf * kSBuf + tid * 16) = RS; };
+    // 32 scale bytes per row and four steps, as [q][step][h]: a lane reads its eight in one
+    // 8-byte load.  Bytes past the row's end become zero (they meet zero weights, and must
+    // not hold another row's infinity).
+    auto store_s = [&](int G) {
+        const uint32_t sh = soff & 3u;
+        uint32_t v[4] = {__builtin_amdgcn_alignbyte(RS.y, RS.x, sh), __builtin_amdgcn_alignbyte(RS.z, RS.y, sh),
+                         __builtin_amdgcn_alignbyte(RS.w, RS.z, sh), __builtin_amdgcn_alignbyte(RS4, RS.w, sh)};
+        const int left = KB - G * 32 - (lane & 1) * 16;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            const int n = max(min(left - 4 * d, 4), 0);
+            v[d] &= n == 4 ? ~0u : (1u << (8 * n)) - 1u;
+        }
+        char *row = lds + kLdsS + (G & 1) * kSBuf + (tid >> 1) * 32 + (lane & 1) * 4;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            // bytes i of the step's groups 0-3 and 4-7, for two steps
+            const uint32_t lo = __builtin_amdgcn_perm(v[1], v[0], 0x0c0c0400u + 0x0101u * i);
+            const uint32_t hi = __builtin_amdgcn_perm(v[3], v[2], 0x0c0c0400u + 0x0101u * i);
+            *reinterpret_cast<uint32_t *>(row + i * 8) = lo | (hi << 16);
+        }
+    };
 
     f32x4 acc[4][NCT];
 #pragma unroll
@@ -309,25 +331,35 @@ __device__ __forceinline__ void grouped_tile(const GemmArgs &a, char *lds, int n
     // its elements 8i .. 8i + 7 (one dword), against the same elements of the tokens.  Wave
     // group kg takes i = 2kg, 2kg + 1 in both forms, so bf16 x gives the sums that fp32 x
     // with the same values gives.
-    auto compute = [&](int S, int h, int abuf, int bbuf) {
-        const char *A = lds + abuf * kABuf, *B = lds + kLdsB + bbuf * kBBuf;
-        const char *Sc = lds + kLdsS + ((S >> 2) & 1) * kSBuf + (S & 3) * 8 + 4 * h + q;
-        const bool live = S * 8 + 4 * h + q < KB;
-        constexpr int NI = 2;
-        uint32_t w[4][NI];
-        float sc[4];
+    uint32_t sw[4][2];                           // this lane's scale bytes of four steps
+    auto read_s = [&](int G) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const uint2 v = *reinterpret_cast<const uint2 *>(A + arow[j] * 128 + (((4 * h + q) ^ (arow[j] & 7)) << 4) + 8 * kg);
-            w[j][0] = v.x, w[j][1] = v.y;
-            const uint32_t b = *reinterpret_cast<const uint8_t *>(Sc + arow[j] * 32);
-            sc[j] = e8m0_to_f32(live ? b : 0u);
+            const uint2 v = *reinterpret_cast<const uint2 *>(lds + kLdsS + (G & 1) * kSBuf + arow[j] * 32 + q * 8);
+            sw[j][0] = v.x, sw[j][1] = v.y;
         }
+    };
+    uint4 wv[4];                                 // this lane's weights of the step: two groups' halves
+    auto read_a = [&](int abuf) {
 #pragma unroll
-        for (int i = 0; i < NI; ++i) {
+        for (int j = 0; j < 4; ++j)
+            wv[j] = *reinterpret_cast<const uint4 *>(lds + abuf * kABuf + arow[j] * 128 +
+                                                     (((4 * kg + q) ^ (arow[j] & 7)) << 4));
+    };
+    auto compute = [&](int P, int h, int bbuf) {
+        const char *B = lds + kLdsB + bbuf * kBBuf;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
             bf16x8 av[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) av[j] = fp4x8_bf16(w[j][i], sc[j]);
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t w4[4] = {wv[j].x, wv[j].y, wv[j].z, wv[j].w};
+                const int byte = (2 * P + h) & 3;
+                const uint32_t s4 = sw[j][P >> 1];
+                // the conversion takes the scale's exponent bits
+                const float sc = __uint_as_float((byte == 3 ? s4 >> 1 : s4 << (23 - 8 * byte)) & 0x7f800000u);
+                av[j] = fp4x8_bf16(w4[2 * h + i], sc);
+            }
 #pragma unroll
             for (int t = 0; t < TERMS; ++t) {
                 const int chunk = 16 * (TERMS == 1 ? h : t) + 4 * q + 2 * kg + i;
@@ -343,50 +375,60 @@ __device__ __forceinline__ void grouped_tile(const GemmArgs &a, char *lds, int n
         }
     };
 
-    // ---- pipeline: step S computes on buffers S % 2 while step S + 1 is stored and steps
-    // S + 2, S + 3 are in flight
+    // ---- pipeline: step S computes on buffers S % 2, then stores step S + 1 and issues step
+    // S + 1 + D.  (The loads wait in order, so B goes ahead of A: a wait for B leaves the newer
+    // A in flight; the fences keep the entry's loads in the loop's order.)
     load_a(0, 0);
-    load_b(0, 0);
     load_s(0);
-    load_a(1, 1);
-    load_b(1, 1);
+    load_b(0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (D == 2) load_b(1, D - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    if (D == 2) load_a(1, D - 1);
+    __builtin_amdgcn_sched_barrier(0);
     store_a(0, 0);
     store_b(0, 0);
     store_s(0);
-    load_a(2, 0);
-    load_b(2, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    load_b(D, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    load_a(D, 0);
+    __builtin_amdgcn_sched_barrier(0);
     auto step = [&](int S, int P) {
-        const int nx = (P + 1) & 1;
+        const int nx = (P + 1) & 1, set = nx & (D - 1);
+        __syncthreads();
+        if (P == 0) read_s(S >> 2);
+        read_a(P & 1);
         if constexpr (TERMS == 1) {
-            __syncthreads();
-            store_a(nx, nx);
-            store_b(nx, nx);
-            if (P == 3) store_s(((S >> 2) + 1) & 1);
-            load_a(S + 3, nx);
-            load_b(S + 3, nx);
-            if (P == 0) load_s((S >> 2) + 1);
-            compute(S, 0, P & 1, P & 1);
-            compute(S, 1, P & 1, P & 1);
+            compute(P, 0, P & 1);
+            compute(P, 1, P & 1);
+            store_b(set, nx);
+            load_b(S + 1 + D, set);
         } else {
+            compute(P, 0, 0);
+            store_b(D - 1, 1);
+            load_b(2 * S + 1 + D, D - 1);
             __syncthreads();
-            store_b(1, 1);
-            load_b(2 * S + 3, 1);
-            if (P == 0) load_s((S >> 2) + 1);
-            compute(S, 0, P & 1, 0);
-            __syncthreads();
-            store_a(nx, nx);
+            compute(P, 1, 1);
             store_b(0, 0);
-            if (P == 3) store_s(((S >> 2) + 1) & 1);
-            load_a(S + 3, nx);
-            load_b(2 * S + 4, 0);
-            compute(S, 1, P & 1, 1);
+            load_b(2 * S + 2 + D, 0);
         }
+        store_a(set, nx);
+        if (P == 3) store_s((S >> 2) + 1);
+        if (P == 0) load_s((S >> 2) + 1);
+        load_a(S + 1 + D, set);
     };
-    for (int S = 0; S < NS; S += 4) {
+    // (left by break only, so the loop head has one predecessor besides the entry and the
+    // compiler's counted waits there stay exact)
+    for (int S = 0;; S += 4) {
         step(S, 0);
-        if (S + 1 < NS) step(S + 1, 1);
-        if (S + 2 < NS) step(S + 2, 2);
-        if (S + 3 < NS) step(S + 3, 3);
+        if (S + 1 >= NS) break;
+        step(S + 1, 1);
+        if (S + 2 >= NS) break;
+        step(S + 2, 2);
+        if (S + 3 >= NS) break;
+        step(S + 3, 3);
+        if (S + 4 >= NS) break;
     }
 
     // ---- the two wave groups' sums meet: group kg finishes column groups ct % 2 == kg and
