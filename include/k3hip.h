@@ -161,24 +161,48 @@ int k3_moe_layer_decode(const void *x, int x_dtype, const void *router_w, const 
                         int64_t n_experts, int64_t top_k, int act_kind, float beta,
                         float linear_beta, void *workspace, int64_t workspace_bytes, void *stream);
 
+/* ---- dense projections for many tokens ------------------------------------------------- */
+
+/* Workspace bytes k3_dense needs for these shapes (partial sums where the reduction is split
+ * over blocks; 0 otherwise).  N [n_mats] is host memory.  No initialisation. */
+int64_t k3_dense_workspace_size(int64_t M, int64_t K, const int64_t *N, int64_t n_mats, int a_dtype);
+
+/* out[i] [M, N[i]] fp32 = a [M, K] w[i]^T for up to 8 bf16 weight matrices w[i] [N[i], K] in one
+ * launch; a is bf16 or fp32 (a_dtype) with row pitch lda elements.  fp32 values enter as three
+ * bf16 terms whose sum is exact, so products are exact and sums fp32.  add (or NULL): fp32
+ * [M, N[0]] added to the output, for n_mats == 1.  w, out and N are host arrays.  K a multiple
+ * of 8, rows of a 16-byte aligned.  Deterministic.
+ * Replaces the reference's promoted matmuls of prefill (moe.py:67-68, attention_mla.py:168-216,
+ * attention_kda.py:94-115). */
+int k3_dense(const void *a, int a_dtype, int64_t lda, const void *const *w, void *const *out,
+             const int64_t *N, int64_t n_mats, const float *add, int64_t M, int64_t K, void *workspace,
+             int64_t workspace_bytes, void *stream);
+
+/* out [M, K] = w * x * rsqrt(mean(x^2) + eps) per row of x (row pitch ldx), all fp32
+ * (KimiRMSNorm, air_llm/models/kimi_k3/ops.py:11-14). */
+int k3_rmsnorm_rows(const float *x, int64_t ldx, const float *w, float eps, float *out, int64_t M, int64_t K,
+                    void *stream);
+
+/* out[i] = act(g[i], u[i]) for n fp32 values (ops.py:17-28, 42-43); n a multiple of 4. */
+int k3_act_rows(const float *g, const float *u, float *out, int64_t n, int act_kind, float beta,
+                float linear_beta, void *stream);
+
 /* ---- grouped routed experts for many tokens (prefill) ------------------------------------ */
 
-/* Workspace bytes k3_moe_grouped_ffn needs (grouping records, the E4M3 terms of x and of the
- * activations of every routed pair with their E8M0 scales, fp32 per-pair expert outputs).
+/* Workspace bytes k3_moe_grouped_ffn needs (grouping records, the bf16 terms of an fp32 x and of
+ * the activations of every routed pair, fp32 per-pair expert outputs).
  * No initialisation. */
 int64_t k3_moe_grouped_workspace_size(int64_t T, int64_t top_k, int64_t n_experts, int64_t H, int64_t I);
 
 /* y[t] = sum_j w[t, j] * expert_{idx[t, j]}(x[t]) for T tokens at once:
  *   x [T, H] bf16 or fp32 (x_dtype); expert_idx int32 [T, top_k] (every id in 0..n_experts-1); expert_w f32
  *   [T, top_k]; expert_table as in k3_moe_layer_decode (packed pointers 16-byte aligned,
- *   scale pointers 2-byte aligned, E8M0 bytes 2..252); out [T, H] f32 or bf16.
+ *   E8M0 bytes 2..252); out [T, H] f32 or bf16.
  * The (token, slot) pairs are grouped by expert on the device and each expert runs as a
- * GEMM with M = its token count on native MXFP4 MFMA (v_mfma_scale_f32_16x16x128_f8f6f4:
- * the weights as stored, bf16 x as two E4M3 terms (exact), fp32 x and the activation as
- * three (about 12 bits), all with E8M0
- * scales per 32), so each expert's weights are read once per 64-token tile.  Normwise error
- * about 1e-4 of fp64 (the MFMA's own accumulation).  Deterministic.  H and I must be
- * multiples of 64.
+ * GEMM with M = its token count on the bf16 matrix cores (the weights decoded exactly, bf16 x
+ * exact, fp32 x and the activation as two bf16 terms, 16 bits), so each expert's weights are
+ * read once.  Normwise error about 5e-6 of fp64.  Deterministic.  H and I must be multiples
+ * of 64.
  * Replaces the per-expert dispatch loop of LatentMoE.__call__
  * (air_llm/models/kimi_k3/moe.py:110-132; k3ref/layers.py:241-261) for prefill. */
 int k3_moe_grouped_ffn(const void *x, int x_dtype, const int32_t *expert_idx, const float *expert_w,

@@ -402,14 +402,17 @@ __device__ __forceinline__ void grouped_tile(const GemmArgs &a, char *lds, int n
         if constexpr (TERMS == 1) {
             compute(P, 0, P & 1);
             compute(P, 1, P & 1);
+            __builtin_amdgcn_sched_barrier(0);  // the stores wait for loads the sums above cover
             store_b(set, nx);
             load_b(S + 1 + D, set);
         } else {
             compute(P, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
             store_b(D - 1, 1);
             load_b(2 * S + 1 + D, D - 1);
             __syncthreads();
             compute(P, 1, 1);
+            __builtin_amdgcn_sched_barrier(0);
             store_b(0, 0);
             load_b(2 * S + 2 + D, 0);
         }

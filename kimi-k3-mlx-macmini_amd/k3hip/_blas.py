@@ -1,15 +1,17 @@
-"""Dense projections on the BLAS library (hipBLASLt through torch) for the multi-token paths.
+"""Dense projections for the multi-token paths.
 
 ``mm_f32(a, w)`` is ``a @ w.T`` with fp32 output, exact products and fp32 accumulation for
 bf16 or fp32 ``a`` against bf16 or fp32 ``w``, without copying the weight:
 
-* bf16 ``a``, bf16 ``w``: one GEMM with fp32 output;
-* fp32 ``a``, bf16 ``w``: ``a`` is the exact sum of three bf16 terms (8 + 8 + 8 significant
-  bits), each one GEMM with fp32 output, summed;
+* bf16 ``a``, bf16 ``w``: one GEMM with fp32 output on the BLAS library;
+* fp32 ``a``, bf16 ``w``: ``k3_dense`` (``a`` as the exact sum of three bf16 terms against the
+  weight in one launch);
 * fp32 ``w``: an fp32 GEMM.
 
 This is the arithmetic of the reference's fp32 router and of MLX's promotion of a bf16
 weight against an fp32 activation (``air_llm/models/kimi_k3/moe.py:67-68``).
+
+``dense(a, ws)`` is ``k3_dense`` itself: several bf16 weight matrices against one ``a``.
 
 ``mm_ref(a, w)`` keeps the reference's dtype promotion instead: operands of one dtype give
 that dtype (a bf16 GEMM returns bf16, as MLX's bf16 matmul does), mixed operands give fp32.
@@ -17,7 +19,12 @@ The paths that restate the reference's own unfused definitions use it.
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
+
+from . import _lib, _workspace
+from . import _torch as T
 
 
 def bf16_terms(a: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
@@ -33,6 +40,35 @@ def _mm_bf16_f32(a2: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return torch.mm(a2, w.t(), out_dtype=torch.float32)
 
 
+def dense_ok(a: torch.Tensor, *ws: torch.Tensor) -> bool:
+    """k3_dense takes these operands as they are (device tensors, bf16 weights of whole
+    16-byte rows) and no gradient is asked for."""
+    if not a.is_cuda or a.dtype not in (torch.float32, torch.bfloat16) or a.shape[-1] % 8:
+        return False
+    if torch.is_grad_enabled() and (a.requires_grad or any(w.requires_grad for w in ws)):
+        return False
+    return all(w.is_cuda and w.dim() == 2 and w.dtype == torch.bfloat16 and w.is_contiguous()
+               and w.data_ptr() % 16 == 0 and w.shape[1] == a.shape[-1] and w.device == a.device for w in ws)
+
+
+def dense(a: torch.Tensor, ws, add: torch.Tensor | None = None) -> list[torch.Tensor]:
+    """[a [M, K] @ w[N, K]^T in fp32 for w in ws] (k3_dense; operands checked by dense_ok), plus
+    ``add`` [M, N] fp32 where one weight is given."""
+    M, K = a.shape
+    if a.stride(1) != 1 or (a.stride(0) * a.element_size()) % 16 or a.stride(0) < K or a.data_ptr() % 16:
+        a = T.contiguous_aligned(a)
+    n = len(ws)
+    outs = [torch.empty((M, w.shape[0]), dtype=torch.float32, device=a.device) for w in ws]
+    N = (ctypes.c_int64 * n)(*(w.shape[0] for w in ws))
+    code = T.dtype_code(a.dtype)
+    nbytes = int(_lib.lib().k3_dense_workspace_size(M, K, N, n, code))
+    buf = _workspace.get(a.device, nbytes, "dense") if nbytes else None
+    _lib.call("k3_dense", T.ptr(a), code, a.stride(0) if M > 1 else K, (ctypes.c_void_p * n)(*(w.data_ptr() for w in ws)),
+              (ctypes.c_void_p * n)(*(o.data_ptr() for o in outs)), N, n, T.ptr(add), M, K, T.ptr(buf), nbytes,
+              T.stream(a))
+    return outs
+
+
 def mm_f32(a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """a [..., K] @ w[N, K]^T -> fp32 [..., N] with exact products and fp32 accumulation."""
     lead = a.shape[:-1]
@@ -42,6 +78,8 @@ def mm_f32(a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     elif w.dtype == torch.bfloat16:
         if a2.dtype == torch.bfloat16:
             out = _mm_bf16_f32(a2, w)
+        elif a2.dtype == torch.float32 and a2.shape[0] > 0 and dense_ok(a2, w):
+            out = dense(a2, [w])[0]
         else:
             t1, t2, t3 = bf16_terms(a2.to(torch.float32))
             out = _mm_bf16_f32(t1, w)
