@@ -161,6 +161,27 @@ int k3_moe_layer_decode(const void *x, int x_dtype, const void *router_w, const 
                         int64_t n_experts, int64_t top_k, int act_kind, float beta,
                         float linear_beta, void *workspace, int64_t workspace_bytes, void *stream);
 
+/* ---- KDA layer over many tokens, around the recurrence ------------------------------------- */
+
+/* The inputs of k3_kda_recurrent for B sequences of T tokens, from the fp32 projections (rows
+ * b * T + t: q_raw, k_raw, v_raw, fb [B*T, heads*128], b_raw [B*T, heads]): the short convolutions
+ * with SiLU over each sequence continued from its window (q_win, k_win, v_win [B, conv_size-1,
+ * heads*128], or all NULL: zeros; ops.py:46-60), the L2 norms of q and k, the log decay and beta
+ * (attention_kda.py:94-115).  Outputs time-major fp32: q, k, v, g [T, B, heads, 128], beta
+ * [T, B, heads]; the windows after the last token go to *_win_out (not the input windows). */
+int k3_kda_prefill_inputs(const float *q_raw, const float *k_raw, const float *v_raw, const float *fb,
+                          const float *b_raw, const float *q_conv, const float *k_conv, const float *v_conv,
+                          const float *q_win, const float *k_win, const float *v_win, float *q_win_out,
+                          float *k_win_out, float *v_win_out, const float *A_log, const float *dt_bias,
+                          float *q, float *k, float *v, float *g, float *beta, int64_t B, int64_t T,
+                          int64_t heads, int64_t head_dim, int64_t conv_size, float gate_lower_bound,
+                          void *stream);
+
+/* out [B*T, heads*128] = gated RMSNorm of the recurrence's o (time-major [T, B, heads, 128]):
+ * o * rsqrt(mean(o^2) + eps) * w * sigmoid(gate), gate [B*T, heads*128] (ops.py:36-39). */
+int k3_kda_gated_norm(const float *o, const float *gate, const float *w, float eps, float *out, int64_t B,
+                      int64_t T, int64_t heads, int64_t head_dim, void *stream);
+
 /* ---- dense projections for many tokens ------------------------------------------------- */
 
 /* Workspace bytes k3_dense needs for these shapes (partial sums where the reduction is split

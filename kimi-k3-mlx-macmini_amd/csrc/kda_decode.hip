@@ -122,57 +122,269 @@ __device__ __forceinline__ void kda_load_state(float *S, int h, int V, int c0, f
     }
 }
 
-// T tokens in order; the block's state columns stay in registers between them, so the
-// state is read and written once whatever T is.  The next token's inputs are loaded while
-// the current one is reduced.
-template <bool MULTI>
+// One token.
 __global__ __launch_bounds__(256) void kda_decode_kernel(KdaArgs a) {
     __shared__ float red[2][4][kKdaVS];
     const int nvb = a.V / kKdaVS;
     const int h = blockIdx.x / nvb, vb = blockIdx.x % nvb;
-    const int hq = h / a.G, HQ = a.HV / a.G;
+    const int hq = h / a.G;
     const int t = threadIdx.x, cg = t & 7, r = t >> 3;
     const int c0 = vb * kKdaVS + 4 * cg;
     const int bf = a.in_bf16;
     float *Sp[4];
     float4 x[4];
     kda_load_state(a.S, h, a.V, c0, x, Sp);
-    float kk[4], qq[4], dk[4], vv[4], b;
-    auto load = [&](int i, float(&k_)[4], float(&q_)[4], float(&d_)[4], float(&v_)[4], float &b_) {
-        const int64_t qo = (static_cast<int64_t>(i) * HQ + hq) * kKdaK, go = (static_cast<int64_t>(i) * a.HV + h) * kKdaK;
+    float kk[4], qq[4], dk[4], vv[4];
+    const int64_t qo = static_cast<int64_t>(hq) * kKdaK, go = static_cast<int64_t>(h) * kKdaK;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            k_[j] = ldx(a.k, qo + r + 32 * j, bf);
-            q_[j] = ldx(a.q, qo + r + 32 * j, bf) * a.scale;
-            d_[j] = ldx(a.g, go + r + 32 * j, bf);
-        }
-        const int64_t vo = (static_cast<int64_t>(i) * a.HV + h) * a.V + c0;
+    for (int j = 0; j < 4; ++j) {
+        kk[j] = ldx(a.k, qo + r + 32 * j, bf);
+        qq[j] = ldx(a.q, qo + r + 32 * j, bf) * a.scale;
+        dk[j] = expf(ldx(a.g, go + r + 32 * j, bf));
+    }
+    const int64_t vo = static_cast<int64_t>(h) * a.V + c0;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) v_[c] = ldx(a.v, vo + c, bf);
-        b_ = ldx(a.beta, static_cast<int64_t>(i) * a.HV + h, bf);
-    };
-    load(0, kk, qq, dk, vv, b);
-    const int T = MULTI ? a.T : 1;
-    for (int i = 0; i < T; ++i) {
-        float nk[4], nq[4], nd[4], nv[4], nb = 0.f;
-        if (MULTI && i + 1 < T) load(i + 1, nk, nq, nd, nv, nb);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) dk[j] = expf(dk[j]);
-        const float o = kda_apply(x, kk, qq, dk, vv, b, red);
-        if (t < kKdaVS) {
-            const int64_t oi = (static_cast<int64_t>(i) * a.HV + h) * a.V + vb * kKdaVS + t;
-            if (a.out_bf16)
-                static_cast<uint16_t *>(a.out)[oi] = f32_to_bf16(o);
-            else
-                static_cast<float *>(a.out)[oi] = o;
-        }
-        if (MULTI && i + 1 < T) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) kk[j] = nk[j], qq[j] = nq[j], dk[j] = nd[j], vv[j] = nv[j];
-            b = nb;
-        }
+    for (int c = 0; c < 4; ++c) vv[c] = ldx(a.v, vo + c, bf);
+    const float o = kda_apply(x, kk, qq, dk, vv, ldx(a.beta, h, bf), red);
+    if (t < kKdaVS) {
+        const int64_t oi = static_cast<int64_t>(h) * a.V + vb * kKdaVS + t;
+        if (a.out_bf16)
+            static_cast<uint16_t *>(a.out)[oi] = f32_to_bf16(o);
+        else
+            static_cast<float *>(a.out)[oi] = o;
     }
     kda_store_state(x, Sp);
+}
+
+// Many tokens, in order.  The tokens are a serial chain, so what bounds the launch is the
+// length of one token's step; the state stays in registers throughout.  A wave owns 8 value
+// columns: lane (rg, cp) holds rows 4 rg .. + 3 and 64 + 4 rg .. + 3 of columns 2 cp, 2 cp + 1,
+// so a column's reduction over the 128 key channels is 8 terms in a lane and four DPP steps
+// inside a 16-lane row, with no LDS round trip and no barrier.  Both reductions run on the
+// decayed state at once, since
+//   q . (S' + (beta k) (x) d) = q . S' + (q . k) (beta d),  d = v - k . S'
+// and q . k needs no state.  The inputs of 16 tokens at a time (scaled q, k, exp(g), v, beta,
+// q . k) are staged in LDS, double buffered, one barrier per 16 tokens, and each token's are
+// read one token ahead.
+// 256 tokens, 96 heads of 128 x 128: 470 us with two barriers and two LDS reductions per
+// token, @@KDA@@.
+constexpr int kKdaChunk = 16;
+
+__device__ __forceinline__ float row16_sum(float v) {  // sum over the 16 lanes of a DPP row, in all of them
+    v += dpp_or_zero<0xb1>(v);
+    v += dpp_or_zero<0x4e>(v);
+    v += dpp_or_zero<0x141>(v);
+    v += dpp_or_zero<0x140>(v);
+    return v;
+}
+
+__global__ __launch_bounds__(256) void kda_sequence_kernel(KdaArgs a) {
+    __shared__ float4 in[2][kKdaChunk][3][kKdaK / 4];  // k, q, decay
+    __shared__ float2 vs[2][kKdaChunk][kKdaVS / 2];
+    __shared__ float2 bq[2][kKdaChunk];                // beta, q . k
+    const int nvb = a.V / kKdaVS;
+    const int h = blockIdx.x / nvb, vb = blockIdx.x % nvb;
+    const int hq = h / a.G, HQ = a.HV / a.G;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, rg = lane & 15, cp = lane >> 4;
+    const int col = vb * kKdaVS + wave * 8 + 2 * cp;
+    const int bf = a.in_bf16;
+    float S[8][2];
+    float *Sp = a.S + (static_cast<int64_t>(h) * kKdaK + 4 * rg) * a.V + col;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+        const float2 v = *reinterpret_cast<const float2 *>(Sp + static_cast<int64_t>((r >> 2) * 64 + (r & 3)) * a.V);
+        S[r][0] = v.x, S[r][1] = v.y;
+    }
+    // staging: thread (token tid / 16, channels 8 (tid % 16) .. + 7)
+    const int st = tid >> 4, sp = tid & 15;
+    float k8[8], q8[8], g8[8], v2[2], sb;
+    auto load8 = [&](const void *p, int64_t i, float (&o)[8]) {
+        if (bf) {
+            const uint4 u = *reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(p) + i);
+            const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+            for (int x = 0; x < 4; ++x) o[2 * x] = __uint_as_float(w[x] << 16), o[2 * x + 1] = __uint_as_float(w[x] & 0xffff0000u);
+        } else {
+            const float4 *f = reinterpret_cast<const float4 *>(static_cast<const float *>(p) + i);
+            const float4 x = f[0], y = f[1];
+            o[0] = x.x, o[1] = x.y, o[2] = x.z, o[3] = x.w, o[4] = y.x, o[5] = y.y, o[6] = y.z, o[7] = y.w;
+        }
+    };
+    auto load = [&](int i0) {
+        const int64_t i = min(i0 + st, a.T - 1);  // past the end: the last token, not used
+        load8(a.k, (i * HQ + hq) * kKdaK + 8 * sp, k8);
+        load8(a.q, (i * HQ + hq) * kKdaK + 8 * sp, q8);
+        load8(a.g, (i * a.HV + h) * kKdaK + 8 * sp, g8);
+        const int64_t vo = (i * a.HV + h) * a.V + vb * kKdaVS + 2 * sp;
+        v2[0] = ldx(a.v, vo, bf), v2[1] = ldx(a.v, vo + 1, bf);
+        sb = ldx(a.beta, i * a.HV + h, bf);
+    };
+    auto store = [&](int buf) {
+        float dot = 0.f;
+#pragma unroll
+        for (int x = 0; x < 8; ++x) {
+            q8[x] *= a.scale;
+            dot = fmaf(q8[x], k8[x], dot);
+            g8[x] = expf(g8[x]);
+        }
+        dot = row16_sum(dot);
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            in[buf][st][0][2 * sp + x] = make_float4(k8[4 * x], k8[4 * x + 1], k8[4 * x + 2], k8[4 * x + 3]);
+            in[buf][st][1][2 * sp + x] = make_float4(q8[4 * x], q8[4 * x + 1], q8[4 * x + 2], q8[4 * x + 3]);
+            in[buf][st][2][2 * sp + x] = make_float4(g8[4 * x], g8[4 * x + 1], g8[4 * x + 2], g8[4 * x + 3]);
+        }
+        vs[buf][st][sp] = make_float2(v2[0], v2[1]);
+        if (sp == 0) bq[buf][st] = make_float2(sb, dot);
+    };
+    struct Token {
+        float4 k[2], q[2], d[2];
+        float2 v, bq;
+    };
+    auto read = [&](int buf, int i, Token &t) {
+#pragma unroll
+        for (int x = 0; x < 2; ++x) t.k[x] = in[buf][i][0][rg + 16 * x], t.q[x] = in[buf][i][1][rg + 16 * x], t.d[x] = in[buf][i][2][rg + 16 * x];
+        t.v = vs[buf][i][wave * 4 + cp];
+        t.bq = bq[buf][i];
+    };
+    load(0);
+    store(0);
+    __syncthreads();
+    for (int i0 = 0, buf = 0; i0 < a.T; i0 += kKdaChunk, buf ^= 1) {
+        const int n = min(kKdaChunk, a.T - i0);
+        const bool more = i0 + kKdaChunk < a.T;
+        if (more) load(i0 + kKdaChunk);
+        Token t;
+        read(buf, 0, t);
+        for (int i = 0; i < n; ++i) {
+            Token nx;
+            read(buf, min(i + 1, n - 1), nx);
+            const float kk[8] = {t.k[0].x, t.k[0].y, t.k[0].z, t.k[0].w, t.k[1].x, t.k[1].y, t.k[1].z, t.k[1].w};
+            const float qq[8] = {t.q[0].x, t.q[0].y, t.q[0].z, t.q[0].w, t.q[1].x, t.q[1].y, t.q[1].z, t.q[1].w};
+            const float dd[8] = {t.d[0].x, t.d[0].y, t.d[0].z, t.d[0].w, t.d[1].x, t.d[1].y, t.d[1].z, t.d[1].w};
+            float p[2] = {0.f, 0.f}, o[2] = {0.f, 0.f};
+#pragma unroll
+            for (int r = 0; r < 8; ++r)
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    S[r][c] *= dd[r];
+                    p[c] = fmaf(kk[r], S[r][c], p[c]);
+                    o[c] = fmaf(qq[r], S[r][c], o[c]);
+                }
+            p[0] = row16_sum(p[0]), p[1] = row16_sum(p[1]), o[0] = row16_sum(o[0]), o[1] = row16_sum(o[1]);
+            const float d[2] = {t.bq.x * (t.v.x - p[0]), t.bq.x * (t.v.y - p[1])};
+#pragma unroll
+            for (int r = 0; r < 8; ++r)
+#pragma unroll
+                for (int c = 0; c < 2; ++c) S[r][c] = fmaf(kk[r], d[c], S[r][c]);
+            if (rg == 0) {
+                const float y0 = fmaf(t.bq.y, d[0], o[0]), y1 = fmaf(t.bq.y, d[1], o[1]);
+                const int64_t oi = (static_cast<int64_t>(i0 + i) * a.HV + h) * a.V + col;
+                if (a.out_bf16)
+                    *reinterpret_cast<uint32_t *>(static_cast<uint16_t *>(a.out) + oi) =
+                        f32_to_bf16(y0) | (static_cast<uint32_t>(f32_to_bf16(y1)) << 16);
+                else
+                    *reinterpret_cast<float2 *>(static_cast<float *>(a.out) + oi) = make_float2(y0, y1);
+            }
+            t = nx;
+        }
+        if (more) {
+            store(buf ^ 1);
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+        *reinterpret_cast<float2 *>(Sp + static_cast<int64_t>((r >> 2) * 64 + (r & 3)) * a.V) = make_float2(S[r][0], S[r][1]);
+}
+
+// ------------------------------------------------------------------ around the recurrence, many tokens
+// The recurrence's inputs of B sequences of T tokens from the projections (token-major rows
+// b * T + t): short convolutions with SiLU, L2 norms of q and k, decay gate, beta, as
+// kda_step_kernel builds them for one token.  A block takes one head and eight tokens.
+// Outputs are time-major, [T, B, H, 128] and [T, B, H].
+struct KdaPrepArgs {
+    const float *raw[3];                     // q, k, v projections [B * T, P]
+    const float *fb, *b_raw;                 // [B * T, P], [B * T, H]
+    const float *conv[3];                    // [P, kc]
+    const float *win[3];                     // [B, kc - 1, P], or null (zeros)
+    float *win_out[3];                       // [B, kc - 1, P]
+    const float *A_log, *dt_bias;
+    float lower;
+    float *q, *k, *v, *g, *beta;
+    int B, T, H, kc;
+};
+constexpr int kPrepTokens = 8;
+
+__global__ __launch_bounds__(128) void kda_prep_kernel(KdaPrepArgs a) {
+    __shared__ float part[2][kPrepTokens][2];
+    const int c = threadIdx.x, h = blockIdx.x, t0 = blockIdx.y * kPrepTokens, b = blockIdx.z;
+    const int P = a.H * kKdaK, ch = h * kKdaK + c, kc = a.kc, lane = c & 63, wave = c >> 6;
+    const int64_t row0 = static_cast<int64_t>(b) * a.T;
+    // input i of the padded sequence: the window, then the tokens
+    auto xp = [&](int m, int i) -> float {
+        if (i >= kc - 1) return a.raw[m][(row0 + i - (kc - 1)) * P + ch];
+        return a.win[m] ? a.win[m][(static_cast<int64_t>(b) * (kc - 1) + i) * P + ch] : 0.f;
+    };
+    float y[3][kPrepTokens];
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+        float w[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) w[j] = j < kc ? a.conv[m][static_cast<int64_t>(ch) * kc + j] : 0.f;
+#pragma unroll
+        for (int i = 0; i < kPrepTokens; ++i) {
+            const int t = min(t0 + i, a.T - 1);
+            float z = 0.f;
+            if (kc == 4) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) z = fmaf(w[j], xp(m, t + j), z);
+            } else {
+                for (int j = 0; j < kc; ++j) z = fmaf(a.conv[m][static_cast<int64_t>(ch) * kc + j], xp(m, t + j), z);
+            }
+            y[m][i] = z / (1.0f + expf(-z));
+        }
+        if (blockIdx.y == 0)
+            for (int j = 0; j < kc - 1; ++j) a.win_out[m][(static_cast<int64_t>(b) * (kc - 1) + j) * P + ch] = xp(m, a.T + j);
+    }
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int i = 0; i < kPrepTokens; ++i) {
+            const float s = wave_sum_all(y[m][i] * y[m][i]);
+            if (lane == 0) part[m][i][wave] = s;
+        }
+    __syncthreads();
+    const float ea = expf(a.A_log[h]), db = a.dt_bias[ch];
+#pragma unroll
+    for (int i = 0; i < kPrepTokens; ++i) {
+        const int t = t0 + i;
+        if (t < a.T) {
+            const int64_t th = (static_cast<int64_t>(t) * a.B + b) * a.H + h, o = th * kKdaK + c;
+            a.q[o] = y[0][i] / sqrtf(part[0][i][0] + part[0][i][1] + 1e-6f);
+            a.k[o] = y[1][i] / sqrtf(part[1][i][0] + part[1][i][1] + 1e-6f);
+            a.v[o] = y[2][i];
+            const float z = ea * (a.fb[(row0 + t) * P + ch] + db);
+            a.g[o] = a.lower / (1.0f + expf(-z));
+            if (c == 0) a.beta[th] = 1.0f / (1.0f + expf(-a.b_raw[(row0 + t) * a.H + h]));
+        }
+    }
+}
+
+// out [B * T, P] = o * rsqrt(mean(o^2) + eps) * w * sigmoid(og): o time-major [T, B, H, 128], one
+// wave per (token, head) (ops.py:36-39).
+__global__ __launch_bounds__(256) void kda_gated_norm_kernel(const float *o, const float *og, const float *w, float eps,
+                                                             float *out, int B, int T, int H) {
+    const int64_t id = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (id >= static_cast<int64_t>(B) * T * H) return;
+    const int h = static_cast<int>(id % H);
+    const int64_t row = id / H, b = row / T, t = row % T;
+    const float2 x = reinterpret_cast<const float2 *>(o + ((t * B + b) * H + h) * kKdaK)[lane];
+    const float s = 1.0f / sqrtf(wave_sum_all(x.x * x.x + x.y * x.y) * (1.0f / kKdaK) + eps);
+    const float2 g = reinterpret_cast<const float2 *>(og + id * kKdaK)[lane], wn = reinterpret_cast<const float2 *>(w)[lane];
+    reinterpret_cast<float2 *>(out + id * kKdaK)[lane] =
+        make_float2(x.x * s * wn.x / (1.0f + expf(-g.x)), x.y * s * wn.y / (1.0f + expf(-g.y)));
 }
 
 // ------------------------------------------------------------------ whole KDA layer step
@@ -316,9 +528,9 @@ static int kda_recurrent_impl(const void *q, const void *k, const void *v, const
     a.scale = scale;
     const int64_t blocks = v_heads * (value_dim / kKdaVS);
     if (T == 1)
-        kda_decode_kernel<false><<<dim3(static_cast<unsigned>(blocks)), 256, 0, static_cast<hipStream_t>(stream)>>>(a);
+        kda_decode_kernel<<<dim3(static_cast<unsigned>(blocks)), 256, 0, static_cast<hipStream_t>(stream)>>>(a);
     else
-        kda_decode_kernel<true><<<dim3(static_cast<unsigned>(blocks)), 256, 0, static_cast<hipStream_t>(stream)>>>(a);
+        kda_sequence_kernel<<<dim3(static_cast<unsigned>(blocks)), 256, 0, static_cast<hipStream_t>(stream)>>>(a);
     return check_hip(hipGetLastError(), "kda recurrence launch");
 }
 
@@ -335,6 +547,49 @@ extern "C" int k3_kda_recurrent(const void *q, const void *k, const void *v, con
                                 int64_t v_heads, int64_t key_dim, int64_t value_dim, float scale, void *stream) {
     return kda_recurrent_impl(q, k, v, g, beta, in_dtype, state, out, out_dtype, T, qk_heads, v_heads, key_dim,
                               value_dim, scale, stream);
+}
+
+extern "C" int k3_kda_prefill_inputs(const float *q_raw, const float *k_raw, const float *v_raw, const float *fb,
+                                     const float *b_raw, const float *q_conv, const float *k_conv, const float *v_conv,
+                                     const float *q_win, const float *k_win, const float *v_win, float *q_win_out,
+                                     float *k_win_out, float *v_win_out, const float *A_log, const float *dt_bias,
+                                     float *q, float *k, float *v, float *g, float *beta, int64_t B, int64_t T,
+                                     int64_t heads, int64_t head_dim, int64_t conv_size, float gate_lower_bound,
+                                     void *stream) {
+    if (!q_raw || !k_raw || !v_raw || !fb || !b_raw || !q_conv || !k_conv || !v_conv || !q_win_out || !k_win_out ||
+        !v_win_out || !A_log || !dt_bias || !q || !k || !v || !g || !beta || (!q_win != !k_win) || (!q_win != !v_win))
+        return set_error(K3_ERR_NULL, "kda prefill inputs: null pointer");
+    if (head_dim != kKdaK) return set_error(K3_ERR_SHAPE, "kda prefill inputs: head_dim=%lld; the kernels take %d",
+                                            (long long)head_dim, kKdaK);
+    if (conv_size < 2 || conv_size > 8) return set_error(K3_ERR_SHAPE, "kda prefill inputs: conv_size=%lld", (long long)conv_size);
+    if (B <= 0 || T <= 0 || heads <= 0 || B > 65535 || T > 8 * 65535 || heads > (1 << 20))
+        return set_error(K3_ERR_SHAPE, "kda prefill inputs: B=%lld, T=%lld, heads=%lld", (long long)B, (long long)T,
+                         (long long)heads);
+    KdaPrepArgs a{};
+    a.raw[0] = q_raw, a.raw[1] = k_raw, a.raw[2] = v_raw, a.fb = fb, a.b_raw = b_raw;
+    a.conv[0] = q_conv, a.conv[1] = k_conv, a.conv[2] = v_conv;
+    a.win[0] = q_win, a.win[1] = k_win, a.win[2] = v_win;
+    a.win_out[0] = q_win_out, a.win_out[1] = k_win_out, a.win_out[2] = v_win_out;
+    a.A_log = A_log, a.dt_bias = dt_bias, a.lower = gate_lower_bound;
+    a.q = q, a.k = k, a.v = v, a.g = g, a.beta = beta;
+    a.B = static_cast<int>(B), a.T = static_cast<int>(T), a.H = static_cast<int>(heads), a.kc = static_cast<int>(conv_size);
+    const dim3 grid(static_cast<unsigned>(heads), static_cast<unsigned>(cdiv(T, kPrepTokens)), static_cast<unsigned>(B));
+    kda_prep_kernel<<<grid, 128, 0, static_cast<hipStream_t>(stream)>>>(a);
+    return check_hip(hipGetLastError(), "kda prefill inputs launch");
+}
+
+extern "C" int k3_kda_gated_norm(const float *o, const float *gate, const float *w, float eps, float *out, int64_t B,
+                                 int64_t T, int64_t heads, int64_t head_dim, void *stream) {
+    if (!o || !gate || !w || !out) return set_error(K3_ERR_NULL, "kda gated norm: null pointer");
+    if (head_dim != kKdaK) return set_error(K3_ERR_SHAPE, "kda gated norm: head_dim=%lld; the kernel takes %d",
+                                            (long long)head_dim, kKdaK);
+    if (B <= 0 || T <= 0 || heads <= 0 || B * T * heads >= (1ll << 31))
+        return set_error(K3_ERR_SHAPE, "kda gated norm: B=%lld, T=%lld, heads=%lld", (long long)B, (long long)T, (long long)heads);
+    if (!aligned16(o) || !aligned16(gate) || !aligned16(w) || !aligned16(out))
+        return set_error(K3_ERR_ALIGN, "kda gated norm: 16-byte alignment");
+    kda_gated_norm_kernel<<<dim3(static_cast<unsigned>(cdiv(B * T * heads, 4))), 256, 0, static_cast<hipStream_t>(stream)>>>(
+        o, gate, w, eps, out, static_cast<int>(B), static_cast<int>(T), static_cast<int>(heads));
+    return check_hip(hipGetLastError(), "kda gated norm launch");
 }
 
 namespace {

@@ -69,6 +69,22 @@ def dense(a: torch.Tensor, ws, add: torch.Tensor | None = None) -> list[torch.Te
     return outs
 
 
+def project(a: torch.Tensor, ws) -> list[torch.Tensor]:
+    """[a [M, K] @ w[N, K]^T in fp32 for w in ws], all against one activation.
+
+    fp32 a: one k3_dense launch.  bf16 a, which needs one matrix-core pass: k3_dense while the
+    launch streams weights (up to 32 tokens, or up to 256 when the matrices give half the CUs
+    a tile each), where one launch for all matrices beats a library GEMM each (24,576 + 224
+    rows of 7168, six matrices: 2 tokens 120 against 153 us, 256 tokens 269 against 352 us);
+    beyond that the library's larger tiles win (10,304 rows, three matrices: 64 tokens 70
+    against 62 us, 1000 tokens 197 against 160 us)."""
+    M = a.shape[0]
+    tiles = sum((w.shape[0] + 255) // 256 for w in ws)
+    if M and dense_ok(a, *ws) and (a.dtype == torch.float32 or M <= 32 or (M <= 256 and tiles >= 128)):
+        return dense(a, list(ws))
+    return [mm_f32(a, w) for w in ws]
+
+
 def mm_f32(a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """a [..., K] @ w[N, K]^T -> fp32 [..., N] with exact products and fp32 accumulation."""
     lead = a.shape[:-1]

@@ -59,6 +59,8 @@ SIGNATURES: dict[str, list] = {
     "k3_kda_step_workspace_size": [_I64],
     "k3_kda_step_decode": [_P, _I32, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I32,
                            _I64, _I64, _I64, _I64, _F32, _F32, _P, _I64, _P],
+    "k3_kda_prefill_inputs": [_P] * 21 + [_I64] * 5 + [_F32, _P],
+    "k3_kda_gated_norm": [_P, _P, _P, _F32, _P, _I64, _I64, _I64, _I64, _P],
     "k3_dense_workspace_size": [_I64, _I64, _P, _I64, _I32],
     "k3_dense": [_P, _I32, _I64, _P, _P, _P, _I64, _P, _I64, _I64, _P, _I64, _P],
     "k3_rmsnorm_rows": [_P, _I64, _P, _F32, _P, _I64, _I64, _P],
