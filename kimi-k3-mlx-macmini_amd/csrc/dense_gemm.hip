@@ -100,15 +100,39 @@ __global__ __launch_bounds__(kThreads, 2) void dense_kernel(DenseArgs a) {
         aoff[n] = row < mrows ? static_cast<uint32_t>(row * a.lda * ES) + ac * 16u + k0 * ES : kOob;
     }
     uint4 RW[4], RA[NA];
-    auto load = [&](int S) {
-        const bool wok = k0 + S * kBK + wc * 8 < kend, aok = k0 + S * kBK + ac * (16 / ES) < kend;
+    uint2 RT[NA][3];                                       // the split terms of RA (fp32 a)
+    auto load_w = [&](int S) {
+        const bool ok = k0 + S * kBK + wc * 8 < kend;
 #pragma unroll
-        for (int n = 0; n < NA; ++n) RA[n] = buf_load16(ra, aok ? aoff[n] + S * (kBK * ES) : kOob);
-#pragma unroll
-        for (int n = 0; n < 4; ++n) RW[n] = buf_load16(rw, wok ? woff[n] + S * (kBK * 2u) : kOob);
+        for (int n = 0; n < 4; ++n) RW[n] = buf_load16(rw, ok ? woff[n] + S * (kBK * 2u) : kOob);
     };
-    auto store = [&](int buf) {
-        char *W = lds + buf * kStage, *A = W + kW;
+    auto load_a = [&](int S) {
+        const bool ok = k0 + S * kBK + ac * (16 / ES) < kend;
+#pragma unroll
+        for (int n = 0; n < NA; ++n) RA[n] = buf_load16(ra, ok ? aoff[n] + S * (kBK * ES) : kOob);
+    };
+    auto store_w = [&](int buf) {
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            const int row = wave * 32 + 8 * n + (lane >> 3);
+            *reinterpret_cast<uint4 *>(lds + buf * kStage + row * 128 + ((wc ^ (row & 7)) << 4)) = RW[n];
+        }
+    };
+    auto split = [&] {
+        if constexpr (TERMS == 3) {
+#pragma unroll
+            for (int n = 0; n < NA; ++n) {
+                const uint32_t v[4] = {RA[n].x, RA[n].y, RA[n].z, RA[n].w};
+                uint32_t t[3][4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) split3(__uint_as_float(v[i]), t[0][i], t[1][i], t[2][i]);
+#pragma unroll
+                for (int x = 0; x < 3; ++x) RT[n][x] = make_uint2(hi16x2(t[x][0], t[x][1]), hi16x2(t[x][2], t[x][3]));
+            }
+        }
+    };
+    auto store_a = [&](int buf) {
+        char *A = lds + buf * kStage + kW;
 #pragma unroll
         for (int n = 0; n < NA; ++n) {
             const int row = arow0 + n * RPI;
@@ -116,22 +140,11 @@ __global__ __launch_bounds__(kThreads, 2) void dense_kernel(DenseArgs a) {
                 if constexpr (TERMS == 1) {
                     *reinterpret_cast<uint4 *>(A + row * 128 + ((ac ^ (row & 7)) << 4)) = RA[n];
                 } else {
-                    const uint32_t v[4] = {RA[n].x, RA[n].y, RA[n].z, RA[n].w};
-                    uint32_t t[3][4];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) split3(__uint_as_float(v[i]), t[0][i], t[1][i], t[2][i]);
                     char *p = A + row * 128 + (((ac >> 1) ^ (row & 7)) << 4) + (ac & 1) * 8;
 #pragma unroll
-                    for (int x = 0; x < 3; ++x)
-                        *reinterpret_cast<uint2 *>(p + x * kA) =
-                            make_uint2(hi16x2(t[x][0], t[x][1]), hi16x2(t[x][2], t[x][3]));
+                    for (int x = 0; x < 3; ++x) *reinterpret_cast<uint2 *>(p + x * kA) = RT[n][x];
                 }
             }
-        }
-#pragma unroll
-        for (int n = 0; n < 4; ++n) {
-            const int row = wave * 32 + 8 * n + (lane >> 3);
-            *reinterpret_cast<uint4 *>(W + row * 128 + ((wc ^ (row & 7)) << 4)) = RW[n];
         }
     };
 
@@ -140,46 +153,66 @@ __global__ __launch_bounds__(kThreads, 2) void dense_kernel(DenseArgs a) {
     for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (int i = 0; i < MT; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    auto compute = [&](int buf) {
+    bf16x8 wv[NT], av[TERMS][MT];
+    auto read = [&](int buf, int kk) {
         const char *W = lds + buf * kStage + (wn * NT * 16 + r16) * 128;
         const char *A = lds + buf * kStage + kW + (wm * MT * 16 + r16) * 128;
+        const int c = ((4 * kk + q) ^ (r16 & 7)) << 4;
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-            const int c = ((4 * kk + q) ^ (r16 & 7)) << 4;
-            bf16x8 av[TERMS][MT];
+        for (int j = 0; j < NT; ++j) wv[j] = *reinterpret_cast<const bf16x8 *>(W + j * 2048 + c);
 #pragma unroll
-            for (int t = 0; t < TERMS; ++t)
+        for (int t = 0; t < TERMS; ++t)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) av[t][i] = *reinterpret_cast<const bf16x8 *>(A + t * kA + i * 2048 + c);
+    };
+    auto multiply = [&] {
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int t = TERMS - 1; t >= 0; --t)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
 #pragma unroll
                 for (int i = 0; i < MT; ++i)
-                    av[t][i] = *reinterpret_cast<const bf16x8 *>(A + t * kA + i * 2048 + c);
-#pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                const bf16x8 wv = *reinterpret_cast<const bf16x8 *>(W + j * 2048 + c);
-#pragma unroll
-                for (int t = TERMS - 1; t >= 0; --t)
-#pragma unroll
-                    for (int i = 0; i < MT; ++i)
-                        acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, av[t][i], acc[j][i], 0, 0, 0);
-            }
-        }
+                    acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[j], av[t][i], acc[j][i], 0, 0, 0);
+        __builtin_amdgcn_s_setprio(0);
     };
-    load(0);
-    store(0);
-    load(1);
-    for (int S = 0;; S += 2) {
-        __syncthreads();
-        compute(0);
-        __builtin_amdgcn_sched_barrier(0);  // the stores wait for loads the sums above cover
-        if (S + 1 >= NS) break;
-        store(1);
-        load(S + 2);
-        __syncthreads();
-        compute(1);
+    auto phase = [&] {
         __builtin_amdgcn_sched_barrier(0);
-        if (S + 2 >= NS) break;
-        store(0);
-        load(S + 3);
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // Two groups of four waves, one wave of each per SIMD, run half a beat apart: while one
+    // multiplies (and splits the fp32 values it loaded), the other reads its next operands
+    // from LDS and stores its part of the next step, so the matrix cores do not wait for LDS.
+    // A buffer is overwritten at the earliest one barrier after its last read and read at the
+    // earliest one barrier after its last store.
+    const bool late = wave >= 4;
+    load_w(0);
+    load_a(0);
+    store_w(0);
+    split();
+    store_a(0);
+    load_w(1);
+    load_a(1);
+    phase();
+    if (late) phase();
+    for (int S = 0; S < NS; ++S) {
+        const int buf = S & 1;
+        read(buf, 0);
+        store_w(buf ^ 1);
+        load_w(S + 2);
+        phase();
+        split();
+        multiply();
+        phase();
+        read(buf, 1);
+        store_a(buf ^ 1);
+        load_a(S + 2);
+        phase();
+        multiply();
+        phase();
     }
+    if (!late) phase();
 
     // ---- lane: outputs n0 + 16 j + 4q .. + 3 of token r16
 #pragma unroll

@@ -30,6 +30,7 @@ struct KdaArgs {
     float *S;                 // [HV, K, V] fp32, updated in place
     void *out;                // [T, HV, V]
     int out_bf16;
+    int vec;                  // q, k, g are 16-byte aligned and out holds aligned pairs (many tokens)
     int HV, G, V, T;          // G = HV / HQ value heads per q/k head
     float scale;
 };
@@ -178,6 +179,14 @@ __device__ __forceinline__ float row16_sum(float v) {  // sum over the 16 lanes 
     return v;
 }
 
+// four of them side by side, so no step waits for the one before it
+__device__ __forceinline__ void row16_sum4(float &a, float &b, float &c, float &d) {
+    a += dpp_or_zero<0xb1>(a), b += dpp_or_zero<0xb1>(b), c += dpp_or_zero<0xb1>(c), d += dpp_or_zero<0xb1>(d);
+    a += dpp_or_zero<0x4e>(a), b += dpp_or_zero<0x4e>(b), c += dpp_or_zero<0x4e>(c), d += dpp_or_zero<0x4e>(d);
+    a += dpp_or_zero<0x141>(a), b += dpp_or_zero<0x141>(b), c += dpp_or_zero<0x141>(c), d += dpp_or_zero<0x141>(d);
+    a += dpp_or_zero<0x140>(a), b += dpp_or_zero<0x140>(b), c += dpp_or_zero<0x140>(c), d += dpp_or_zero<0x140>(d);
+}
+
 __global__ __launch_bounds__(256) void kda_sequence_kernel(KdaArgs a) {
     __shared__ float4 in[2][kKdaChunk][3][kKdaK / 4];  // k, q, decay
     __shared__ float2 vs[2][kKdaChunk][kKdaVS / 2];
@@ -199,7 +208,10 @@ __global__ __launch_bounds__(256) void kda_sequence_kernel(KdaArgs a) {
     const int st = tid >> 4, sp = tid & 15;
     float k8[8], q8[8], g8[8], v2[2], sb;
     auto load8 = [&](const void *p, int64_t i, float (&o)[8]) {
-        if (bf) {
+        if (!a.vec) {
+#pragma unroll
+            for (int x = 0; x < 8; ++x) o[x] = ldx(p, i + x, bf);
+        } else if (bf) {
             const uint4 u = *reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(p) + i);
             const uint32_t w[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
@@ -254,11 +266,9 @@ __global__ __launch_bounds__(256) void kda_sequence_kernel(KdaArgs a) {
         const int n = min(kKdaChunk, a.T - i0);
         const bool more = i0 + kKdaChunk < a.T;
         if (more) load(i0 + kKdaChunk);
-        Token t;
-        read(buf, 0, t);
-        for (int i = 0; i < n; ++i) {
-            Token nx;
-            read(buf, min(i + 1, n - 1), nx);
+        // one token: the state's step; lane rg == i of each row keeps the read-out
+        float y[2] = {0.f, 0.f};
+        auto token = [&](const Token &t, int i) {
             const float kk[8] = {t.k[0].x, t.k[0].y, t.k[0].z, t.k[0].w, t.k[1].x, t.k[1].y, t.k[1].z, t.k[1].w};
             const float qq[8] = {t.q[0].x, t.q[0].y, t.q[0].z, t.q[0].w, t.q[1].x, t.q[1].y, t.q[1].z, t.q[1].w};
             const float dd[8] = {t.d[0].x, t.d[0].y, t.d[0].z, t.d[0].w, t.d[1].x, t.d[1].y, t.d[1].z, t.d[1].w};
@@ -271,22 +281,39 @@ __global__ __launch_bounds__(256) void kda_sequence_kernel(KdaArgs a) {
                     p[c] = fmaf(kk[r], S[r][c], p[c]);
                     o[c] = fmaf(qq[r], S[r][c], o[c]);
                 }
-            p[0] = row16_sum(p[0]), p[1] = row16_sum(p[1]), o[0] = row16_sum(o[0]), o[1] = row16_sum(o[1]);
+            row16_sum4(p[0], p[1], o[0], o[1]);
             const float d[2] = {t.bq.x * (t.v.x - p[0]), t.bq.x * (t.v.y - p[1])};
 #pragma unroll
             for (int r = 0; r < 8; ++r)
 #pragma unroll
                 for (int c = 0; c < 2; ++c) S[r][c] = fmaf(kk[r], d[c], S[r][c]);
-            if (rg == 0) {
-                const float y0 = fmaf(t.bq.y, d[0], o[0]), y1 = fmaf(t.bq.y, d[1], o[1]);
-                const int64_t oi = (static_cast<int64_t>(i0 + i) * a.HV + h) * a.V + col;
-                if (a.out_bf16)
-                    *reinterpret_cast<uint32_t *>(static_cast<uint16_t *>(a.out) + oi) =
-                        f32_to_bf16(y0) | (static_cast<uint32_t>(f32_to_bf16(y1)) << 16);
-                else
-                    *reinterpret_cast<float2 *>(static_cast<float *>(a.out) + oi) = make_float2(y0, y1);
+#pragma unroll
+            for (int c = 0; c < 2; ++c) y[c] = rg == i ? fmaf(t.bq.y, d[c], o[c]) : y[c];
+        };
+        Token t0, t1;
+        read(buf, 0, t0);
+        for (int i = 0; i < n; i += 2) {
+            read(buf, min(i + 1, n - 1), t1);
+            token(t0, i);
+            if (i + 1 >= n) break;
+            read(buf, min(i + 2, n - 1), t0);
+            token(t1, i + 1);
+        }
+        if (rg < n) {
+            const int64_t oi = (static_cast<int64_t>(i0 + rg) * a.HV + h) * a.V + col;
+            if (!a.vec) {
+                for (int c = 0; c < 2; ++c) {
+                    if (a.out_bf16)
+                        static_cast<uint16_t *>(a.out)[oi + c] = f32_to_bf16(y[c]);
+                    else
+                        static_cast<float *>(a.out)[oi + c] = y[c];
+                }
+            } else if (a.out_bf16) {
+                *reinterpret_cast<uint32_t *>(static_cast<uint16_t *>(a.out) + oi) =
+                    f32_to_bf16(y[0]) | (static_cast<uint32_t>(f32_to_bf16(y[1])) << 16);
+            } else {
+                *reinterpret_cast<float2 *>(static_cast<float *>(a.out) + oi) = make_float2(y[0], y[1]);
             }
-            t = nx;
         }
         if (more) {
             store(buf ^ 1);
@@ -322,28 +349,35 @@ __global__ __launch_bounds__(128) void kda_prep_kernel(KdaPrepArgs a) {
     const int P = a.H * kKdaK, ch = h * kKdaK + c, kc = a.kc, lane = c & 63, wave = c >> 6;
     const int64_t row0 = static_cast<int64_t>(b) * a.T;
     // input i of the padded sequence: the window, then the tokens
-    auto xp = [&](int m, int i) -> float {
-        if (i >= kc - 1) return a.raw[m][(row0 + i - (kc - 1)) * P + ch];
-        return a.win[m] ? a.win[m][(static_cast<int64_t>(b) * (kc - 1) + i) * P + ch] : 0.f;
+    auto xp = [&](int m, int i) -> float {  // (uniform choices; one load, unconditional but for a null window)
+        const bool tok = i >= kc - 1;
+        if (!tok && !a.win[m]) return 0.f;
+        const float *p = tok ? a.raw[m] + (row0 + i - (kc - 1)) * P : a.win[m] + (static_cast<int64_t>(b) * (kc - 1) + i) * P;
+        return p[ch];
     };
     float y[3][kPrepTokens];
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
-        float w[8];
+        const float *cw = a.conv[m] + static_cast<int64_t>(ch) * kc;
+        if (kc == 4) {
+            float x[kPrepTokens + 3];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) w[j] = j < kc ? a.conv[m][static_cast<int64_t>(ch) * kc + j] : 0.f;
+            for (int i = 0; i < kPrepTokens + 3; ++i) x[i] = xp(m, min(t0 + i, a.T + 2));
+            const float w0 = cw[0], w1 = cw[1], w2 = cw[2], w3 = cw[3];
 #pragma unroll
-        for (int i = 0; i < kPrepTokens; ++i) {
-            const int t = min(t0 + i, a.T - 1);
-            float z = 0.f;
-            if (kc == 4) {
+            for (int i = 0; i < kPrepTokens; ++i)
+                y[m][i] = fmaf(w3, x[i + 3], fmaf(w2, x[i + 2], fmaf(w1, x[i + 1], w0 * x[i])));
+        } else {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) z = fmaf(w[j], xp(m, t + j), z);
-            } else {
-                for (int j = 0; j < kc; ++j) z = fmaf(a.conv[m][static_cast<int64_t>(ch) * kc + j], xp(m, t + j), z);
+            for (int i = 0; i < kPrepTokens; ++i) {
+                const int t = min(t0 + i, a.T - 1);
+                float z = 0.f;
+                for (int j = 0; j < kc; ++j) z = fmaf(cw[j], xp(m, t + j), z);
+                y[m][i] = z;
             }
-            y[m][i] = z / (1.0f + expf(-z));
         }
+#pragma unroll
+        for (int i = 0; i < kPrepTokens; ++i) y[m][i] = y[m][i] / (1.0f + expf(-y[m][i]));
         if (blockIdx.y == 0)
             for (int j = 0; j < kc - 1; ++j) a.win_out[m][(static_cast<int64_t>(b) * (kc - 1) + j) * P + ch] = xp(m, a.T + j);
     }
@@ -525,6 +559,7 @@ static int kda_recurrent_impl(const void *q, const void *k, const void *v, const
     a.G = static_cast<int>(v_heads / qk_heads);
     a.V = static_cast<int>(value_dim);
     a.T = static_cast<int>(T);
+    a.vec = aligned16(q) && aligned16(k) && aligned16(g) && (reinterpret_cast<uintptr_t>(out) & 7) == 0;
     a.scale = scale;
     const int64_t blocks = v_heads * (value_dim / kKdaVS);
     if (T == 1)

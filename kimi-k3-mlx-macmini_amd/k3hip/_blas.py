@@ -72,15 +72,14 @@ def dense(a: torch.Tensor, ws, add: torch.Tensor | None = None) -> list[torch.Te
 def project(a: torch.Tensor, ws) -> list[torch.Tensor]:
     """[a [M, K] @ w[N, K]^T in fp32 for w in ws], all against one activation.
 
-    fp32 a: one k3_dense launch.  bf16 a, which needs one matrix-core pass: k3_dense while the
-    launch streams weights (up to 32 tokens, or up to 256 when the matrices give half the CUs
-    a tile each), where one launch for all matrices beats a library GEMM each (24,576 + 224
-    rows of 7168, six matrices: 2 tokens 120 against 153 us, 256 tokens 269 against 352 us);
-    beyond that the library's larger tiles win (10,304 rows, three matrices: 64 tokens 70
-    against 62 us, 1000 tokens 197 against 160 us)."""
+    fp32 a: one k3_dense launch.  bf16 a, which needs one matrix-core pass: k3_dense for several
+    matrices of up to 1024 tokens, where one launch replaces a library GEMM each (224 + 4 x
+    12,288 rows of 7168: 2 tokens 120 against 153 us, 256 tokens 217 against 349 us; 10,304 rows
+    in three matrices: 64 tokens 34 against 63 us, 1000 tokens 156 against 158 us), and for one
+    matrix of 65 to 256 tokens, where its K split fills the chip (256 x 7168 x 12288: 64 against
+    111 us); the library elsewhere (700 x 7168 x 2048: 48 against 28 us)."""
     M = a.shape[0]
-    tiles = sum((w.shape[0] + 255) // 256 for w in ws)
-    if M and dense_ok(a, *ws) and (a.dtype == torch.float32 or M <= 32 or (M <= 256 and tiles >= 128)):
+    if M and dense_ok(a, *ws) and (a.dtype == torch.float32 or (len(ws) > 1 and M <= 1024) or 64 < M <= 256):
         return dense(a, list(ws))
     return [mm_f32(a, w) for w in ws]
 
