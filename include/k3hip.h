@@ -161,6 +161,24 @@ int k3_moe_layer_decode(const void *x, int x_dtype, const void *router_w, const 
                         int64_t n_experts, int64_t top_k, int act_kind, float beta,
                         float linear_beta, void *workspace, int64_t workspace_bytes, void *stream);
 
+/* ---- MLA attention for many query tokens ----------------------------------------------------- */
+
+/* Workspace bytes k3_mla_prefill needs over Tk cached tokens (the expanded keys and values of a
+ * group of heads, within 1 GiB or one head's).  No initialisation. */
+int64_t k3_mla_prefill_workspace_size(int64_t Tk, int64_t heads);
+
+/* Causal attention of T query tokens, the last T of the Tk cached positions:
+ *   q [T, heads, 192] fp32 (128 nope, 64 rotary; row pitch ldq); kv_b [heads * 256, 512] bf16 (128 key
+ *   rows then 128 value rows per head); lat [Tk, 512], rot [Tk, 64] cache rows, bf16 or fp32
+ *   (cache_dtype), row pitches ld_lat, ld_rot; gate NULL or [T, heads * 128] fp32 logits whose sigmoid
+ *   multiplies the result; out [T, heads * 128] fp32.
+ * fp32 operands enter the bf16 matrix cores as three terms, sums are fp32: fp32 accuracy.
+ * Replaces the multi-token branch of MLAAttention.__call__ (attention_mla.py:193-214). */
+int k3_mla_prefill(const float *q, int64_t ldq, const void *kv_b, const void *lat, int64_t ld_lat,
+                   const void *rot, int64_t ld_rot, int cache_dtype, const float *gate, float *out, int64_t T,
+                   int64_t Tk, int64_t heads, int64_t kv_lora_rank, int64_t rope_dim, int64_t nope_dim,
+                   int64_t v_dim, float scale, void *workspace, int64_t workspace_bytes, void *stream);
+
 /* ---- KDA layer over many tokens, around the recurrence ------------------------------------- */
 
 /* The inputs of k3_kda_recurrent for B sequences of T tokens, from the fp32 projections (rows

@@ -17,6 +17,7 @@
 // in order by a second launch, while there are fewer blocks than CUs.
 // @@MEASURED@@
 #include <algorithm>
+#include <type_traits>
 
 #include "k3_common.h"
 #include "moe_common.h"
@@ -39,23 +40,16 @@ struct DenseArgs {
     float *out[kMaxSeg];             // [M, N] fp32 each
     int N[kMaxSeg], t0[kMaxSeg];     // rows and first weight tile of each matrix
     const float *add;                // [M, N] fp32 added to the (single) output, or null
-    float *part;                     // [ksplit][nt * 256][M'] when ksplit > 1 (M' = mt * BM)
+    float *part;                     // [ksplit][M'][nt * 256] when ksplit > 1 (M' = mt * BM)
+    uint16_t *kp, *vt;               // MLA keys and values (k3_common.h): bf16 terms
+    int tpad;
 };
 
-// fp32 -> three bf16 terms (upper halves of t1, t2, t3); infinities and NaNs stay in the first
-__device__ __forceinline__ void split3(float v, uint32_t &t1, uint32_t &t2, uint32_t &t3) {
-    const uint32_t u = __float_as_uint(v);
-    t1 = u & 0xffff0000u;
-    const float r = (u & 0x7f800000u) == 0x7f800000u ? 0.f : v - __uint_as_float(t1);
-    t2 = __float_as_uint(r) & 0xffff0000u;
-    t3 = __float_as_uint(r - __uint_as_float(t2));
-    if ((u & 0x7fffffffu) > 0x7f800000u) t1 |= 0x00400000u;  // a NaN whose payload is cut stays one
-}
-__device__ __forceinline__ uint32_t hi16x2(uint32_t a, uint32_t b) {  // (a >> 16) | (b & 0xffff0000)
-    return __builtin_amdgcn_perm(b, a, 0x07060302u);
-}
-
-template <int TERMS, int WM, int MT>
+// KV: the expansion of the MLA latent cache into keys and values.  A weight tile is one head's
+// kv_b rows, 128 key rows (waves wn == 0) then 128 value rows (wn == 1, WN == 2), and the results
+// are stored as three bf16 terms in the order the attention reads them; the value waves swap
+// the MFMA operands, so a lane ends with four consecutive tokens of one value column.
+template <int TERMS, int WM, int MT, bool KV>
 __global__ __launch_bounds__(kThreads, 2) void dense_kernel(DenseArgs a) {
     constexpr int WN = 8 / WM, NT = kBN / WN / 16, BM = WM * MT * 16;
     constexpr int kW = kBN * 128, kA = BM * 128, kStage = kW + TERMS * kA;
@@ -165,7 +159,7 @@ __global__ __launch_bounds__(kThreads, 2) void dense_kernel(DenseArgs a) {
 #pragma unroll
             for (int i = 0; i < MT; ++i) av[t][i] = *reinterpret_cast<const bf16x8 *>(A + t * kA + i * 2048 + c);
     };
-    auto multiply = [&] {
+    auto multiply = [&](auto swap) {
         __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int t = TERMS - 1; t >= 0; --t)
@@ -173,7 +167,8 @@ __global__ __launch_bounds__(kThreads, 2) void dense_kernel(DenseArgs a) {
             for (int j = 0; j < NT; ++j)
 #pragma unroll
                 for (int i = 0; i < MT; ++i)
-                    acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[j], av[t][i], acc[j][i], 0, 0, 0);
+                    acc[j][i] = swap ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[t][i], wv[j], acc[j][i], 0, 0, 0)
+                                           : __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[j], av[t][i], acc[j][i], 0, 0, 0);
         __builtin_amdgcn_s_setprio(0);
     };
     auto phase = [&] {
@@ -196,23 +191,56 @@ __global__ __launch_bounds__(kThreads, 2) void dense_kernel(DenseArgs a) {
     load_a(1);
     phase();
     if (late) phase();
-    for (int S = 0; S < NS; ++S) {
-        const int buf = S & 1;
-        read(buf, 0);
-        store_w(buf ^ 1);
-        load_w(S + 2);
-        phase();
-        split();
-        multiply();
-        phase();
-        read(buf, 1);
-        store_a(buf ^ 1);
-        load_a(S + 2);
-        phase();
-        multiply();
-        phase();
+    auto steps = [&](auto swap) {
+        for (int S = 0; S < NS; ++S) {
+            const int buf = S & 1;
+            read(buf, 0);
+            store_w(buf ^ 1);
+            load_w(S + 2);
+            phase();
+            split();
+            multiply(swap);
+            phase();
+            read(buf, 1);
+            store_a(buf ^ 1);
+            load_a(S + 2);
+            phase();
+            multiply(swap);
+            phase();
+        }
+    };
+    if constexpr (KV) {
+        if (wn)  // (uniform per wave; both sides meet the same barriers)
+            steps(std::true_type{});
+        else
+            steps(std::false_type{});
+    } else {
+        steps(std::false_type{});
     }
     if (!late) phase();
+
+    if constexpr (KV) {
+        static_assert(WN == 2, "one wave column per half of a head's rows");
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            const int mt0 = m0 + (wm * MT + i) * 16, key = mt0 + (wn ? 4 * q : r16);
+            if (key < a.tpad) {
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    uint32_t t[3][4];
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) split3(acc[j][i][x], t[0][x], t[1][x], t[2][x]);
+#pragma unroll
+                    for (int x = 0; x < 3; ++x) {
+                        uint16_t *dst = wn ? a.vt + mla_v_index(ntile, a.tpad, x, 16 * j + r16, mt0) + q * 8
+                                           : a.kp + mla_k_index(ntile, a.tpad, key, x) + 16 * j + 4 * q;
+                        *reinterpret_cast<uint2 *>(dst) = make_uint2(hi16x2(t[x][0], t[x][1]), hi16x2(t[x][2], t[x][3]));
+                    }
+                }
+            }
+        }
+        return;
+    }
 
     // ---- lane: outputs n0 + 16 j + 4q .. + 3 of token r16
 #pragma unroll
@@ -277,15 +305,15 @@ Plan make_plan(int64_t M, int64_t K, int nt, bool f32) {
     return p;
 }
 
-template <int TERMS, int WM, int MT>
+template <int TERMS, int WM, int MT, bool KV = false>
 int launch_dense(const DenseArgs &a, hipStream_t st) {
     constexpr int BM = WM * MT * 16, bytes = 2 * (kBN * 128 + TERMS * BM * 128);
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&dense_kernel<TERMS, WM, MT>),
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&dense_kernel<TERMS, WM, MT, KV>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     int rc = check_hip(attr, "dense: LDS size attribute");
     if (rc) return rc;
     const int64_t total = static_cast<int64_t>(a.mt) * a.nt * a.ksplit;
-    dense_kernel<TERMS, WM, MT><<<dim3(static_cast<unsigned>(8 * cdiv(total, 8))), kThreads, bytes, st>>>(a);
+    dense_kernel<TERMS, WM, MT, KV><<<dim3(static_cast<unsigned>(8 * cdiv(total, 8))), kThreads, bytes, st>>>(a);
     rc = check_hip(hipGetLastError(), "dense launch");
     if (rc || a.ksplit == 1) return rc;
     const int64_t threads = static_cast<int64_t>(a.M) * a.nt * (kBN / 4);
@@ -330,6 +358,20 @@ __global__ __launch_bounds__(256) void act_rows_kernel(const float *g, const flo
 }
 
 }  // namespace
+
+int mla_expand_kv(const void *lat, int cache_dtype, int64_t ld_lat, const void *kv_b, int64_t Tk, int64_t heads,
+                  uint16_t *kp, uint16_t *vt, int64_t tpad, hipStream_t st) {
+    DenseArgs d{};
+    d.a = lat, d.lda = ld_lat, d.M = static_cast<int>(Tk), d.K = 512;
+    d.w[0] = static_cast<const uint16_t *>(kv_b);
+    d.N[0] = static_cast<int>(heads * 256);
+    d.nt = static_cast<int>(heads), d.nseg = 1, d.ksplit = 1, d.ksteps = 512 / kBK;
+    d.kp = kp, d.vt = vt, d.tpad = static_cast<int>(tpad);
+    const bool f32 = cache_dtype == K3_F32;
+    d.mt = static_cast<int>(cdiv(Tk, 128));
+    return f32 ? launch_dense<3, 4, 2, true>(d, st) : launch_dense<1, 4, 2, true>(d, st);
+}
+
 }  // namespace k3
 
 using namespace k3;

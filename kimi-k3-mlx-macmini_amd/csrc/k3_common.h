@@ -30,6 +30,21 @@ int mla_decode_core(const void *q_nope, const void *q_rot, int64_t ld_q, int64_t
                     int64_t v_dim, float scale, void *out, int out_dtype, int64_t ld_out, const float *gate,
                     void *workspace, int64_t workspace_bytes, void *stream, int cache_dtype = K3_BF16);
 
+// The multi-token MLA attention's keys and values: every head's expansion of the latent cache,
+// as three bf16 terms.  tpad: the tokens rounded up to 32 (the added ones are zero).
+//   keys    [heads][tpad][3][128]
+//   values  [heads][tpad / 32][3][128 columns][32 tokens], the tokens of a block in the order of
+//           the P V product's reduction: slot 8 q + 4 h + v holds token 16 h + 4 q + v
+__host__ __device__ inline int64_t mla_k_index(int64_t head, int64_t tpad, int64_t key, int term) {
+    return ((head * tpad + key) * 3 + term) * 128;
+}
+// index of (value column, first slot of q == 0) for the 16-token tile that starts at `token`
+__host__ __device__ inline int64_t mla_v_index(int64_t head, int64_t tpad, int term, int col, int64_t token) {
+    return (((head * (tpad >> 5) + (token >> 5)) * 3 + term) * 128 + col) * 32 + ((token >> 4) & 1) * 4;
+}
+int mla_expand_kv(const void *lat, int cache_dtype, int64_t ld_lat, const void *kv_b, int64_t Tk, int64_t heads,
+                  uint16_t *kp, uint16_t *vt, int64_t tpad, hipStream_t st);
+
 // ---------------------------------------------------------------- bf16 <-> f32
 __device__ __forceinline__ float bf16_to_f32(uint16_t b) {
     return __uint_as_float(static_cast<uint32_t>(b) << 16);
@@ -40,6 +55,19 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
     if ((u & 0x7fffffffu) > 0x7f800000u) return static_cast<uint16_t>((u >> 16) | 0x40u);
     u += 0x7fffu + ((u >> 16) & 1u);
     return static_cast<uint16_t>(u >> 16);
+}
+
+// fp32 -> three bf16 terms (upper halves of t1, t2, t3); infinities and NaNs stay in the first
+__device__ __forceinline__ void split3(float v, uint32_t &t1, uint32_t &t2, uint32_t &t3) {
+    const uint32_t u = __float_as_uint(v);
+    t1 = u & 0xffff0000u;
+    const float r = (u & 0x7f800000u) == 0x7f800000u ? 0.f : v - __uint_as_float(t1);
+    t2 = __float_as_uint(r) & 0xffff0000u;
+    t3 = __float_as_uint(r - __uint_as_float(t2));
+    if ((u & 0x7fffffffu) > 0x7f800000u) t1 |= 0x00400000u;  // a NaN whose payload is cut stays one
+}
+__device__ __forceinline__ uint32_t hi16x2(uint32_t a, uint32_t b) {  // (a >> 16) | (b & 0xffff0000)
+    return __builtin_amdgcn_perm(b, a, 0x07060302u);
 }
 
 // E8M0 byte -> float32 2^(b-127).  Byte 0 is the subnormal 2^-127, byte 255 is +inf

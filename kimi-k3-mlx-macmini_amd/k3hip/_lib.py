@@ -59,6 +59,9 @@ SIGNATURES: dict[str, list] = {
     "k3_kda_step_workspace_size": [_I64],
     "k3_kda_step_decode": [_P, _I32, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I32,
                            _I64, _I64, _I64, _I64, _F32, _F32, _P, _I64, _P],
+    "k3_mla_prefill_workspace_size": [_I64, _I64],
+    "k3_mla_prefill": [_P, _I64, _P, _P, _I64, _P, _I64, _I32, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64,
+                       _F32, _P, _I64, _P],
     "k3_kda_prefill_inputs": [_P] * 21 + [_I64] * 5 + [_F32, _P],
     "k3_kda_gated_norm": [_P, _P, _P, _F32, _P, _I64, _I64, _I64, _I64, _P],
     "k3_dense_workspace_size": [_I64, _I64, _P, _I64, _I32],
@@ -90,6 +93,7 @@ _RESTYPE = {"k3_last_error": ctypes.c_char_p, "k3_version": ctypes.c_char_p,
             "k3_mla_step_workspace_size": ctypes.c_int64,
             "k3_kda_step_workspace_size": ctypes.c_int64,
             "k3_dense_workspace_size": ctypes.c_int64,
+            "k3_mla_prefill_workspace_size": ctypes.c_int64,
             "k3_moe_grouped_workspace_size": ctypes.c_int64,
             "k3_moe_routed_workspace_size": ctypes.c_int64,
             "k3_moe_layer_multi_workspace_size": ctypes.c_int64,

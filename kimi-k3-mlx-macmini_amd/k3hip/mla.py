@@ -17,8 +17,10 @@ by default: the kernel reads the valid prefix directly, so ``view`` does not upc
 bf16 projection weights (the checkpoint dtype) the decode step (one token, batch 1) is
 ``k3_mla_step_decode``: the projections, RMSNorms, cache append, attention core, output
 gate and o_proj in seven HIP launches.  With other weight dtypes the projections are torch
-fp32 matmuls around the HIP core.  Prefill (T > 1) keeps the reference's dense masked form
-in torch on the GPU.
+fp32 matmuls around the HIP core.  Prefill (T > 1) runs the projections of all tokens
+(``_blas.project``) and the causal attention over keys and values expanded from the cache
+(``k3_mla_prefill``); fp32 weights, batches and other widths keep the reference's dense
+masked form in torch.
 
 The cache defaults to bf16 (``cfg.mla_cache_dtype``), which the HIP core reads in place; the
 reference's default is an fp32 cache (``attention_mla.py:164``), which it calls lossless.
@@ -26,7 +28,7 @@ An fp32 cache (``mla_cache_dtype=torch.float32``, or a caller's fp32 ``MLACache`
 accepted: a decode token on it runs the HIP core on the fp32 rows
 (``k3_mla_decode_absorbed_f32``; with bf16 ``kv_b``, the checkpoint dtype, whose halves the
 core takes as they are), the projections around it in fp32; fp32 ``kv_b`` (validation mode)
-and prefill run the fp32 masked form.
+runs the fp32 masked form.
 """
 from __future__ import annotations
 
@@ -34,7 +36,7 @@ from dataclasses import dataclass
 
 import torch
 
-from . import _lib, _workspace
+from . import _blas, _lib, _workspace
 from . import _torch as T
 
 CACHE_STEP = 256
@@ -191,6 +193,17 @@ def _rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
     return w.to(torch.float32) * (xf * torch.rsqrt((xf * xf).mean(-1, keepdim=True) + eps))
 
 
+def _rmsnorm_rows(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
+    """_rmsnorm of the rows of an fp32 [M, K] device tensor in one launch."""
+    M, K = x.shape
+    w = T.contiguous_aligned(w.to(torch.float32))
+    if K % 4 or x.stride(1) != 1 or x.stride(0) % 4 or x.data_ptr() % 16 or M == 0:
+        return _rmsnorm(x, w, eps)
+    out = torch.empty((M, K), dtype=torch.float32, device=x.device)
+    _lib.call("k3_rmsnorm_rows", T.ptr(x), x.stride(0) if M > 1 else K, T.ptr(w), float(eps), T.ptr(out), M, K, T.stream(x))
+    return out
+
+
 class MLAAttention:
     """Drop-in for MLAAttention (attention_mla.py:137-216).  Weights are the checkpoint
     tensors as-is ([out, in], applied as x @ W.T), on the GPU."""
@@ -244,11 +257,23 @@ class MLAAttention:
         nh, qhd, vhd = c.num_attention_heads, c.q_head_dim, c.v_head_dim
         nope, rope, klr = c.qk_nope_head_dim, c.qk_rope_head_dim, c.kv_lora_rank
         eps = c.rms_norm_eps
-        q = self._mm(_rmsnorm(self._mm(x, self.q_a), self.q_an, eps), self.q_b)
-        q = q.reshape(B, Tn, nh, qhd).transpose(1, 2)               # [B, H, T, qhd]
-        ckv = self._mm(x, self.kv_a)
-        c_new = _rmsnorm(ckv[..., :klr], self.kv_an, eps)
-        r_new = ckv[..., klr:]
+        gated = bool(getattr(c, "mla_use_output_gate", False))
+        mats = [self.q_a, self.kv_a] + ([self.g_w] if gated else [])
+        xf = x.reshape(B * Tn, x.shape[-1])
+        if B * Tn > 1 and _blas.dense_ok(xf, *mats) and _blas.weights_ok(self.q_b, self.o_w):
+            qa, ckv, *g = _blas.project(xf, mats)
+            qa = _rmsnorm_rows(qa, self.q_an, eps)
+            q = _blas.project(qa, [self.q_b])[0].reshape(B, Tn, nh, qhd)
+            c_new = _rmsnorm_rows(ckv[:, :klr], self.kv_an, eps).reshape(B, Tn, klr)
+            r_new = ckv[:, klr:].reshape(B, Tn, -1)
+            gate = g[0].reshape(B, Tn, nh * vhd) if gated else None
+            mm = lambda a, w: _blas.project(a.reshape(B * Tn, -1), [w])[0].reshape(B, Tn, -1)  # noqa: E731
+        else:
+            mm = self._mm
+            q = mm(_rmsnorm(mm(x, self.q_a), self.q_an, eps), self.q_b).reshape(B, Tn, nh, qhd)
+            ckv = mm(x, self.kv_a)
+            c_new, r_new = _rmsnorm(ckv[..., :klr], self.kv_an, eps), ckv[..., klr:]
+            gate = mm(x, self.g_w) if gated else None
         if cache is None:
             cache = new_cache(B, klr, rope, Tn, self.cache_dtype, x.device)
         cache.append(c_new, r_new)
@@ -259,13 +284,50 @@ class MLAAttention:
         # since the core takes W_UK / W_UV in bf16
         if Tn == 1 and B == 1 and (lat.dtype == torch.bfloat16 or
                                    (lat.dtype == torch.float32 and self.kv_b.dtype == torch.bfloat16)):
-            o = mla_decode_absorbed(q[0, :, 0, :nope], q[0, :, 0, nope:], self.wk, self.wv,
+            o = mla_decode_absorbed(q[0, 0, :, :nope], q[0, 0, :, nope:], self.wk, self.wv,
                                     lat[0], rot[0], scale).reshape(1, 1, nh * vhd)
+        elif self._expanded_ok(q, lat, rot):
+            o, gate = self._expanded(q, lat[0], rot[0], scale, gate), None
         else:
-            o = self._dense(q, lat, rot, scale).transpose(1, 2).reshape(B, Tn, nh * vhd)
-        if getattr(c, "mla_use_output_gate", False):
-            o = o * torch.sigmoid(self._mm(x, self.g_w))
-        return self._mm(o, self.o_w), cache
+            o = self._dense(q.transpose(1, 2), lat, rot, scale).transpose(1, 2).reshape(B, Tn, nh * vhd)
+        if gate is not None:
+            o = o * torch.sigmoid(gate)
+        return mm(o, self.o_w), cache
+
+    # The expanded form forms every head's keys and values of all Tk cached positions, the
+    # absorbed form 3.4 times the work per (query, position): with few queries over a long
+    # cache the latter is less.
+    EXPAND_QUERIES, EXPAND_POSITIONS = 16, 4096
+
+    def _expanded_ok(self, q, lat, rot) -> bool:
+        c = self.cfg
+        B, Tn = q.shape[:2]
+        if torch.is_grad_enabled() and (q.requires_grad or lat.requires_grad or self.kv_b.requires_grad):
+            return False
+        return (B == 1 and Tn > 1 and q.is_cuda and q.dtype == torch.float32 and lat.dtype == rot.dtype
+                and lat.dtype in (torch.bfloat16, torch.float32) and self.kv_b.dtype == torch.bfloat16
+                and self.kv_b.is_contiguous() and self.kv_b.data_ptr() % 16 == 0
+                and (c.kv_lora_rank, c.qk_rope_head_dim, c.qk_nope_head_dim, c.v_head_dim) == (KV_LORA_RANK, ROPE_DIM, 128, 128)
+                and c.q_head_dim == 192
+                and (Tn >= self.EXPAND_QUERIES or lat.shape[1] <= self.EXPAND_POSITIONS))
+
+    def _expanded(self, q, lat, rot, scale, gate):
+        """Multi-token form (prefill) of one sequence through k3_mla_prefill: q [1, T, H, 192] fp32 over the
+        cache rows, causal, times the sigmoid of gate [1, T, H * v] if given -> [1, T, H * v]."""
+        c = self.cfg
+        Tn, nh, vhd = q.shape[1], c.num_attention_heads, c.v_head_dim
+        lat = _cache_rows(lat, c.kv_lora_rank, "lat")
+        rot = _cache_rows(rot, c.qk_rope_head_dim, "rot")
+        T.require_device(q, lat, rot, self.kv_b, gate)
+        q = T.contiguous_aligned(q)
+        gate = None if gate is None else T.contiguous_aligned(gate)
+        out = torch.empty((1, Tn, nh * vhd), dtype=torch.float32, device=q.device)
+        nbytes = int(_lib.lib().k3_mla_prefill_workspace_size(lat.shape[0], nh))
+        ws = _workspace.get(q.device, nbytes, "mla_prefill")
+        _lib.call("k3_mla_prefill", T.ptr(q), nh * c.q_head_dim, T.ptr(self.kv_b), T.ptr(lat), lat.stride(0), T.ptr(rot),
+                  rot.stride(0), T.dtype_code(lat.dtype), T.ptr(gate), T.ptr(out), Tn, lat.shape[0], nh, c.kv_lora_rank,
+                  c.qk_rope_head_dim, c.qk_nope_head_dim, vhd, float(scale), T.ptr(ws), ws.numel(), T.stream(q))
+        return out
 
     def decode_step(self, x: torch.Tensor, cache: MLACache | None = None):
         """One token at batch 1 through k3_mla_step_decode (attention_mla.py:168-216): the

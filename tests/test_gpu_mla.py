@@ -471,3 +471,61 @@ def test_mla_fused_decode_step_other_shapes(hidden, heads, q_lora, gate):
         worst = max(worst, om.normwise_rel(o.float().cpu().numpy().reshape(-1), oo @ w["o_proj.weight"].T))
     print(f"hidden={hidden} heads={heads} q_lora={q_lora} gate={gate}: {worst:.2e}")
     assert worst <= 1e-4
+
+
+@pytest.mark.parametrize("T,past,heads,cache,gate", [(2, 0, 4, torch.bfloat16, True), (31, 1, 16, torch.float32, False),
+                                                     (128, 0, 3, torch.bfloat16, False), (129, 287, 8, torch.float32, True),
+                                                     (300, 33, 8, torch.bfloat16, True), (17, 4200, 16, torch.bfloat16, False)])
+def test_mla_many_tokens_match_fp64(T, past, heads, cache, gate):
+    """k3_mla_prefill (query tiles of 128, 16 per wave, steps of 32 cached tokens, both cache
+    dtypes, past lengths that leave part steps) against the masked form in fp64 over the same
+    cache rows.  Six products of three-term operands leave 2^-24 of a product, so the error is
+    that of fp32 sums of 192 and 128 (context of up to 4217) products: 1e-5 normwise."""
+    from types import SimpleNamespace
+    from k3hip.mla import MLAAttention, new_cache
+    g = torch.Generator(device=DEV)
+    g.manual_seed(T + past)
+    rn = lambda *s: torch.randn(*s, device=DEV, generator=g)  # noqa: E731
+    hid, ql = 256, 512
+    lin = lambda o, i: (rn(o, i) * i ** -0.5).to(torch.bfloat16)  # noqa: E731
+    w = {"q_a_proj.weight": lin(ql, hid), "q_a_layernorm.weight": 1 + 0.1 * rn(ql), "q_b_proj.weight": lin(heads * 192, ql),
+         "kv_a_proj_with_mqa.weight": lin(576, hid), "kv_a_layernorm.weight": 1 + 0.1 * rn(512),
+         "kv_b_proj.weight": lin(heads * 256, 512), "g_proj.weight": lin(heads * 128, hid),
+         "o_proj.weight": lin(hid, heads * 128)}
+    cfg = SimpleNamespace(hidden_size=hid, num_attention_heads=heads, q_lora_rank=ql, kv_lora_rank=512, qk_nope_head_dim=128,
+                          qk_rope_head_dim=64, v_head_dim=128, q_head_dim=192, rms_norm_eps=1e-5, mla_use_output_gate=gate,
+                          mla_cache_dtype=cache)
+    attn = MLAAttention(cfg, w)
+    Tk = past + T
+    lat, rot, q = rn(1, Tk, 512).to(cache), rn(1, Tk, 64).to(cache), rn(1, T, heads, 192)
+    gl = rn(1, T, heads * 128)
+    assert attn._expanded_ok(q, lat, rot)
+    got = attn._expanded(q, lat[0], rot[0], 192 ** -0.5, gl if gate else None)
+    kb = w["kv_b_proj.weight"].double().view(heads, 256, 512)
+    ld, rd, qd = lat[0].double(), rot[0].double(), q[0].double()
+    s = (torch.einsum("thd,hdr->htr", qd[..., :128].cpu(), kb[:, :128].cpu()) @ ld.T.cpu()
+         + qd[..., 128:].transpose(0, 1).cpu() @ rd.T.cpu()) * 192 ** -0.5
+    mask = torch.arange(Tk)[None] > torch.arange(past, Tk)[:, None]
+    ctx = torch.softmax(s.masked_fill(mask, float("-inf")), -1) @ ld.cpu()
+    want = torch.einsum("htr,hvr->thv", ctx, kb[:, 128:].cpu()).reshape(T, -1)
+    if gate:
+        want = want * torch.sigmoid(gl[0].double().cpu())
+    rel = float((got[0].double().cpu() - want).norm() / want.norm())
+    old = attn._dense(q.transpose(1, 2), lat, rot, 192 ** -0.5).transpose(1, 2).reshape(T, -1)
+    if gate:
+        old = old * torch.sigmoid(gl[0])
+    ref = float((old.double().cpu() - want).norm() / want.norm())
+    print(f"T={T} past={past} H={heads} {cache}: rel {rel:.2e} (fp32 masked form {ref:.2e})")
+    assert rel <= 1e-5
+    # the whole call: tokens in one call, then the cache it leaves continues with one more
+    x = rn(1, T, hid).to(torch.bfloat16)
+    if past:
+        c = new_cache(1, 512, 64, Tk, cache, DEV).append(lat[:, :past], rot[:, :past])
+        out, c2 = attn(x, c)
+    else:
+        out, c2 = attn(x)
+    assert c2.length == Tk and torch.isfinite(out).all()
+    # row T - 1 alone, through the one-token core on the same cache
+    c2.length = Tk - 1
+    one, _ = attn(x[:, -1:], c2)
+    assert float((one[0, 0] - out[0, -1]).norm() / out[0, -1].norm()) <= 2e-3
