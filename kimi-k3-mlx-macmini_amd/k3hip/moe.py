@@ -260,16 +260,25 @@ class RoutedMoE:
         u = self._proj(h, e, "w3")
         return self._proj(_act_torch(g.float(), u.float(), act, beta, lb), e, "w2")
 
-    def shared_forward(self, x: torch.Tensor) -> torch.Tensor:
-        """Shared expert on the original hidden state (moe.py:105-107).  Fused: exact
+    def shared_forward(self, x: torch.Tensor, add: torch.Tensor | None = None) -> torch.Tensor:
+        """Shared expert on the original hidden state (moe.py:105-107), plus ``add`` [M, H] fp32
+        if given.  Fused: exact
         products with fp32 accumulation and fp32 intermediates on the BLAS library, no weight
         copy (inside a decode step it runs in the layer kernels).  Unfused: the reference's
         dtype promotion (a bf16 input against bf16 weights gives bf16 gate / up)."""
         act, beta, lb = self._act()
+        mats = [self.sh_gate, self.sh_up]
+        flat = x.reshape(-1, x.shape[-1])
+        if self.fused and flat.shape[0] and _blas.dense_ok(flat, *mats) and _blas.weights_ok(self.sh_down):
+            g, u = _blas.project(flat, mats)
+            _lib.call("k3_act_rows", T.ptr(g), T.ptr(u), T.ptr(g), g.numel(), _act_code(act), float(beta),
+                      float(lb or 0.0), T.stream(g))
+            return _blas.dense(g, [self.sh_down], add)[0].reshape(x.shape)
         mm = _blas.mm_f32 if self.fused else _blas.mm_ref
         g = mm(x, self.sh_gate)
         u = mm(x, self.sh_up)
-        return mm(_act_torch(g.float(), u.float(), act, beta, lb), self.sh_down).float()
+        y = mm(_act_torch(g.float(), u.float(), act, beta, lb), self.sh_down).float()
+        return y if add is None else y + add
 
     def _combine_loop(self, h: torch.Tensor, r: RouterResult, width: int) -> torch.Tensor:
         """The reference's dispatch loop (moe.py:119-127): for each distinct routed expert,
@@ -314,7 +323,7 @@ class RoutedMoE:
         y = routed_fn(flat, router.expert_indices, router.expert_weights, self.expert_table(), self._I,
                       act, beta, lb, out_dtype=torch.float32, validate=validate)
         if self.sh_gate is not None:
-            y = y + self.shared_forward(flat)
+            y = self.shared_forward(flat, y)
         return y.to(out_dtype).reshape(*orig[:-1], self._H)
 
     def __call__(self, x: torch.Tensor, return_router: bool = False, out_dtype=torch.float32):
@@ -401,6 +410,16 @@ def _rmsnorm32(y: torch.Tensor, w32: torch.Tensor, eps: float) -> torch.Tensor:
     return w32 * (y * torch.rsqrt((y * y).mean(dim=-1, keepdim=True) + eps))
 
 
+def _rmsnorm_rows(y: torch.Tensor, w32: torch.Tensor, eps: float) -> torch.Tensor:
+    """_rmsnorm32 of the contiguous rows of an fp32 [M, K] device tensor in one launch."""
+    M, K = y.shape
+    if M == 0 or K % 4 or not y.is_contiguous() or y.data_ptr() % 16 or w32.data_ptr() % 16 or y.dtype != torch.float32:
+        return _rmsnorm32(y, w32, eps)
+    out = torch.empty_like(y)
+    _lib.call("k3_rmsnorm_rows", T.ptr(y), K, T.ptr(w32), eps, T.ptr(out), M, K, T.stream(y))
+    return out
+
+
 class LatentMoE:
     """Drop-in for K3's routed layer, LatentMoE (air_llm/models/kimi_k3/moe.py:40-132).
 
@@ -468,9 +487,9 @@ class LatentMoE:
         """One routed expert on latent rows h [N, L] (moe.py:90-103)."""
         return self._routed.expert_forward(h, e)
 
-    def shared_forward(self, x: torch.Tensor) -> torch.Tensor:
-        """Shared expert(s) on the original hidden state (moe.py:105-107)."""
-        return self._routed.shared_forward(x)
+    def shared_forward(self, x: torch.Tensor, add: torch.Tensor | None = None) -> torch.Tensor:
+        """Shared expert(s) on the original hidden state (moe.py:105-107), plus ``add`` if given."""
+        return self._routed.shared_forward(x, add)
 
     def __call__(self, x: torch.Tensor, return_router: bool = False, out_dtype=torch.float32):
         orig = x.shape
@@ -584,10 +603,10 @@ class LatentMoE:
         act, beta, lb = self._routed._act()
         y = routed_fn(h.contiguous(), r.expert_indices, r.expert_weights, self._routed.expert_table(),
                       int(c.moe_intermediate_size), act, beta, lb, out_dtype=torch.float32, validate=False)
-        y = _rmsnorm32(y, self._norm32, float(c.rms_norm_eps))
+        y = _rmsnorm_rows(y, self._norm32, float(c.rms_norm_eps))
         y = _blas.mm_f32(y, self.up)                                      # latent -> hidden
         if self._routed.sh_gate is not None:
-            y = y + self.shared_forward(flat)
+            y = self.shared_forward(flat, y)
         y = y.to(out_dtype).reshape(*orig[:-1], orig[-1])
         return (y, r) if return_router else y
 
