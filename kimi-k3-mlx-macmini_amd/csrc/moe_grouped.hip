@@ -131,6 +131,26 @@ __device__ __forceinline__ void bf16_split2(float v, uint16_t &hi, uint16_t &lo)
     lo = (hi & 0x7f80u) == 0x7f80u ? 0 : f32_to_bf16(v - h);
 }
 
+// The activation of moe_common.h's act_fn in straight-line code on the hardware's exp2 and
+// reciprocal (each within one unit in the last place): about 1e-6 relative, against the 2^-17
+// its two-term storage keeps.
+__device__ __forceinline__ float fast_sigmoid(float x) {
+    return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * x));
+}
+__device__ __forceinline__ float fast_tanh(float x) {
+    const float a = fabsf(x), e = __builtin_amdgcn_exp2f(-2.8853900817779268f * a), s = x * x;
+    // below 1/4 the difference 1 - e cancels: the Taylor polynomial, next term 2e-2 x^8
+    const float p = x * (1.0f + s * (-0.33333333f + s * (0.13333333f - s * 0.053968254f)));
+    return a < 0.25f ? p : copysignf((1.0f - e) * __builtin_amdgcn_rcpf(1.0f + e), x);
+}
+__device__ __forceinline__ float fast_act(float g, float u, int kind, float beta, float ibeta, float lbeta, float ilbeta) {
+    if (kind == K3_ACT_SITU) {
+        const float a = beta * fast_tanh(g * ibeta) * fast_sigmoid(g);
+        return a * (lbeta > 0.f ? lbeta * fast_tanh(u * ilbeta) : u);
+    }
+    return g * fast_sigmoid(g) * u;
+}
+
 // A two-term row: per 128 elements, 128 hi values then 128 lo values (512 bytes), so one
 // staging step of the GEMM reads 512 contiguous bytes per row in either form.
 constexpr int kBlk = 128;
@@ -277,14 +297,17 @@ __device__ __forceinline__ void grouped_tile(const GemmArgs &a, char *lds, int n
         RS4 = buf_load4(rs, off + 16u);
     };
     // LDS row of A: 16-byte unit p = 4 kg + q holds what lane (., q) of wave group kg takes in
-    // the step, dwords 2kg, 2kg + 1 of groups q and 4 + q
+    // the step, dwords 2kg, 2kg + 1 of groups q and 4 + q.  The units of neighbouring rows are
+    // XOR-ed apart, the low row bit on the top unit bit, so the 8-byte stores of two rows (half
+    // a row each) meet different banks, as do eight rows' 16-byte reads of one unit.
+    auto aswz = [](int R) { return ((R & 1) << 2) | ((R >> 1) & 3); };
     auto store_a = [&](int set, int buf) {
 #pragma unroll
         for (int n = 0; n < 4; ++n) {
             const int R = wave * 32 + 8 * n + (lane >> 3);
             char *row = lds + buf * kABuf + R * 128 + (ac >> 2) * 8;
-            *reinterpret_cast<uint2 *>(row + (((ac & 3) ^ (R & 7)) << 4)) = make_uint2(RA[set][n].x, RA[set][n].y);
-            *reinterpret_cast<uint2 *>(row + (((4 + (ac & 3)) ^ (R & 7)) << 4)) = make_uint2(RA[set][n].z, RA[set][n].w);
+            *reinterpret_cast<uint2 *>(row + (((ac & 3) ^ aswz(R)) << 4)) = make_uint2(RA[set][n].x, RA[set][n].y);
+            *reinterpret_cast<uint2 *>(row + (((4 + (ac & 3)) ^ aswz(R)) << 4)) = make_uint2(RA[set][n].z, RA[set][n].w);
         }
     };
     auto store_b = [&](int set, int buf) {
@@ -344,7 +367,7 @@ __device__ __forceinline__ void grouped_tile(const GemmArgs &a, char *lds, int n
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             wv[j] = *reinterpret_cast<const uint4 *>(lds + abuf * kABuf + arow[j] * 128 +
-                                                     (((4 * kg + q) ^ (arow[j] & 7)) << 4));
+                                                     (((4 * kg + q) ^ aswz(arow[j])) << 4));
     };
     auto compute = [&](int P, int h, int bbuf) {
         const char *B = lds + kLdsB + bbuf * kBBuf;
@@ -446,6 +469,7 @@ __device__ __forceinline__ void grouped_tile(const GemmArgs &a, char *lds, int n
         }
     __syncthreads();
     // (C: lane holds weight rows 4q + v of each A tile, column r16 of each column group)
+    const float ib = 1.0f / a.beta, il = 1.0f / a.lbeta;
 #pragma unroll
     for (int ct = 0; ct < NCT; ++ct) {
         const int rr = ct * 16 + r16;
@@ -468,7 +492,7 @@ __device__ __forceinline__ void grouped_tile(const GemmArgs &a, char *lds, int n
                     uint16_t hi[4], lo[4];
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
-                        bf16_split2(act_fn(acc[j][ct][i], acc[j + 2][ct][i], a.act_kind, a.beta, a.lbeta), hi[i], lo[i]);
+                        bf16_split2(fast_act(acc[j][ct][i], acc[j + 2][ct][i], a.act_kind, a.beta, ib, a.lbeta, il), hi[i], lo[i]);
                     *reinterpret_cast<uint2 *>(dst + 16 * j) =
                         make_uint2(hi[0] | (static_cast<uint32_t>(hi[1]) << 16), hi[2] | (static_cast<uint32_t>(hi[3]) << 16));
                     *reinterpret_cast<uint2 *>(dst + kBlk + 16 * j) =
