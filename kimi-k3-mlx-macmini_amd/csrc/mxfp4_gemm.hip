@@ -1,0 +1,209 @@
+// MXFP4 matmul for the tokens gathered for one expert (more than a GEMV's four): y[M, N] =
+// x[M, K] w[N, K]^T, w E2M1 with one E8M0 scale per 32, on the bf16 matrix cores.
+//
+// Reference: the Metal kernel takes M tokens in one call (air_llm/kernels/metal/
+// mxfp4_matvec.py:89-95).  The GEMV form runs four tokens per launch and reads the weights once
+// per launch: at 37 tokens ten launches.
+//
+// One 32-element group is one K step of v_mfma_f32_16x16x32_bf16: the codes become bf16
+// unscaled (exact), bf16 x is exact and fp32 x enters as three bf16 terms whose sum is exact
+// (split3), and each group's sum is scaled once by its power-of-two scale as it is added to
+// the fp32 total, as in the GEMV.
+//
+// Block: R weight rows x 16 TT tokens, eight waves, WR over the rows and 8 / WR over the groups of
+// a step (their sums meet in LDS at the end).  Operands load line-contiguous into registers, two
+// steps ahead, and go through LDS (x in 16-byte chunks XOR-swizzled by the row).  What bounds a
+// small call is latency and the x rows every block reads, so R is 16 while that gives less
+// than two blocks per CU, else 64.
+// @@MM@@
+#include <algorithm>
+
+#include "k3_common.h"
+#include "mxfp4_gemv.h"
+
+namespace k3 {
+namespace {
+
+constexpr int kThreads = 512;
+constexpr int kMaxScale = 16 * 1024;   // LDS bytes for a block's scale rows
+constexpr uint32_t kOob = 0xf0000000u;
+
+template <int TERMS, int WR, int TT>
+struct Shape {
+    static constexpr int R = 16 * WR, WK = 8 / WR;
+    static constexpr int KC = TERMS == 1 ? 256 : 128;            // elements per step
+    static constexpr int G = KC / 32, GW = G / WK > 0 ? G / WK : 1;  // groups per step, per wave
+    static constexpr int XT = 16 * TT * KC * 2;                  // bytes of one x term
+    static constexpr int W = R * KC / 2;
+    static constexpr int Stage = TERMS * XT + W;
+    static constexpr int Acc = 8 * TT * 1024;                    // the waves' sums
+    static constexpr int lds(int scale) { return std::max(2 * Stage, Acc) + scale; }
+};
+
+template <int TERMS, int WR, int TT>
+__global__ __launch_bounds__(kThreads, 2) void mxfp4_gemm_kernel(GemvArgs a) {
+    using Sh = Shape<TERMS, WR, TT>;
+    constexpr int KC = Sh::KC, G = Sh::G, GW = Sh::GW, WK = Sh::WK;
+    extern __shared__ char lds[];
+    char *const sc = lds + (2 * Sh::Stage > Sh::Acc ? 2 * Sh::Stage : Sh::Acc);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wr = wave % WR, wk = wave / WR, r16 = lane & 15, q = lane >> 4;
+    const int K = static_cast<int>(a.K), KB = K >> 5, NS = (K + KC - 1) / KC;
+    const int64_t n0 = static_cast<int64_t>(blockIdx.x) * Sh::R;
+    const int m0 = blockIdx.y * 16 * TT;
+    const int nrows = static_cast<int>(a.N - n0 < Sh::R ? a.N - n0 : Sh::R), mrows = min(16 * TT, a.M - m0);
+
+    // ---- loads.  x: KC * element size bytes per row and step, 16-byte chunks
+    constexpr int ES = TERMS == 1 ? 2 : 4, XC = KC * ES / 16;        // chunks per x row: 32
+    constexpr int XR = kThreads / XC, NX = 16 * TT / XR;             // rows per pass, passes
+    const int xc = tid % XC, xr = tid / XC;
+    const auto rx = make_rsrc(static_cast<const char *>(a.x) + static_cast<int64_t>(m0) * a.ldx * ES,
+                              static_cast<uint32_t>(static_cast<int64_t>(mrows) * a.ldx * ES));
+    constexpr int WC = KC / 32;                                      // 16-byte chunks per weight row: 8 or 4
+    const int wc = tid % WC, wrow = tid / WC;                        // rows past R: no load
+    const uint32_t row_bytes = static_cast<uint32_t>(K >> 1);
+    const auto rw = make_rsrc(static_cast<const char *>(a.packed) + n0 * row_bytes, static_cast<uint32_t>(nrows) * row_bytes);
+    uint4 RX[2][NX], RW[2];
+    auto load = [&](int s, int set) {
+        const bool xok = (s * XC + xc) * (16 / ES) < K, wok = wrow < nrows && s * WC + wc < KB;
+#pragma unroll
+        for (int n = 0; n < NX; ++n) {
+            const int row = xr + n * XR;
+            RX[set][n] = buf_load16(rx, xok && row < mrows ? static_cast<uint32_t>(row * a.ldx * ES) + (s * XC + xc) * 16u : kOob);
+        }
+        RW[set] = buf_load16_nt(rw, wok ? wrow * row_bytes + (s * WC + wc) * 16u : kOob);
+    };
+    auto store = [&](int set, int buf) {
+        char *X = lds + buf * Sh::Stage, *W = X + TERMS * Sh::XT;
+#pragma unroll
+        for (int n = 0; n < NX; ++n) {
+            const int row = xr + n * XR;
+            const uint4 v = RX[set][n];
+            if constexpr (TERMS == 1) {
+                *reinterpret_cast<uint4 *>(X + row * (KC * 2) + ((xc ^ (row & 7)) << 4)) = v;
+            } else {
+                const uint32_t f[4] = {v.x, v.y, v.z, v.w};
+                uint32_t t[3][4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) split3(__uint_as_float(f[i]), t[0][i], t[1][i], t[2][i]);
+                char *p = X + row * (KC * 2) + (((xc >> 1) ^ (row & 7)) << 4) + (xc & 1) * 8;
+#pragma unroll
+                for (int x = 0; x < 3; ++x)
+                    *reinterpret_cast<uint2 *>(p + x * Sh::XT) = make_uint2(hi16x2(t[x][0], t[x][1]), hi16x2(t[x][2], t[x][3]));
+            }
+        }
+        if (wrow < Sh::R) *reinterpret_cast<uint4 *>(W + wrow * (KC / 2) + ((wc ^ (wrow & (WC - 1))) << 4)) = RW[set];
+    };
+    load(0, 0);
+    load(1, 1);
+    // all scales of the block's rows: one contiguous run of bytes, copied as aligned dwords
+    const uintptr_t s0 = reinterpret_cast<uintptr_t>(a.scales) + static_cast<uintptr_t>(n0) * KB;
+    const int sdelta = static_cast<int>(s0 & 3u), sdw = (nrows * KB + sdelta + 3) >> 2;
+    const uint32_t *sp = reinterpret_cast<const uint32_t *>(s0 - sdelta);
+    for (int i = tid; i < sdw; i += kThreads) reinterpret_cast<uint32_t *>(sc)[i] = sp[i];
+    store(0, 0);
+    load(2, 0);
+
+    f32x4 acc[TT];
+#pragma unroll
+    for (int t = 0; t < TT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int wl = wr * 16 + r16;                                    // this lane's weight row
+    auto compute = [&](int s, int buf) {
+        const char *X = lds + buf * Sh::Stage, *W = X + TERMS * Sh::XT;
+#pragma unroll
+        for (int j = 0; j < GW; ++j) {
+            const int g = wk * GW + j;                               // group of the step
+            if (G < WK && g >= G) break;
+            if (s * G + g >= KB) break;
+            const uint32_t w = *reinterpret_cast<const uint32_t *>(W + wl * (KC / 2) + ((g ^ (wl & (WC - 1))) << 4) + 4 * q);
+            const float scale = e8m0_to_f32(static_cast<uint8_t>(sc[sdelta + min(wl, nrows - 1) * KB + s * G + g]));
+            const uint4 wv4 = make_uint4(__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, 1.0f, 0)),
+                                         __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, 1.0f, 1)),
+                                         __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, 1.0f, 2)),
+                                         __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, 1.0f, 3)));
+            const bf16x8 wv = __builtin_bit_cast(bf16x8, wv4);
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+                const char *p = X + (16 * t + r16) * (KC * 2) + (((4 * g + q) ^ (r16 & 7)) << 4);
+                f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int x = TERMS - 1; x >= 0; --x)
+                    v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8 *>(p + x * Sh::XT), wv, v, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[t][i] = fmaf(v[i], scale, acc[t][i]);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int s = 0;; s += 2) {
+        __syncthreads();
+        compute(s, 0);
+        if (s + 1 >= NS) break;
+        store(1, 1);
+        load(s + 3, 1);
+        __syncthreads();
+        compute(s + 1, 1);
+        if (s + 2 >= NS) break;
+        store(0, 0);
+        load(s + 4, 0);
+    }
+
+    // ---- the waves' sums, added in order: wave (wr, wk) leaves [wk][wr][t][lane]
+    __syncthreads();
+    f32x4 *part = reinterpret_cast<f32x4 *>(lds);
+#pragma unroll
+    for (int t = 0; t < TT; ++t) part[((wk * WR + wr) * TT + t) * 64 + lane] = acc[t];
+    __syncthreads();
+    for (int id = tid; id < WR * TT * 64; id += kThreads) {
+        f32x4 v = part[id];
+        for (int k = 1; k < WK; ++k) v += part[k * (WR * TT * 64) + id];
+        const int ln = id & 63, t = (id >> 6) % TT, w = (id >> 6) / TT;
+        const int64_t n = n0 + w * 16 + (ln & 15);
+        if (n < a.N) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int m = m0 + 16 * t + 4 * (ln >> 4) + i;
+                if (m < a.M) {
+                    if (a.out_bf16)
+                        static_cast<uint16_t *>(a.out)[m * a.ldo + n] = f32_to_bf16(v[i]);
+                    else
+                        static_cast<float *>(a.out)[m * a.ldo + n] = v[i];
+                }
+            }
+        }
+    }
+}
+
+template <int TERMS, int WR, int TT>
+int launch(const GemvArgs &a, hipStream_t st) {
+    using Sh = Shape<TERMS, WR, TT>;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&mxfp4_gemm_kernel<TERMS, WR, TT>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, Sh::lds(kMaxScale));
+    const int rc = check_hip(attr, "mxfp4 matmul: LDS size attribute");
+    if (rc) return rc;
+    const int scale = static_cast<int>((Sh::R * (a.K / 32) + 7 + 15) & ~15);
+    mxfp4_gemm_kernel<TERMS, WR, TT><<<dim3(static_cast<unsigned>(cdiv(a.N, Sh::R)), static_cast<unsigned>(cdiv(a.M, 16 * TT))),
+                                       kThreads, Sh::lds(scale), st>>>(a);
+    return check_hip(hipGetLastError(), "mxfp4 matmul launch");
+}
+
+template <int TERMS, int WR>
+int launch_tt(const GemvArgs &a, hipStream_t st) {
+    if (a.M <= 16) return launch<TERMS, WR, 1>(a, st);
+    if (a.M <= 32) return launch<TERMS, WR, 2>(a, st);
+    return launch<TERMS, WR, 4>(a, st);
+}
+
+}  // namespace
+
+bool mxfp4_gemm_takes(int64_t M, int64_t N, int64_t K) {
+    return M > 4 && M <= 64 * 65535 && N < (1ll << 31) && 16 * (K / 32) + 32 <= kMaxScale && K * 64 * 4 < (1ll << 31);
+}
+
+int mxfp4_gemm_launch(const GemvArgs &a, hipStream_t st) {
+    const bool wide = 64 * (a.K / 32) + 32 <= kMaxScale && cdiv(a.N, 16) * cdiv(a.M, 64) >= 2 * 256;
+    if (a.x_bf16) return wide ? launch_tt<1, 4>(a, st) : launch_tt<1, 1>(a, st);
+    return wide ? launch_tt<3, 4>(a, st) : launch_tt<3, 1>(a, st);
+}
+
+}  // namespace k3

@@ -271,6 +271,13 @@ static int matvec_impl(const void *x, int x_dtype, const void *packed, const voi
         return set_error(K3_ERR_SHAPE, "mxfp4 matvec: K=%lld exceeds the %d-element activation tile", (long long)K,
                          x_dtype == K3_BF16 ? 32768 : 16384);
     auto st = static_cast<hipStream_t>(stream);
+    if (mxfp4_gemm_takes(M, N, K)) {
+        GemvArgs a{};
+        a.x = x, a.ldx = K, a.packed = packed, a.scales = scales, a.out = out, a.ldo = N;
+        a.M = static_cast<int>(M), a.N = N, a.K = K;
+        a.x_bf16 = x_dtype == K3_BF16, a.out_bf16 = out_dtype == K3_BF16;
+        return mxfp4_gemm_launch(a, st);
+    }
     for (int64_t m0 = 0; m0 < M; m0 += mt) {  // token tiles share one weight pass
         GemvArgs a{};
         a.x = static_cast<const char *>(x) + m0 * K * xsz;

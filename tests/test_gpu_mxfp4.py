@@ -204,3 +204,33 @@ def test_unfused_path_matches_definition():
     # result carries one bf16 output rounding on top of the exact contraction
     want = om.matvec_unfused_f64(x32, packed, scales)
     assert np.all(np.abs(got - want) <= np.abs(want) * 2.0 ** -8 + 1e-6)
+
+
+# token tiles of 16 / 32 / 64 and their remainders, row tiles of 16 (few blocks) and 64 (many),
+# K of whole and part steps (256 for bf16 x, 128 for fp32 x)
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("m,n,k", [(5, 1, 32), (16, 17, 96), (17, 300, 288), (33, 64, 3584), (65, 3001, 7168),
+                                   (256, 8192, 256), (37, 40000, 544), (130, 5000, 1056)])
+def test_matmul_many_tokens(m, n, k, xdt):
+    """k3_mxfp4_matvec beyond four tokens: exact products, fp32 sums in another order than the
+    GEMV's, so at most k 2^-24 of the sum of |products| and in practice far below: 1e-6 of it."""
+    from k3hip.mxfp4_matvec import mxfp4_matvec_fused
+    g = torch.Generator(device=DEV)
+    g.manual_seed(m * 31 + n)
+    x = torch.randn(m, k, device=DEV, generator=g).to(xdt)
+    packed = torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device=DEV, generator=g)
+    buf = torch.randint(2, 253, (n * (k // 32) + 3,), dtype=torch.uint8, device=DEV, generator=g)
+    lut = torch.tensor([0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0], dtype=torch.float64, device=DEV)
+    lut = torch.cat([lut, -lut])
+    codes = torch.stack([packed & 15, packed >> 4], dim=-1).flatten(1).int()
+    for lo, hi, off in ((110, 135, 0), (110, 135, 3), (2, 6, 1), (249, 253, 0)):   # scale bytes, their alignment
+        buf.random_(lo, hi, generator=g)
+        scales = buf[off:off + n * (k // 32)].view(n, k // 32)
+        xs = x if hi < 200 else x * 2.0 ** -20
+        y = mxfp4_matvec_fused(xs, packed, scales)
+        w = lut[codes] * torch.exp2(scales.double() - 127).repeat_interleave(32, dim=1)
+        want, mag = xs.double() @ w.T, xs.double().abs() @ w.abs().T
+        assert float(((y.double() - want).abs() / mag.clamp_min(1e-300)).max()) <= 1e-6, (lo, off)
+        assert torch.equal(y, mxfp4_matvec_fused(xs, packed, scales))
+    b = mxfp4_matvec_fused(xs, packed, scales, out_dtype=torch.bfloat16)
+    assert torch.equal(b, y.to(torch.bfloat16))
