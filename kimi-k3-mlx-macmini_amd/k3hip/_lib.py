@@ -9,6 +9,7 @@ problems, as ``air_llm/kernels/metal/mxfp4_matvec.py:85-86`` and
 from __future__ import annotations
 
 import ctypes
+import functools
 import threading
 from pathlib import Path
 
@@ -129,9 +130,15 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_fns: dict = {}   # entry points by name, once the library is loaded
+
+
 def call(name: str, *args) -> None:
     """Call a k3_* entry point and turn a nonzero status into an exception."""
-    rc = getattr(lib(), name)(*args)
+    fn = _fns.get(name)
+    if fn is None:
+        fn = _fns[name] = getattr(lib(), name)
+    rc = fn(*args)
     if rc != K3_OK:
         msg = lib().k3_last_error().decode(errors="replace")
         if rc in (K3_ERR_SHAPE, K3_ERR_SCALE_RANGE, K3_ERR_ALIGN, K3_ERR_WORKSPACE, K3_ERR_NULL):
@@ -139,6 +146,12 @@ def call(name: str, *args) -> None:
         if rc == K3_ERR_DTYPE:
             raise TypeError(msg)
         raise RuntimeError(msg)
+
+
+@functools.lru_cache(maxsize=1024)
+def size(name: str, *args: int) -> int:
+    """A k3_*_workspace_size of whole-number arguments (a function of them alone)."""
+    return int(getattr(lib(), name)(*args))
 
 
 def exported_symbols() -> list[str]:

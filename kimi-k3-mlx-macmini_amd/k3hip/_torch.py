@@ -1,8 +1,6 @@
 """Torch tensor plumbing for the C-ABI: device pointers, dtype enums and streams."""
 from __future__ import annotations
 
-import ctypes
-
 import torch
 
 from . import _lib
@@ -17,13 +15,24 @@ def dtype_code(dt: torch.dtype) -> int:
         raise TypeError(f"unsupported dtype {dt}; k3hip takes float32 or bfloat16") from None
 
 
-def ptr(t: torch.Tensor | None):
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+def ptr(t: torch.Tensor | None) -> int:
+    """The device address (0 for None), as the ctypes argument types take it."""
+    return 0 if t is None else t.data_ptr()
 
 
-def stream(t: torch.Tensor):
-    """The current HIP stream of t's device, as a void*."""
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+# The raw handle of the current stream, without the Stream object that
+# torch.cuda.current_stream builds around it (about 1 us per call).
+_raw_stream = torch._C._cuda_getCurrentRawStream
+
+
+def stream(t: torch.Tensor) -> int:
+    """The current HIP stream of t's device."""
+    return _raw_stream(t.get_device())
+
+
+def stream_of(device: torch.device) -> int:
+    """The current HIP stream of a device (the current device where it has no index)."""
+    return _raw_stream(torch.cuda.current_device() if device.index is None else device.index)
 
 
 def require_device(*ts: torch.Tensor) -> None:
@@ -31,12 +40,13 @@ def require_device(*ts: torch.Tensor) -> None:
     for t in ts:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise ValueError(f"k3hip kernels take device tensors; got {t.device}")
+        d = t.get_device()
         if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise ValueError(f"tensors on different devices: {dev} vs {t.device}")
+            dev, first = d, t
+        elif d != dev:
+            raise ValueError(f"tensors on different devices: {first.device} vs {t.device}")
 
 
 def contiguous_aligned(t: torch.Tensor) -> torch.Tensor:

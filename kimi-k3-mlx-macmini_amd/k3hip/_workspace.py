@@ -11,14 +11,15 @@ import threading
 
 import torch
 
+from . import _torch as T
+
 _lock = threading.Lock()
 _cache: dict[tuple, torch.Tensor] = {}
 
 
 def get(device: torch.device, nbytes: int, tag: str = "") -> torch.Tensor:
     """A zero-initialised uint8 device buffer of at least nbytes for the current stream."""
-    stream = torch.cuda.current_stream(device).cuda_stream
-    key = (device.index, stream, tag)
+    key = (device.index, T.stream_of(device), tag)
     with _lock:
         buf = _cache.get(key)
         if buf is None or buf.numel() < nbytes:

@@ -90,7 +90,7 @@ class KDAAttention:
         """One token of one sequence: x1 [hidden], state [H, D, D] fp32 (in place),
         conv_in / conv_out [3, k-1, H*D] fp32, out [hidden] fp32."""
         c = self.cfg
-        nbytes = int(_lib.lib().k3_kda_step_workspace_size(self.H))
+        nbytes = _lib.size("k3_kda_step_workspace_size", self.H)
         ws = _workspace.get(x1.device, nbytes, "kda_step")
         _lib.call("k3_kda_step_decode", T.ptr(x1), T.dtype_code(x1.dtype), T.ptr(self.q_w), T.ptr(self.k_w),
                   T.ptr(self.v_w), T.ptr(self.g_w), T.ptr(self.o_w), T.ptr(self.fa), T.ptr(self.fb), T.ptr(self.b_w),

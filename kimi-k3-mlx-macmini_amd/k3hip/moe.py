@@ -41,9 +41,9 @@ def expert_ffn_fused(x: torch.Tensor, gate, up, down, act: str = "silu", beta: f
     if x2.dtype not in (torch.float32, torch.bfloat16):
         x2 = x2.to(torch.float32)
     x2 = T.contiguous_aligned(x2)
-    gp, upk, dp = (T.contiguous_aligned(t) for t in (gp, upk, dp))
-    gs, us, ds = (t.contiguous() for t in (gs, us, ds))
-    ws_bytes = int(_lib.lib().k3_expert_ffn_workspace_size(I))
+    gp, upk, dp = T.contiguous_aligned(gp), T.contiguous_aligned(upk), T.contiguous_aligned(dp)
+    gs, us, ds = gs.contiguous(), us.contiguous(), ds.contiguous()
+    ws_bytes = _lib.size("k3_expert_ffn_workspace_size", I)
     ws = _workspace.get(x2.device, ws_bytes, "expert_ffn")
     out = torch.empty((1, H), dtype=out_dtype, device=x2.device)
     _lib.call("k3_expert_ffn", T.ptr(x2), T.dtype_code(x2.dtype), T.ptr(gp), T.ptr(gs), T.ptr(upk),
@@ -206,7 +206,7 @@ class RoutedMoE:
         return self._table
 
     def _workspace(self):
-        nbytes = int(_lib.lib().k3_moe_layer_workspace_size(self._H, self._I, self._Is, self._E, self._k))
+        nbytes = _lib.size("k3_moe_layer_workspace_size", self._H, self._I, self._Is, self._E, self._k)
         return _workspace.get(self.device, nbytes, "moe_layer")
 
     def _records(self, ws: torch.Tensor) -> RouterResult:
@@ -381,7 +381,7 @@ class RoutedMoE:
         x = flat if flat.dtype in (torch.float32, torch.bfloat16) else flat.to(torch.float32)
         x = T.contiguous_aligned(x)
         H, I, Is, E, k = self._H, self._I, self._Is, self._E, self._k
-        nbytes = int(_lib.lib().k3_moe_layer_multi_workspace_size(n, H, I, Is, E, k))
+        nbytes = _lib.size("k3_moe_layer_multi_workspace_size", n, H, I, Is, E, k)
         ws = _workspace.get(self.device, nbytes, "moe_layer_multi")
         out = torch.empty((n, H), dtype=out_dtype, device=self.device)
         _lib.call("k3_moe_layer_decode_multi", T.ptr(x), T.dtype_code(x.dtype), T.ptr(self.gate_w), T.ptr(bias),
@@ -522,7 +522,7 @@ class LatentMoE:
         act, beta, lb = R._act()
         table = R.expert_table()
         H, Lw, I, Is, E, k = R._H, self.latent, R._I, R._Is, R._E, R._k
-        nbytes = int(_lib.lib().k3_moe_latent_layer_workspace_size(H, Lw, I, Is, E, k))
+        nbytes = _lib.size("k3_moe_latent_layer_workspace_size", H, Lw, I, Is, E, k)
         outs, recs = [], []
         for t in range(flat.shape[0]):
             xt = R._x1(flat[t])
@@ -555,7 +555,7 @@ class LatentMoE:
         x = flat if flat.dtype in (torch.float32, torch.bfloat16) else flat.to(torch.float32)
         x = T.contiguous_aligned(x)
         H, Lw, I, Is, E, k = R._H, self.latent, R._I, R._Is, R._E, R._k
-        nbytes = int(_lib.lib().k3_moe_latent_layer_multi_workspace_size(n, H, Lw, I, Is, E, k))
+        nbytes = _lib.size("k3_moe_latent_layer_multi_workspace_size", n, H, Lw, I, Is, E, k)
         ws = _workspace.get(R.device, nbytes, "moe_latent_multi")
         out = torch.empty((n, H), dtype=out_dtype, device=R.device)
         _lib.call("k3_moe_latent_layer_decode_multi", T.ptr(x), T.dtype_code(x.dtype), T.ptr(R.gate_w),
@@ -640,7 +640,7 @@ def moe_grouped_ffn(x: torch.Tensor, expert_indices: torch.Tensor, expert_weight
     out = torch.empty((n_tok, H), dtype=out_dtype, device=x.device)
     if n_tok == 0:
         return out
-    nbytes = int(_lib.lib().k3_moe_grouped_workspace_size(n_tok, k, E, H, intermediate))
+    nbytes = _lib.size("k3_moe_grouped_workspace_size", n_tok, k, E, H, intermediate)
     ws = _workspace.get(x.device, nbytes, "moe_grouped")
     _lib.call("k3_moe_grouped_ffn", T.ptr(x), T.dtype_code(x.dtype), T.ptr(idx), T.ptr(w), T.ptr(table),
               T.ptr(out), T.dtype_code(out_dtype), n_tok, H, intermediate, E, k, _act_code(act), float(beta),
@@ -678,7 +678,7 @@ def moe_routed_decode(x: torch.Tensor, expert_indices: torch.Tensor, expert_weig
     out = torch.empty((n_tok, H), dtype=out_dtype, device=x.device)
     if n_tok == 0:
         return out
-    nbytes = int(_lib.lib().k3_moe_routed_workspace_size(n_tok, H, intermediate, E, k))
+    nbytes = _lib.size("k3_moe_routed_workspace_size", n_tok, H, intermediate, E, k)
     ws = _workspace.get(x.device, nbytes, "moe_routed")
     _lib.call("k3_moe_routed_decode", T.ptr(x), T.dtype_code(x.dtype), T.ptr(idx), T.ptr(w), T.ptr(table),
               T.ptr(out), T.dtype_code(out_dtype), n_tok, H, intermediate, E, k, _act_code(act), float(beta),

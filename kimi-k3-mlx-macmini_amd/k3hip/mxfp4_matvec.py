@@ -28,21 +28,22 @@ def mxfp4_matvec_fused(x: torch.Tensor, packed: torch.Tensor, scales: torch.Tens
     """y = x @ W.T with W given by (packed, scales); fp32 accumulation."""
     if x.dim() != 2:
         raise ValueError(f"x must be [M, K]; got shape {tuple(x.shape)}")
-    M = x.shape[0]
-    N = packed.shape[0]
-    if packed.shape[1] * 2 != x.shape[1]:
-        raise ValueError(f"K mismatch: x has {x.shape[1]}, packed implies {packed.shape[1] * 2}")
+    M, K = x.shape
+    pshape = packed.shape
+    N = pshape[0]
+    if pshape[1] * 2 != K:
+        raise ValueError(f"K mismatch: x has {K}, packed implies {pshape[1] * 2}")
     if packed.dtype != torch.uint8 or scales.dtype != torch.uint8:
         raise TypeError("packed and scales must be uint8")
-    if tuple(scales.shape) != (N, x.shape[1] // 32) or x.shape[1] % 32:
-        raise ValueError(f"scales shape {tuple(scales.shape)} does not match K={x.shape[1]}")
+    if scales.shape != (N, K // 32) or K % 32:
+        raise ValueError(f"scales shape {tuple(scales.shape)} does not match K={K}")
     T.require_device(x, packed, scales)
     x = _prep_x(x)
     packed = T.contiguous_aligned(packed)
     scales = scales.contiguous()
     out = torch.empty((M, N), dtype=out_dtype, device=x.device)
-    _lib.call("k3_mxfp4_matvec", T.ptr(x), T.dtype_code(x.dtype), T.ptr(packed), T.ptr(scales), T.ptr(out),
-              T.dtype_code(out_dtype), M, N, x.shape[1], T.stream(x))
+    _lib.call("k3_mxfp4_matvec", x.data_ptr(), T.dtype_code(x.dtype), packed.data_ptr(), scales.data_ptr(),
+              out.data_ptr(), T.dtype_code(out_dtype), M, N, K, T.stream(x))
     return out
 
 
