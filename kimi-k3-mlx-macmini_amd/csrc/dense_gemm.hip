@@ -147,6 +147,24 @@ __global__ __launch_bounds__(kThreads, 2) void dense_kernel(DenseArgs a) {
     for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (int i = 0; i < MT; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // Few tokens (BM 32, where registers are free): each step's sum of 64 products goes into a
+    // sum of eight steps and that into the total, and the second and third terms have sums of
+    // their own, so a long K rounds no more than the one-token row kernels' trees do.
+    constexpr bool kFold = WM == 1;
+    constexpr int FN = kFold ? NT : 1, FM = kFold ? MT : 1;
+    f32x4 tot[FN][FM], mid[FN][FM], lo[FN][FM];
+    if constexpr (kFold) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) tot[j][i] = mid[j][i] = lo[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    auto fold = [](f32x4 (&from)[NT][MT], f32x4 (&to)[NT][MT]) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) to[j][i] += from[j][i], from[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    };
     bf16x8 wv[NT], av[TERMS][MT];
     auto read = [&](int buf, int kk) {
         const char *W = lds + buf * kStage + (wn * NT * 16 + r16) * 128;
@@ -166,9 +184,11 @@ __global__ __launch_bounds__(kThreads, 2) void dense_kernel(DenseArgs a) {
 #pragma unroll
             for (int j = 0; j < NT; ++j)
 #pragma unroll
-                for (int i = 0; i < MT; ++i)
-                    acc[j][i] = swap ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[t][i], wv[j], acc[j][i], 0, 0, 0)
-                                           : __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[j], av[t][i], acc[j][i], 0, 0, 0);
+                for (int i = 0; i < MT; ++i) {
+                    f32x4 &c = kFold && t ? lo[kFold ? j : 0][kFold ? i : 0] : acc[j][i];
+                    c = swap ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[t][i], wv[j], c, 0, 0, 0)
+                             : __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[j], av[t][i], c, 0, 0, 0);
+                }
         __builtin_amdgcn_s_setprio(0);
     };
     auto phase = [&] {
@@ -206,6 +226,10 @@ __global__ __launch_bounds__(kThreads, 2) void dense_kernel(DenseArgs a) {
             load_a(S + 2);
             phase();
             multiply(swap);
+            if constexpr (kFold) {
+                fold(acc, mid);
+                if ((S & 7) == 7) fold(mid, tot);
+            }
             phase();
         }
     };
@@ -218,6 +242,12 @@ __global__ __launch_bounds__(kThreads, 2) void dense_kernel(DenseArgs a) {
         steps(std::false_type{});
     }
     if (!late) phase();
+    if constexpr (kFold) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) acc[j][i] = (tot[j][i] + mid[j][i]) + lo[j][i];
+    }
 
     if constexpr (KV) {
         static_assert(WN == 2, "one wave column per half of a head's rows");

@@ -31,7 +31,10 @@ constexpr uint32_t kOob = 0xf0000000u;
 template <int TERMS, int WR, int TT>
 struct Shape {
     static constexpr int R = 16 * WR, WK = 8 / WR;
-    static constexpr int KC = TERMS == 1 ? 256 : 128;            // elements per step
+    // elements per step: what two steps of x leave room for in LDS (a step costs a barrier and
+    // an LDS round trip whatever its length), and one 16-byte weight load per thread
+    static constexpr int KC = WR == 4 ? (TERMS == 1 ? 256 : 128)
+                                      : TERMS == 1 ? (TT >= 3 ? 512 : 1024) : (TT >= 3 ? 128 : 512 / TT);
     static constexpr int G = KC / 32, GW = G / WK > 0 ? G / WK : 1;  // groups per step, per wave
     static constexpr int XT = 16 * TT * KC * 2;                  // bytes of one x term
     static constexpr int W = R * KC / 2;
@@ -104,9 +107,11 @@ __global__ __launch_bounds__(kThreads, 2) void mxfp4_gemm_kernel(GemvArgs a) {
     store(0, 0);
     load(2, 0);
 
-    f32x4 acc[TT];
+    // two sums per output, alternate groups in each, and the waves' sums added pairwise: as
+    // little rounding as the GEMV's lane sums and tree
+    f32x4 acc[2][TT];
 #pragma unroll
-    for (int t = 0; t < TT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < TT; ++t) acc[0][t] = acc[1][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int wl = wr * 16 + r16;                                    // this lane's weight row
     auto compute = [&](int s, int buf) {
         const char *X = lds + buf * Sh::Stage, *W = X + TERMS * Sh::XT;
@@ -130,7 +135,10 @@ __global__ __launch_bounds__(kThreads, 2) void mxfp4_gemm_kernel(GemvArgs a) {
                 for (int x = TERMS - 1; x >= 0; --x)
                     v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8 *>(p + x * Sh::XT), wv, v, 0, 0, 0);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) acc[t][i] = fmaf(v[i], scale, acc[t][i]);
+                for (int i = 0; i < 4; ++i) {
+                    f32x4 &c = acc[GW == 1 ? buf : j & 1][t];
+                    c[i] = fmaf(v[i], scale, c[i]);
+                }
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -148,15 +156,19 @@ __global__ __launch_bounds__(kThreads, 2) void mxfp4_gemm_kernel(GemvArgs a) {
         load(s + 4, 0);
     }
 
-    // ---- the waves' sums, added in order: wave (wr, wk) leaves [wk][wr][t][lane]
+    static_assert(WK == 8 || WK == 2, "the sum below");
+    // ---- the waves' sums: wave (wr, wk) leaves [wk][wr][t][lane]
     __syncthreads();
     f32x4 *part = reinterpret_cast<f32x4 *>(lds);
 #pragma unroll
-    for (int t = 0; t < TT; ++t) part[((wk * WR + wr) * TT + t) * 64 + lane] = acc[t];
+    for (int t = 0; t < TT; ++t) part[((wk * WR + wr) * TT + t) * 64 + lane] = acc[0][t] + acc[1][t];
     __syncthreads();
     for (int id = tid; id < WR * TT * 64; id += kThreads) {
-        f32x4 v = part[id];
-        for (int k = 1; k < WK; ++k) v += part[k * (WR * TT * 64) + id];
+        constexpr int kStep = WR * TT * 64;
+        f32x4 v = part[id] + part[kStep + id];
+        if constexpr (WK == 8)
+            v = (v + (part[2 * kStep + id] + part[3 * kStep + id])) +
+                ((part[4 * kStep + id] + part[5 * kStep + id]) + (part[6 * kStep + id] + part[7 * kStep + id]));
         const int ln = id & 63, t = (id >> 6) % TT, w = (id >> 6) / TT;
         const int64_t n = n0 + w * 16 + (ln & 15);
         if (n < a.N) {
@@ -191,6 +203,7 @@ template <int TERMS, int WR>
 int launch_tt(const GemvArgs &a, hipStream_t st) {
     if (a.M <= 16) return launch<TERMS, WR, 1>(a, st);
     if (a.M <= 32) return launch<TERMS, WR, 2>(a, st);
+    if (a.M <= 48) return launch<TERMS, WR, 3>(a, st);
     return launch<TERMS, WR, 4>(a, st);
 }
 

@@ -206,11 +206,11 @@ def test_unfused_path_matches_definition():
     assert np.all(np.abs(got - want) <= np.abs(want) * 2.0 ** -8 + 1e-6)
 
 
-# token tiles of 16 / 32 / 64 and their remainders, row tiles of 16 (few blocks) and 64 (many),
+# token tiles of 16 / 32 / 48 / 64 and their remainders, row tiles of 16 (few blocks) and 64 (many),
 # K of whole and part steps (256 for bf16 x, 128 for fp32 x)
 @pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("m,n,k", [(5, 1, 32), (16, 17, 96), (17, 300, 288), (33, 64, 3584), (65, 3001, 7168),
-                                   (256, 8192, 256), (37, 40000, 544), (130, 5000, 1056)])
+                                   (256, 8192, 256), (37, 40000, 544), (48, 100, 1056), (130, 5000, 1056)])
 def test_matmul_many_tokens(m, n, k, xdt):
     """k3_mxfp4_matvec beyond four tokens: exact products, fp32 sums in another order than the
     GEMV's, so at most k 2^-24 of the sum of |products| and in practice far below: 1e-6 of it."""
