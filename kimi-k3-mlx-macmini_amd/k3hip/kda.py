@@ -116,10 +116,10 @@ class KDAAttention:
         if B * Tn <= 32:
             yq, yk, yv, og, fa, br = _blas.project(xf, mats)
         else:
-            # the gates' small matrices on their own, where their reduction is split over blocks:
-            # exp(A_log) multiplies their rounding (the state's error 1.1e-6 -> 8.5e-7, for 20 us)
+            # exp(A_log) multiplies the rounding of the gates' matrices: they take the library's
+            # split reduction (the state's error 1.1e-6 -> 8.5e-7 of 64 bits, for 20 us)
             yq, yk, yv, og = _blas.project(xf, mats[:4])
-            fa, br = _blas.project(xf, mats[4:])
+            fa, br = (_blas.mm_f32(xf, w) for w in mats[4:])
         fb = _blas.project(fa, [self.fb])[0]
         wins = [None] * 3 if conv is None else [
             T.contiguous_aligned(conv[m].detach().to(torch.float32).reshape(B, K - 1, P)) for m in range(3)]
@@ -151,17 +151,21 @@ class KDAAttention:
             raise ValueError(f"state must be [{B}, {H}, {D}, {D}]; got {tuple(state.shape)}")
         elif not (state.dtype == torch.float32 and state.is_contiguous() and state.data_ptr() % 16 == 0):
             state = state.to(torch.float32).contiguous().clone()
-        bufs = [torch.zeros((B, 3, K - 1, P), dtype=torch.float32, device=x.device) for _ in range(2)]
-        if conv is not None:
-            for m in range(3):
-                bufs[0][:, m] = conv[m].to(torch.float32).reshape(B, K - 1, P)
+        # the windows of q, k and v in one buffer (one launch, or none where a caller passes back
+        # the views a call returned); the step writes every element of the next ones
+        fin = torch.empty((1, 3, K - 1, P), dtype=torch.float32, device=x.device)
+        if conv is None:
+            cin = torch.zeros((3, K - 1, P), dtype=torch.float32, device=x.device)
+        else:
+            wins = [c.to(torch.float32).reshape(1, K - 1, P) for c in conv]
+            step = (K - 1) * P * 4
+            T.require_device(x, *wins)
+            if (all(c.is_contiguous() for c in wins) and wins[0].data_ptr() % 16 == 0
+                    and all(wins[m].data_ptr() == wins[0].data_ptr() + m * step for m in (1, 2))):
+                cin = wins[0]
+            else:
+                cin = torch.cat(wins)
         xin = x if x.dtype in (torch.float32, torch.bfloat16) else x.to(torch.float32)
-        xin = xin.contiguous()
-        out = torch.empty((B, Tn, hid), dtype=torch.float32, device=x.device)
-        for t in range(Tn):
-            cin, cout = bufs[t % 2], bufs[(t + 1) % 2]
-            for b in range(B):
-                x1 = T.contiguous_aligned(xin[b, t])
-                self.decode_step(x1, state[b], cin[b], cout[b], out[b, t])
-        fin = bufs[Tn % 2]
+        out = torch.empty((1, 1, hid), dtype=torch.float32, device=x.device)
+        self.decode_step(T.contiguous_aligned(xin[0, 0]), state[0], cin, fin[0], out[0, 0])
         return out, state, (fin[:, 0], fin[:, 1], fin[:, 2])
