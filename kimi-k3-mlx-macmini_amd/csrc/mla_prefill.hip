@@ -137,7 +137,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
         char *L = lds + buf * kStage;
 #pragma unroll
         for (int x = 0; x < 3; ++x) {
-            *reinterpret_cast<uint4 *>(L + x * kK + (tid >> 4) * 256 + (((tid & 15) ^ ((tid >> 4) & 7)) << 4)) = RK[x];
+            *reinterpret_cast<uint4 *>(L + x * kK + (tid >> 4) * 256 + (((tid & 15) ^ ((tid >> 4) & 15)) << 4)) = RK[x];
             *reinterpret_cast<uint4 *>(L + kOffV + x * kVt + (tid >> 2) * 64 + (((tid & 3) ^ ((tid >> 3) & 3)) << 4)) = RV[x];
         }
         if (wave < 4) {
@@ -167,7 +167,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
                 const int row = 16 * h + r16;
 #pragma unroll
                 for (int x = 0; x < kTerms[ks >= 4]; ++x)
-                    kf[h][x] = ks < 4 ? *reinterpret_cast<const bf16x8 *>(L + x * kK + row * 256 + (((4 * ks + q) ^ (row & 7)) << 4))
+                    kf[h][x] = ks < 4 ? *reinterpret_cast<const bf16x8 *>(L + x * kK + row * 256 + (((4 * ks + q) ^ (row & 15)) << 4))
                                       : *reinterpret_cast<const bf16x8 *>(L + kOffR + x * kR + row * 128 +
                                                                           (((4 * (ks - 4) + q) ^ (row & 7)) << 4));
             }

@@ -297,24 +297,29 @@ __device__ __forceinline__ void grouped_tile(const GemmArgs &a, char *lds, int n
         RS4 = buf_load4(rs, off + 16u);
     };
     // LDS row of A: 16-byte unit p = 4 kg + q holds what lane (., q) of wave group kg takes in
-    // the step, dwords 2kg, 2kg + 1 of groups q and 4 + q.  The units of neighbouring rows are
-    // XOR-ed apart, the low row bit on the top unit bit, so the 8-byte stores of two rows (half
-    // a row each) meet different banks, as do eight rows' 16-byte reads of one unit.
-    auto aswz = [](int R) { return ((R & 1) << 2) | ((R >> 1) & 3); };
+    // the step, dwords 2kg, 2kg + 1 of groups q and 4 + q.
+    // The XOR keys: a 16-byte LDS read runs 16 lanes at a time over all 64 banks, lanes 0-3,
+    // 12-15 and 20-27 together (and 4-11, 16-19, 28-31), so the operand rows 0-3, 12-15 of one
+    // q meet rows 4-11 of the next q.  akey sends both sets to different units, and
+    // neighbouring row pairs' 8-byte stores to different halves; bkey does it for B's rows,
+    // whose chunks of neighbouring q are 4 apart.  (3-bit keys of the row: 2-way conflicts,
+    // 124 instead of 228 B/clk.)
+    auto akey = [](int R) { return ((R & 2) << 1) | (((R >> 2) ^ (R >> 3)) & 1) << 1 | ((R >> 3) & 1); };
+    auto bkey = [](int R) { return (((R >> 2) ^ (R >> 3)) & 1) << 3 | ((R >> 3) & 1) << 2 | (R & 3); };
     auto store_a = [&](int set, int buf) {
 #pragma unroll
         for (int n = 0; n < 4; ++n) {
             const int R = wave * 32 + 8 * n + (lane >> 3);
             char *row = lds + buf * kABuf + R * 128 + (ac >> 2) * 8;
-            *reinterpret_cast<uint2 *>(row + (((ac & 3) ^ aswz(R)) << 4)) = make_uint2(RA[set][n].x, RA[set][n].y);
-            *reinterpret_cast<uint2 *>(row + (((4 + (ac & 3)) ^ aswz(R)) << 4)) = make_uint2(RA[set][n].z, RA[set][n].w);
+            *reinterpret_cast<uint2 *>(row + (((ac & 3) ^ akey(R)) << 4)) = make_uint2(RA[set][n].x, RA[set][n].y);
+            *reinterpret_cast<uint2 *>(row + (((4 + (ac & 3)) ^ akey(R)) << 4)) = make_uint2(RA[set][n].z, RA[set][n].w);
         }
     };
     auto store_b = [&](int set, int buf) {
 #pragma unroll
         for (int n = 0; n < NCT; ++n) {
             const int rr = brow0 + 2 * n;
-            *reinterpret_cast<uint4 *>(lds + kLdsB + buf * kBBuf + rr * 512 + ((bc ^ (rr & 7)) << 4)) = RB[set][n];
+            *reinterpret_cast<uint4 *>(lds + kLdsB + buf * kBBuf + rr * 512 + ((bc ^ bkey(rr)) << 4)) = RB[set][n];
         }
     };
     // 32 scale bytes per row and four steps, as [q][step][h]: a lane reads its eight in one
@@ -367,7 +372,7 @@ __device__ __forceinline__ void grouped_tile(const GemmArgs &a, char *lds, int n
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             wv[j] = *reinterpret_cast<const uint4 *>(lds + abuf * kABuf + arow[j] * 128 +
-                                                     (((4 * kg + q) ^ aswz(arow[j])) << 4));
+                                                     (((4 * kg + q) ^ akey(arow[j])) << 4));
     };
     auto compute = [&](int P, int h, int bbuf) {
         const char *B = lds + kLdsB + bbuf * kBBuf;
@@ -389,7 +394,7 @@ __device__ __forceinline__ void grouped_tile(const GemmArgs &a, char *lds, int n
 #pragma unroll
                 for (int ct = 0; ct < NCT; ++ct) {
                     const bf16x8 bv = *reinterpret_cast<const bf16x8 *>(B + (ct * 16 + r16) * 512 +
-                                                                        ((chunk ^ (r16 & 7)) << 4));
+                                                                        ((chunk ^ bkey(r16)) << 4));
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
                         acc[j][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[j], bv, acc[j][ct], 0, 0, 0);

@@ -83,13 +83,13 @@ __global__ __launch_bounds__(kThreads, 2) void mxfp4_gemm_kernel(GemvArgs a) {
             const int row = xr + n * XR;
             const uint4 v = RX[set][n];
             if constexpr (TERMS == 1) {
-                *reinterpret_cast<uint4 *>(X + row * (KC * 2) + ((xc ^ (row & 7)) << 4)) = v;
+                *reinterpret_cast<uint4 *>(X + row * (KC * 2) + ((xc ^ (row & 15)) << 4)) = v;
             } else {
                 const uint32_t f[4] = {v.x, v.y, v.z, v.w};
                 uint32_t t[3][4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) split3(__uint_as_float(f[i]), t[0][i], t[1][i], t[2][i]);
-                char *p = X + row * (KC * 2) + (((xc >> 1) ^ (row & 7)) << 4) + (xc & 1) * 8;
+                char *p = X + row * (KC * 2) + (((xc >> 1) ^ (row & 15)) << 4) + (xc & 1) * 8;
 #pragma unroll
                 for (int x = 0; x < 3; ++x)
                     *reinterpret_cast<uint2 *>(p + x * Sh::XT) = make_uint2(hi16x2(t[x][0], t[x][1]), hi16x2(t[x][2], t[x][3]));
@@ -129,7 +129,7 @@ __global__ __launch_bounds__(kThreads, 2) void mxfp4_gemm_kernel(GemvArgs a) {
             const bf16x8 wv = __builtin_bit_cast(bf16x8, wv4);
 #pragma unroll
             for (int t = 0; t < TT; ++t) {
-                const char *p = X + (16 * t + r16) * (KC * 2) + (((4 * g + q) ^ (r16 & 7)) << 4);
+                const char *p = X + (16 * t + r16) * (KC * 2) + (((4 * g + q) ^ r16) << 4);
                 f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int x = TERMS - 1; x >= 0; --x)
