@@ -28,6 +28,8 @@
 namespace k3 {
 namespace {
 
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
 constexpr int kThreads = 512, kBQ = 128, kBT = 32;
 constexpr int kNope = 128, kRope = 64, kV = 128, kQ = kNope + kRope;
 
@@ -110,40 +112,35 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
     // the first four waves
     const char *kp = reinterpret_cast<const char *>(a.kp + mla_k_index(head, a.tpad, 0, 0)) + (tid >> 4) * 768 + (tid & 15) * 16;
     const char *vt = reinterpret_cast<const char *>(a.vt + mla_v_index(head, a.tpad, 0, 0, 0)) + tid * 16;
-    const int rk = tid >> 3, rc = tid & 7;
-    uint4 RK[3], RV[3], RR[RT];
-    auto load = [&](int s) {
-        if (s >= nsteps) return;
+    const int rk = (tid >> 3) & 31, rc = tid & 7;
+    u32x4 RK[3], RV[3], RR[RT];
+    // (native vectors, straight-line and unconditional, past the last step that step again: as
+    // uint4 structs the staged values went through private memory and every step waited for
+    // its loads)
+    auto load = [&](int step) {
+        const int s = min(step, nsteps - 1);
 #pragma unroll
         for (int x = 0; x < 3; ++x) {
-            RK[x] = *reinterpret_cast<const uint4 *>(kp + static_cast<int64_t>(s) * (kBT * 768) + x * 256);
-            RV[x] = *reinterpret_cast<const uint4 *>(vt + static_cast<int64_t>(s) * (3 * kVt) + x * kVt);
+            RK[x] = *reinterpret_cast<const u32x4 *>(kp + static_cast<int64_t>(s) * (kBT * 768) + x * 256);
+            RV[x] = *reinterpret_cast<const u32x4 *>(vt + static_cast<int64_t>(s) * (3 * kVt) + x * kVt);
         }
-        if (wave < 4) {
-            if constexpr (RT == 1) {
-                const int t = s * kBT + rk;
-                RR[0] = make_uint4(0u, 0u, 0u, 0u);
-                if (t < a.Tk)
-                    RR[0] = *reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(a.rot) + t * a.ld_rot + rc * 8);
-            } else {
+        const int t = s * kBT + rk;    // rows past the cache (never seen): its last row
+        const uint16_t *row = RT == 1 ? static_cast<const uint16_t *>(a.rot) + min(t, a.Tk - 1) * a.ld_rot
+                                      : static_cast<const uint16_t *>(a.rot) + static_cast<int64_t>(t) * 3 * kRope;
 #pragma unroll
-                for (int x = 0; x < RT; ++x)
-                    RR[x] = *reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(a.rot) +
-                                                             (static_cast<int64_t>(s * kBT + rk) * 3 + x) * kRope + rc * 8);
-            }
-        }
+        for (int x = 0; x < RT; ++x) RR[x] = *reinterpret_cast<const u32x4 *>(row + x * kRope + rc * 8);
     };
     auto store = [&](int buf) {
         char *L = lds + buf * kStage;
 #pragma unroll
         for (int x = 0; x < 3; ++x) {
-            *reinterpret_cast<uint4 *>(L + x * kK + (tid >> 4) * 256 + (((tid & 15) ^ ((tid >> 4) & 15)) << 4)) = RK[x];
-            *reinterpret_cast<uint4 *>(L + kOffV + x * kVt + (tid >> 2) * 64 + (((tid & 3) ^ ((tid >> 3) & 3)) << 4)) = RV[x];
+            *reinterpret_cast<u32x4 *>(L + x * kK + (tid >> 4) * 256 + (((tid & 15) ^ ((tid >> 4) & 15)) << 4)) = RK[x];
+            *reinterpret_cast<u32x4 *>(L + kOffV + x * kVt + (tid >> 2) * 64 + (((tid & 3) ^ ((tid >> 3) & 3)) << 4)) = RV[x];
         }
         if (wave < 4) {
 #pragma unroll
             for (int x = 0; x < RT; ++x)
-                *reinterpret_cast<uint4 *>(L + kOffR + x * kR + rk * 128 + ((rc ^ (rk & 7)) << 4)) = RR[x];
+                *reinterpret_cast<u32x4 *>(L + kOffR + x * kR + rk * 128 + ((rc ^ (rk & 7)) << 4)) = RR[x];
         }
     };
 

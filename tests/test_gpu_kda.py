@@ -196,3 +196,49 @@ def test_kda_layer_prefill_path_matches_oracle_and_decode():
     o2, S2, _ = attn(xd[:, 12:], state=S, conv=conv)
     want2, _, _ = okda.kda_layer(cfg, w, x[:, 12:], S_want, conv_want)
     assert om.normwise_rel(o2.cpu().numpy(), want2) <= 2e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("Tn,H,HV,V,shift", [(2, 1, 1, 32, 0), (15, 2, 2, 96, 1), (16, 2, 4, 128, 0), (17, 1, 2, 64, 3),
+                                             (33, 3, 3, 32, 0)])
+def test_kda_sequence_edges(Tn, H, HV, V, shift, dtype):
+    """Sequences around the 16 tokens staged at a time, grouped value heads, part column
+    blocks, and q, k, g off 16-byte alignment, against the oracle."""
+    from k3hip import _lib
+    from k3hip import _torch as T
+    rng = np.random.default_rng(Tn * 7 + V)
+    q, k, v, g, beta, S0 = _inputs(rng, 1, Tn, H, HV, V=V)
+    host = [om.bf16_round(a) if dtype == torch.bfloat16 else a for a in (q, k, v, g, beta)]
+    dev = []
+    for a in host:
+        buf = torch.empty(a.size + shift, dtype=dtype, device=DEV)
+        buf[shift:] = torch.from_numpy(a.reshape(-1)).to(DEV).to(dtype)
+        dev.append(buf[shift:])
+    S, o = _dev(S0)[0], torch.empty(Tn, HV, V, device=DEV)
+    _lib.call("k3_kda_recurrent", *(T.ptr(t) for t in dev), T.dtype_code(dtype), T.ptr(S), T.ptr(o), _lib.K3_F32, Tn, H, HV,
+              128, V, 128 ** -0.5, T.stream(o))
+    want_o, want_S = okda.kda_recurrent(*host, None, S0)
+    assert om.normwise_rel(o.cpu().numpy(), want_o[0]) <= TOL
+    assert om.normwise_rel(S.cpu().numpy(), want_S) <= TOL
+
+
+@pytest.mark.parametrize("B,Tn,conv", [(1, 2, 4), (1, 8, 3), (2, 17, 4), (1, 35, 2), (3, 9, 5)])
+def test_kda_prefill_windows_and_batches(B, Tn, conv):
+    """The many-token path from kept states: convolutions of 2 to 5 (calls shorter than the
+    window too), tokens around its blocks of eight, batches, against the fp64 layer."""
+    from k3hip.kda import KDAAttention
+    cfg = KdaCfg(256, 4)
+    cfg.kda_conv_size = conv
+    rng = np.random.default_rng(Tn)
+    w = okda.random_kda_weights(rng, cfg, 0.05)
+    for n in ("q_proj", "k_proj", "v_proj", "g_proj", "o_proj", "f_a_proj", "f_b_proj", "b_proj"):
+        w[n + ".weight"] = om.bf16_round(w[n + ".weight"])
+    attn = KDAAttention(cfg, {n: torch.from_numpy(a).to(DEV) for n, a in w.items()})
+    x = om.bf16_round(rng.standard_normal((B, Tn, 256)).astype(np.float32))
+    S0 = (rng.standard_normal((B, 4, 128, 128)) * 0.1).astype(np.float32)
+    cv0 = tuple((rng.standard_normal((B, conv - 1, 512)) * 0.5).astype(np.float32) for _ in range(3))
+    out, S, cv = attn(torch.from_numpy(x).to(DEV).to(torch.bfloat16), torch.from_numpy(S0).to(DEV),
+                      tuple(torch.from_numpy(c).to(DEV) for c in cv0))
+    want, want_S, want_cv = okda.kda_layer(cfg, w, x, S0, cv0)
+    assert om.normwise_rel(out.cpu().numpy(), want) <= 2e-5 and om.normwise_rel(S.cpu().numpy(), want_S) <= 2e-5
+    assert max(om.normwise_rel(a.cpu().numpy(), b) for a, b in zip(cv, want_cv)) <= 2e-6

@@ -204,3 +204,48 @@ def test_routed_moe_grouped_forward_matches_decode_path():
     a = moe.grouped_forward(x).cpu().numpy()
     b = moe(x).cpu().numpy()
     assert om.normwise_rel(a, b) <= TOL
+
+
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,I,off", [(320, 192, 0), (256, 128, 1), (1088, 448, 3), (64, 64, 2)])
+def test_grouped_tile_edges(H, I, off, xdt):
+    """Experts of 1, 15, 16, 17, 33, 48, 49, 64, 65 and 130 rows (every column-group count, full
+    and part tiles), K of whole and part 256-steps, row blocks that end past the last weight
+    row, scale rows at every byte alignment, bf16 and fp32 x, against fp64 torch.  Products are
+    exact; x in fp32 and the activation keep 16 bits (2^-17 each), sums are fp32: 2e-5."""
+    from k3hip.moe import moe_grouped_ffn
+    g = torch.Generator(device=DEV)
+    g.manual_seed(H + I + off)
+    counts = [1, 15, 16, 17, 33, 48, 49, 64, 65, 130, 0]
+    E = len(counts)
+    ids = torch.cat([torch.full((c,), e, device=DEV) for e, c in enumerate(counts)])
+    ids = ids[torch.randperm(len(ids), device=DEV, generator=g)].view(-1, 2)      # top-2, an id twice at times
+    T = ids.shape[0]
+    lut = torch.tensor([0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0], dtype=torch.float64, device=DEV)
+    lut = torch.cat([lut, -lut])
+
+    def mx(n, k):
+        p = torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device=DEV, generator=g)
+        buf = torch.randint(118, 124, (n * (k // 32) + 4,), dtype=torch.uint8, device=DEV, generator=g)
+        return p, buf[off:off + n * (k // 32)].view(n, k // 32)
+
+    def dec(w):
+        codes = torch.stack([w[0] & 15, w[0] >> 4], dim=-1).flatten(1).int()
+        return lut[codes] * torch.exp2(w[1].double() - 127).repeat_interleave(32, dim=1)
+
+    ex = [(mx(I, H), mx(I, H), mx(H, I)) for _ in range(E)]
+    table = torch.tensor([[t.data_ptr() for pair in e for t in pair] for e in ex], dtype=torch.int64, device=DEV)
+    x = torch.randn(T, H, device=DEV, generator=g).to(xdt)
+    w = torch.rand(T, 2, device=DEV, generator=g)
+    got = moe_grouped_ffn(x, ids, w, table, I, "situ", 2.0, 3.0)
+    want = torch.zeros(T, H, dtype=torch.float64, device=DEV)
+    for j in range(2):
+        for e in range(E):
+            t = (ids[:, j] == e).nonzero().flatten()
+            a, u = x[t].double() @ dec(ex[e][0]).T, x[t].double() @ dec(ex[e][1]).T
+            act = 2 * torch.tanh(a / 2) * torch.sigmoid(a) * 3 * torch.tanh(u / 3)
+            want.index_add_(0, t, act @ dec(ex[e][2]).T * w[t, j, None].double())
+    rel = float((got.double() - want).norm() / want.norm())
+    print(f"H={H} I={I} scale offset {off} {xdt}: {rel:.2e}")
+    assert rel <= 2e-5
+    assert torch.equal(got, moe_grouped_ffn(x, ids, w, table, I, "situ", 2.0, 3.0))
