@@ -13,7 +13,7 @@ timed on a bounded sample on this host.  The same line carries, as sub-objects:
                      a fresh token per step;
   k3_latent_layer    K3's routed layer with its latent wrapper (896 experts, top-16);
   checkpoint_ingest  host-to-HBM ingest of K3-shaped experts from safetensors shards;
-  moe_prefill        2048 tokens x top-8 on the grouped MXFP4-MFMA path, Zipf(1.1) load;
+  moe_prefill        2048 tokens x top-8 on the grouped matrix-core path, Zipf(1.1) load;
   gemv               one [2048 x 7168] projection;
   mla_decode         the absorbed MLA core, 64 heads over 32768 cached tokens;
   mla_step           one token through a whole MLA layer at K3 shapes;
@@ -638,8 +638,8 @@ def bench_kda_step(torch, steps, warmup, dev):
 
     sec, _ = graph_time(torch, step, steps, warmup)
     stats = None if EAGER else step_stats(torch, step, 32)
-    # a 256-token prompt through KDAAttention's prefill path (eager: GEMMs on the BLAS
-    # library, one recurrence launch), timed with events
+    # a 256-token prompt through KDAAttention's prefill path (eager: projections on
+    # k3_dense, one recurrence launch), timed with events
     xp = torch.randn(1, 256, KS_HID, device=dev, generator=gen).to(torch.bfloat16)
     attn(xp)
     torch.cuda.synchronize()
@@ -895,7 +895,7 @@ def main():
             "ms": round(pst * 1e3, 3), "GB/s": round(pbytes / pst / 1e9, 1),
             "pct_hbm_peak": round(100 * pbytes / pst / 1e9 / HBM_PEAK_GBS, 1), "bytes": pbytes,
             "useful_TFLOP/s": round(PF_FLOPS / pst / 1e12, 1),
-            "mfma": "v_mfma_scale_f32_16x16x128_f8f6f4 (MXFP4 x E4M3 terms; issues at the FP8 rate)",
+            "mfma": "v_mfma_f32_16x16x32_bf16 (MXFP4 decoded to bf16 in registers; act as two bf16 terms)",
             "pct_fp8_mfma_peak": round(100 * PF_FLOPS / pst / 5.0e15, 1),
             "tokens": PF_T, "top_k": PF_K, "experts": E_LAYER, "routing": "zipf(1.1), seeded",
             "expert_load": {"max": int(counts.max()), "mean": round(float(counts.mean()), 1),
@@ -950,7 +950,7 @@ def main():
                             "bytes": KS_BYTES, "hidden": KS_HID, "heads": KDA_H, "head_dim": KDA_D, "conv": 4,
                             "weights": "bf16", "launches": 4, "step_us": kstats2,
                             "prefill_256_tokens": {"ms": round(kpre2 * 1e3, 3), "tokens_per_s": round(256 / kpre2, 1),
-                                                   "what": "KDAAttention.prefill: BLAS GEMMs + one k3_kda_recurrent"}}
+                                                   "what": "KDAAttention.prefill: k3_dense projections, fused inputs, one k3_kda_recurrent"}}
     if "ceiling" in work:
         ce = bench_read_ceiling(torch, EXPERT_BYTES, 256, dev)
         cl = bench_read_ceiling(torch, LAYER_BYTES, 64, dev)

@@ -137,7 +137,7 @@ __device__ __forceinline__ uint4 buf_load16(__amdgpu_buffer_rsrc_t r, uint32_t o
 // Inputs that several blocks stage (x, act, norm weights) keep the default policy: the hint
 // on every load made the expert step 20% slower.  The grouped prefill's weight tiles (read
 // once per token tile of an expert) and the MLA cache rows (read by the four head-group
-// blocks of a split) keep it too: with the hint, 4.65 -> 5.18 ms and no gain.
+// blocks of a split) keep it too: no gain with the hint.
 __device__ __forceinline__ uint4 buf_load16_nt(__amdgpu_buffer_rsrc_t r, uint32_t off) {
     return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 2));
 }

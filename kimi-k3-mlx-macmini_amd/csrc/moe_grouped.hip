@@ -215,7 +215,16 @@ struct GemmArgs {
 // rows and split the reduction (their sums meet in LDS at the end), so no wave converts or
 // reads what another one does.  Weights become bf16 in registers (4 v_cvt per 8 values of
 // a row, reused by the tile's column groups and both terms).
-// Measured (2048 tokens, 896 experts top-16, latent 3584 / 3072): @@GU@@
+// Measured (2048 tokens, 896 experts top-16, latent 3584 / 3072; the former form fed the scaled
+// FP4 x FP8 MFMA in operand order): gate/up 4470 -> 2840 us, down 2366 -> 1930 us; 700 tokens over
+// 384 experts: 1850 -> 1270 and 1208 -> 860 us.  What bounds it now: a step costs a barrier, the
+// LDS round trip and the products in turn, 1.2 us at one column group (its weights take 1.2 us
+// of HBM), 1.6 at three, 1.9 at four (matrix cores busy 28% in gate/up, 39% in down).  Measured
+// and not kept: the two wave groups half a beat apart (gate/up 3030 -> 3940 us: too little work
+// between barriers), sixteen waves of 32 rows (B is read twice as often from LDS: 2720 -> 3800
+// us), persistent blocks that read the next tile's record and first lines ahead (3030 -> 3740
+// us, static shares), non-temporal weight loads (no change), loads one step further ahead at
+// three column groups (no change).
 constexpr int kThreads = 512;
 constexpr uint32_t kOob = 0xf0000000u;      // past every buffer size the host lets through
 constexpr int kABuf = 256 * 128, kBBuf = 64 * 512, kSBuf = 256 * 32;

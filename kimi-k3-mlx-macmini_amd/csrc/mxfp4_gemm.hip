@@ -15,7 +15,10 @@
 // steps ahead, and go through LDS (x in 16-byte chunks XOR-swizzled by the row).  What bounds a
 // small call is latency and the x rows every block reads, so R is 16 while that gives less
 // than two blocks per CU, else 64.
-// @@MM@@
+// Measured: 37 tokens of a [3072 x 3584] projection 51.6 us (ten GEMV launches) -> 8.9 us.  It is
+// bound by its chain of steps (seven of 512 elements: barrier, LDS, products) and the 190 KB of
+// x every block reads; one step of 256 elements instead of 512: 11.5 against 11.2 us at 64 token
+// slots, 48 slots instead of 64 for 37 tokens: 11.2 -> 9.1 us.
 #include <algorithm>
 
 #include "k3_common.h"

@@ -263,8 +263,8 @@ class RoutedMoE:
     def shared_forward(self, x: torch.Tensor, add: torch.Tensor | None = None) -> torch.Tensor:
         """Shared expert on the original hidden state (moe.py:105-107), plus ``add`` [M, H] fp32
         if given.  Fused: exact
-        products with fp32 accumulation and fp32 intermediates on the BLAS library, no weight
-        copy (inside a decode step it runs in the layer kernels).  Unfused: the reference's
+        products with fp32 accumulation and fp32 intermediates (_blas.project, k3_dense), no weight copy
+        (inside a decode step it runs in the layer kernels).  Unfused: the reference's
         dtype promotion (a bf16 input against bf16 weights gives bf16 gate / up)."""
         act, beta, lb = self._act()
         mats = [self.sh_gate, self.sh_up]
@@ -299,7 +299,7 @@ class RoutedMoE:
                         out_dtype=torch.float32) -> torch.Tensor:
         """Prefill form of __call__ for x [..., H]: route every token on x as given (or take
         the given RouterResult), then run the routed experts grouped by expert on the device
-        (moe_grouped_ffn); the shared expert, if any, runs on the BLAS library."""
+        (moe_grouped_ffn); the shared expert, if any, is shared_forward."""
         return self._forward_routed(x, router, out_dtype, moe_grouped_ffn)
 
     def multi_forward(self, x: torch.Tensor, router: RouterResult | None = None,
@@ -307,7 +307,7 @@ class RoutedMoE:
         """Decode form of __call__ for a few tokens x [..., H] (at most DECODE_TOKENS): route
         every token, then every expert any token selects runs once against all the tokens
         routed to it (moe_routed_decode: the union of the routed experts built on the device,
-        fp32 accumulation); the shared expert, if any, runs on the BLAS library."""
+        fp32 accumulation); the shared expert, if any, is shared_forward."""
         return self._forward_routed(x, router, out_dtype, moe_routed_decode)
 
     def _forward_routed(self, x, router, out_dtype, routed_fn, validate=None):
@@ -337,7 +337,7 @@ class RoutedMoE:
             y = y.to(out_dtype).reshape(*orig[:-1], self._H)
             return (y, r) if return_router else y
         if flat.shape[0] > self.DECODE_TOKENS:
-            # many tokens: grouped GEMMs on MXFP4 MFMA, every routed expert read once per tile
+            # many tokens: grouped GEMMs on the matrix cores, every routed expert read once per tile
             r = self.route(flat)
             y = self._forward_routed(flat, r, out_dtype, moe_grouped_ffn, validate=False)
             y = y.reshape(*orig[:-1], self._H)
@@ -582,12 +582,12 @@ class LatentMoE:
         """Many tokens: route every token on x as given; h = x W_down^T on the BLAS library
         (bf16 for a bf16 x, fp32 for an fp32 x); the routed experts grouped by expert on the
         device (k3_moe_grouped_ffn); the norm in fp32; the up projection and the shared
-        experts on the BLAS library with exact products and fp32 accumulation."""
+        experts on k3_dense with exact products and fp32 accumulation."""
         return self._forward_routed(flat, return_router, out_dtype, orig, moe_grouped_ffn)
 
     def multi_forward(self, flat, return_router=False, out_dtype=torch.float32, orig=None):
-        """A few decode tokens (at most DECODE_TOKENS) with the dense projections on the BLAS
-        library: as grouped_forward, with the routed experts run by moe_routed_decode, so
+        """A few decode tokens (at most DECODE_TOKENS) with the dense projections as separate
+        products: as grouped_forward, with the routed experts run by moe_routed_decode, so
         every expert any token selects is read once against all the tokens routed to it.
         ``__call__`` runs the same step with every projection in HIP (_decode_multi)."""
         return self._forward_routed(flat, return_router, out_dtype, orig, moe_routed_decode)
