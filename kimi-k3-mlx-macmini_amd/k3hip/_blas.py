@@ -23,7 +23,7 @@ import ctypes
 
 import torch
 
-from . import _lib, _workspace
+from . import _lib
 from . import _torch as T
 
 
@@ -64,7 +64,9 @@ def dense(a: torch.Tensor, ws, add: torch.Tensor | None = None) -> list[torch.Te
     N = (ctypes.c_int64 * n)(*(w.shape[0] for w in ws))
     code = T.dtype_code(a.dtype)
     nbytes = int(_lib.lib().k3_dense_workspace_size(M, K, N, n, code))
-    buf = _workspace.get(a.device, nbytes, "dense") if nbytes else None
+    # the partial sums are the call's own: calls of several threads on one stream, and a captured
+    # graph whose call is followed by a larger one, must not meet in a kept buffer
+    buf = torch.empty(nbytes, dtype=torch.uint8, device=a.device) if nbytes else None
     _lib.call("k3_dense", T.ptr(a), code, a.stride(0) if M > 1 else K, (ctypes.c_void_p * n)(*(w.data_ptr() for w in ws)),
               (ctypes.c_void_p * n)(*(o.data_ptr() for o in outs)), N, n, T.ptr(add), M, K, T.ptr(buf), nbytes,
               T.stream(a))

@@ -323,7 +323,7 @@ class MLAAttention:
         gate = None if gate is None else T.contiguous_aligned(gate)
         out = torch.empty((1, Tn, nh * vhd), dtype=torch.float32, device=q.device)
         nbytes = int(_lib.lib().k3_mla_prefill_workspace_size(lat.shape[0], nh))
-        ws = _workspace.get(q.device, nbytes, "mla_prefill")
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)   # the call's own, as the scores of _dense
         _lib.call("k3_mla_prefill", T.ptr(q), nh * c.q_head_dim, T.ptr(self.kv_b), T.ptr(lat), lat.stride(0), T.ptr(rot),
                   rot.stride(0), T.dtype_code(lat.dtype), T.ptr(gate), T.ptr(out), Tn, lat.shape[0], nh, c.kv_lora_rank,
                   c.qk_rope_head_dim, c.qk_nope_head_dim, vhd, float(scale), T.ptr(ws), ws.numel(), T.stream(q))

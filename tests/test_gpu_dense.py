@@ -78,3 +78,33 @@ def test_rmsnorm_and_act_rows():
                       (_lib.K3_ACT_SITU, 2 * torch.tanh(gd / 2) * torch.sigmoid(gd) * 3 * torch.tanh(ud / 3))):
         _lib.call("k3_act_rows", T.ptr(gt), T.ptr(u), T.ptr(o), gt.numel(), kind, 2.0, 3.0, T.stream(gt))
         assert float((o.double() - ref).abs().max()) <= 2e-6 * float(ref.abs().max())
+
+
+def test_dense_replay_after_larger_calls():
+    """A captured call (K split over blocks, so with partial sums) keeps its own scratch: later
+    larger calls and whatever takes freed memory leave its replays as the eager result."""
+    g = _g(11)
+    a = torch.randn(40, 4096, device=DEV, generator=g)
+    w = torch.randn(512, 4096, device=DEV, generator=g).to(torch.bfloat16)
+    big = torch.randn(200, 4096, device=DEV, generator=g)
+    wide = torch.randn(2048, 4096, device=DEV, generator=g).to(torch.bfloat16)
+    want = _blas.dense(a, [w])[0].clone()
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        _blas.dense(a, [w])
+    torch.cuda.current_stream().wait_stream(stream)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        out = _blas.dense(a, [w])[0]
+    for i in range(3):
+        with torch.cuda.stream(stream):
+            _blas.dense(big[:100 + 50 * i], [wide])
+            junk = [torch.full((n,), float("nan"), device=DEV) for n in (1 << 18, 1 << 20, 1 << 22)]
+        torch.cuda.synchronize()
+        del junk
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        assert torch.equal(_blas.dense(a, [w])[0], want)
