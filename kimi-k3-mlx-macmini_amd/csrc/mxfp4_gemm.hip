@@ -212,8 +212,22 @@ int launch_tt(const GemvArgs &a, hipStream_t st) {
 
 }  // namespace
 
-bool mxfp4_gemm_takes(int64_t M, int64_t N, int64_t K) {
-    return M > 4 && M <= 64 * 65535 && N < (1ll << 31) && 16 * (K / 32) + 32 <= kMaxScale && K * 64 * 4 < (1ll << 31);
+// A few tokens of few weights finish sooner in GEMV launches of four tokens: the matmul stages
+// whole 16-token tiles and walks K in one chain of steps, whatever M and N.  Both sides as fits
+// in us of launches measured over M 5..32, N 300..8192, K 1024..7168 (GEMV / matmul): fp32 x,
+// K = 7168: 5 tokens of 300 rows 9.0 / 17.5, 8 of 1024 rows 13.1 / 17.7, 12 of 1024 rows 19.3 /
+// 17.4, 8 of 2048 rows 23.1 / 17.4; K = 1024: 5 of 300 rows 5.3 / 5.0.  bf16 x, K = 7168: 5 tokens
+// of 300 rows 6.9 / 8.1, 8 of 300 rows 8.9 / 8.1.
+static bool gemv_sooner(int64_t M, int64_t N, int64_t K, bool x_bf16) {
+    if (M > 20 || K < 2048 || K > 8192 || (x_bf16 && N > 4096)) return false;
+    const double k = static_cast<double>(K), w = static_cast<double>(N) * k, waves = static_cast<double>(cdiv(N, 16 * 256));
+    const double per = x_bf16 ? 0.8e-4 + w / 400e9 : 0.95e-4 + w / 95e9;   // of a GEMV, per token and element
+    const double step = (x_bf16 ? k / 1500 : k / 500) * static_cast<double>(cdiv(M, 16));
+    return 2.0 * static_cast<double>(cdiv(M, 4)) + static_cast<double>(M) * k * per < (3.2 + step) * waves;
+}
+
+bool mxfp4_gemm_takes(int64_t M, int64_t N, int64_t K, bool x_bf16) {
+    return M > 4 && !gemv_sooner(M, N, K, x_bf16) && M <= 64 * 65535 && N < (1ll << 31) && 16 * (K / 32) + 32 <= kMaxScale && K * 64 * 4 < (1ll << 31);
 }
 
 int mxfp4_gemm_launch(const GemvArgs &a, hipStream_t st) {

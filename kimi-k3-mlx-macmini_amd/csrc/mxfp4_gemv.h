@@ -25,7 +25,7 @@ void gemv_default_cfg(int64_t N, int64_t K, int *rpw, int *gpl);
 int gemv_token_tile(int64_t K, int x_bf16);  // tokens per launch (0: K too long)
 int gemv_launch(const GemvArgs &a, int rpw, int gpl, hipStream_t st);
 // the matrix-core form for more tokens than one GEMV launch takes (mxfp4_gemm.hip)
-bool mxfp4_gemm_takes(int64_t M, int64_t N, int64_t K);
+bool mxfp4_gemm_takes(int64_t M, int64_t N, int64_t K, bool x_bf16);
 int mxfp4_gemm_launch(const GemvArgs &a, hipStream_t st);
 int gemv_validate(const void *x, int x_dtype, const void *packed, const void *scales,
                   const void *out, int out_dtype, int64_t M, int64_t N, int64_t K);

@@ -271,7 +271,7 @@ static int matvec_impl(const void *x, int x_dtype, const void *packed, const voi
         return set_error(K3_ERR_SHAPE, "mxfp4 matvec: K=%lld exceeds the %d-element activation tile", (long long)K,
                          x_dtype == K3_BF16 ? 32768 : 16384);
     auto st = static_cast<hipStream_t>(stream);
-    if (mxfp4_gemm_takes(M, N, K)) {
+    if (mxfp4_gemm_takes(M, N, K, x_dtype == K3_BF16)) {
         GemvArgs a{};
         a.x = x, a.ldx = K, a.packed = packed, a.scales = scales, a.out = out, a.ldo = N;
         a.M = static_cast<int>(M), a.N = N, a.K = K;

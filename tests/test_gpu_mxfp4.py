@@ -234,3 +234,23 @@ def test_matmul_many_tokens(m, n, k, xdt):
         assert torch.equal(y, mxfp4_matvec_fused(xs, packed, scales))
     b = mxfp4_matvec_fused(xs, packed, scales, out_dtype=torch.bfloat16)
     assert torch.equal(b, y.to(torch.bfloat16))
+
+
+# around the line between GEMV launches of four tokens and the matmul (few weights, fp32 x)
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("m,n,k", [(5, 300, 7168), (8, 1024, 7168), (8, 2048, 7168), (17, 300, 7168), (6, 4096, 2048)])
+def test_few_tokens_of_few_weights(m, n, k, xdt):
+    """Both forms: exact products and fp32 sums, far below k 2^-24 of the sum of |products|."""
+    from k3hip.mxfp4_matvec import mxfp4_matvec_fused
+    g = torch.Generator(device=DEV)
+    g.manual_seed(m + n + k)
+    x = torch.randn(m, k, device=DEV, generator=g).to(xdt)
+    packed = torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device=DEV, generator=g)
+    scales = torch.randint(118, 131, (n, k // 32), dtype=torch.uint8, device=DEV, generator=g)
+    lut = torch.tensor([0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0], dtype=torch.float64, device=DEV)
+    codes = torch.stack([packed & 15, packed >> 4], dim=-1).flatten(1).int()
+    w = torch.cat([lut, -lut])[codes] * torch.exp2(scales.double() - 127).repeat_interleave(32, dim=1)
+    y = mxfp4_matvec_fused(x, packed, scales)
+    want, mag = x.double() @ w.T, x.double().abs() @ w.abs().T
+    assert float(((y.double() - want).abs() / mag).max()) <= 1e-6
+    assert torch.equal(y, mxfp4_matvec_fused(x, packed, scales))
