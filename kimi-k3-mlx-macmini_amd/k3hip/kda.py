@@ -99,6 +99,17 @@ class KDAAttention:
                   _lib.K3_F32, x1.shape[-1], self.H, self.D, self.K, float(c.kda_gate_lower_bound),
                   float(c.rms_norm_eps), T.ptr(ws), ws.numel(), T.stream(x1))
 
+    def _check_widths(self) -> None:
+        """The launches of prefill read these weights at the layer's widths, whatever their shapes."""
+        P = self.H * self.D
+        for name, w, rows in (("q_proj", self.q_w, P), ("k_proj", self.k_w, P), ("v_proj", self.v_w, P),
+                              ("g_proj", self.g_w, P), ("f_b_proj", self.fb, P), ("b_proj", self.b_w, self.H)):
+            if w.dim() != 2 or w.shape[0] != rows:
+                raise ValueError(f"{name} must have {rows} rows; got {tuple(w.shape)}")
+        if self.dt_bias.numel() != P or self.o_norm_w.numel() != self.D or self.A_log.numel() < self.H:
+            raise ValueError(f"dt_bias [{P}], o_norm [{self.D}] and A_log for {self.H} heads expected; got "
+                             f"{self.dt_bias.numel()}, {self.o_norm_w.numel()} and {self.A_log.numel()} values")
+
     def prefill(self, x: torch.Tensor, state: torch.Tensor | None = None, conv: tuple | None = None):
         """Many tokens (attention_kda.py:94-115): the projections of all tokens (each weight
         read once), the convolutions, norms and gates in one launch, the recurrence over every
@@ -107,6 +118,7 @@ class KDAAttention:
         B, Tn, hid = x.shape
         H, D, K = self.H, self.D, self.K
         P = H * D
+        self._check_widths()
         dev = x.device
         xf = x.reshape(B * Tn, hid)
         if xf.dtype not in (torch.float32, torch.bfloat16):

@@ -1,0 +1,37 @@
+"""What the Python layer settles before anything is launched: shapes that the kernels take on
+trust, and which path a call goes to.  No GPU: a call that should be refused is refused by the
+shape check and not by the check for device tensors, which comes after it."""
+from __future__ import annotations
+
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+BF16 = torch.bfloat16
+
+
+def _kda(H=2, hid=64, K=4, **other):
+    from k3hip.kda import KDAAttention
+    P, D = H * 128, 128
+    z = lambda *s: torch.zeros(*s, dtype=BF16)  # noqa: E731
+    w = {"q_proj.weight": z(P, hid), "k_proj.weight": z(P, hid), "v_proj.weight": z(P, hid), "g_proj.weight": z(P, hid),
+         "o_proj.weight": z(hid, P), "q_conv1d.weight": z(P, 1, K), "k_conv1d.weight": z(P, 1, K),
+         "v_conv1d.weight": z(P, 1, K), "f_a_proj.weight": z(D, hid), "f_b_proj.weight": z(P, D), "b_proj.weight": z(H, hid),
+         "o_norm.weight": z(D), "A_log": torch.zeros(D), "dt_bias": torch.zeros(P)}
+    w.update(other)
+    cfg = SimpleNamespace(kda_num_heads=H, kda_head_dim=D, kda_conv_size=K, kda_gate_lower_bound=-5.0, rms_norm_eps=1e-5)
+    return KDAAttention(cfg, w)
+
+
+@pytest.mark.parametrize("name,shape", [("q_proj.weight", (128, 64)), ("v_proj.weight", (512, 64)), ("g_proj.weight", (255, 64)),
+                                        ("f_b_proj.weight", (128, 128)), ("b_proj.weight", (1, 64)), ("dt_bias", (255,)),
+                                        ("o_norm.weight", (64,))])
+def test_kda_many_tokens_refuse_weights_of_other_widths(name, shape):
+    with pytest.raises(ValueError, match=name.split(".")[0]):
+        _kda(**{name: torch.zeros(*shape)}).prefill(torch.zeros(1, 3, 64))
+
+
+def test_kda_many_tokens_refuse_more_heads_than_A_log_holds():
+    with pytest.raises(ValueError, match="A_log"):
+        _kda(H=129).prefill(torch.zeros(1, 2, 64))
