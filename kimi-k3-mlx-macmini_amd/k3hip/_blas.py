@@ -54,9 +54,12 @@ def dense_ok(a: torch.Tensor, *ws: torch.Tensor) -> bool:
 
 
 def dense(a: torch.Tensor, ws, add: torch.Tensor | None = None) -> list[torch.Tensor]:
-    """[a [M, K] @ w[N, K]^T in fp32 for w in ws] (k3_dense; operands checked by dense_ok), plus
-    ``add`` [M, N] fp32 where one weight is given."""
+    """[a [M, K] @ w[N, K]^T in fp32 for w in ws] (k3_dense; dtypes and alignment checked by dense_ok),
+    plus ``add`` [M, N] fp32 where one weight is given."""
     M, K = a.shape
+    if any(w.shape[1] != K for w in ws):
+        raise ValueError(f"a is [{M}, {K}]; weights {[tuple(w.shape) for w in ws]}")
+    T.require_device(a, *ws)
     if a.stride(1) != 1 or (a.stride(0) * a.element_size()) % 16 or a.stride(0) < K or a.data_ptr() % 16:
         a = T.contiguous_aligned(a)
     n = len(ws)

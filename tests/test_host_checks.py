@@ -35,3 +35,36 @@ def test_kda_many_tokens_refuse_weights_of_other_widths(name, shape):
 def test_kda_many_tokens_refuse_more_heads_than_A_log_holds():
     with pytest.raises(ValueError, match="A_log"):
         _kda(H=129).prefill(torch.zeros(1, 2, 64))
+
+
+def _layer(Is=64, hid=32, up=None, down=None):
+    from k3hip.moe import MoEConfig, RoutedMoE
+    z = lambda *s: torch.zeros(*s, dtype=BF16)  # noqa: E731
+    w = {"gate.weight": z(4, hid), "shared_experts.gate_proj.weight": z(Is, hid),
+         "shared_experts.up_proj.weight": z(*(up or (Is, hid))), "shared_experts.down_proj.weight": z(*(down or (hid, Is)))}
+    return RoutedMoE(MoEConfig(hid, 32, 4, 2), 0, w, lambda *a: None)
+
+
+def _no_device(monkeypatch, launches):
+    """The layers' own checks without a GPU: device checks pass, launches are recorded and the
+    matrix products are torch's."""
+    from k3hip import _blas, _lib
+    from k3hip import _torch as T
+    monkeypatch.setattr(T, "require_device", lambda *ts: None)
+    monkeypatch.setattr(T, "stream", lambda t: 0)
+    monkeypatch.setattr(_blas, "weights_ok", lambda *ws: True)
+    monkeypatch.setattr(_blas, "dense_ok", lambda a, *ws: True)
+    monkeypatch.setattr(_blas, "_mm_bf16_f32", lambda a, w: a.float() @ w.float().t())
+    monkeypatch.setattr(_lib, "call", lambda name, *a: launches.append(name))
+
+
+@pytest.mark.parametrize("kw", [dict(up=(48, 32)), dict(down=(32, 48)), dict(down=(32, 72))])
+def test_shared_expert_refuses_matrices_that_do_not_match(monkeypatch, kw):
+    """gate and up of different rows, and a down projection of another width."""
+    launches = []
+    _no_device(monkeypatch, launches)
+    with pytest.raises((ValueError, RuntimeError)):
+        _layer(**kw).shared_forward(torch.zeros(3, 32, dtype=BF16))
+    if "up" in kw:
+        assert "k3_act_rows" not in launches
+    assert launches.count("k3_dense") <= 1
