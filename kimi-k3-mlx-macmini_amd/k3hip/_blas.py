@@ -59,7 +59,11 @@ def dense(a: torch.Tensor, ws, add: torch.Tensor | None = None) -> list[torch.Te
     M, K = a.shape
     if any(w.shape[1] != K for w in ws):
         raise ValueError(f"a is [{M}, {K}]; weights {[tuple(w.shape) for w in ws]}")
-    T.require_device(a, *ws)
+    if add is not None:
+        if len(ws) != 1 or tuple(add.shape) != (M, ws[0].shape[0]) or add.dtype != torch.float32:
+            raise ValueError(f"add must be float32 [{M}, N] beside one weight [N, {K}]; got {add.dtype} {tuple(add.shape)}")
+        add = T.contiguous_aligned(add)
+    T.require_device(a, add, *ws)
     if a.stride(1) != 1 or (a.stride(0) * a.element_size()) % 16 or a.stride(0) < K or a.data_ptr() % 16:
         a = T.contiguous_aligned(a)
     n = len(ws)

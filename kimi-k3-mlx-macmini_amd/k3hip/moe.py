@@ -260,12 +260,15 @@ class RoutedMoE:
         u = self._proj(h, e, "w3")
         return self._proj(_act_torch(g.float(), u.float(), act, beta, lb), e, "w2")
 
-    def shared_forward(self, x: torch.Tensor, add: torch.Tensor | None = None) -> torch.Tensor:
-        """Shared expert on the original hidden state (moe.py:105-107), plus ``add`` [M, H] fp32
-        if given.  Fused: exact
+    def shared_forward(self, x: torch.Tensor) -> torch.Tensor:
+        """Shared expert on the original hidden state (moe.py:105-107).  Fused: exact
         products with fp32 accumulation and fp32 intermediates (_blas.project, k3_dense), no weight copy
         (inside a decode step it runs in the layer kernels).  Unfused: the reference's
         dtype promotion (a bf16 input against bf16 weights gives bf16 gate / up)."""
+        return self._shared(x, None)
+
+    def _shared(self, x: torch.Tensor, add: torch.Tensor | None) -> torch.Tensor:
+        """shared_forward(x), plus ``add`` (fp32, one row per token of x) where given."""
         act, beta, lb = self._act()
         mats = [self.sh_gate, self.sh_up]
         flat = x.reshape(-1, x.shape[-1])
@@ -325,7 +328,7 @@ class RoutedMoE:
         y = routed_fn(flat, router.expert_indices, router.expert_weights, self.expert_table(), self._I,
                       act, beta, lb, out_dtype=torch.float32, validate=validate)
         if self.sh_gate is not None:
-            y = self.shared_forward(flat, y)
+            y = self._shared(flat, y)
         return y.to(out_dtype).reshape(*orig[:-1], self._H)
 
     def __call__(self, x: torch.Tensor, return_router: bool = False, out_dtype=torch.float32):
@@ -489,9 +492,9 @@ class LatentMoE:
         """One routed expert on latent rows h [N, L] (moe.py:90-103)."""
         return self._routed.expert_forward(h, e)
 
-    def shared_forward(self, x: torch.Tensor, add: torch.Tensor | None = None) -> torch.Tensor:
-        """Shared expert(s) on the original hidden state (moe.py:105-107), plus ``add`` if given."""
-        return self._routed.shared_forward(x, add)
+    def shared_forward(self, x: torch.Tensor) -> torch.Tensor:
+        """Shared expert(s) on the original hidden state (moe.py:105-107)."""
+        return self._routed.shared_forward(x)
 
     def __call__(self, x: torch.Tensor, return_router: bool = False, out_dtype=torch.float32):
         orig = x.shape
@@ -608,7 +611,7 @@ class LatentMoE:
         y = _rmsnorm_rows(y, self._norm32, float(c.rms_norm_eps))
         y = _blas.mm_f32(y, self.up)                                      # latent -> hidden
         if self._routed.sh_gate is not None:
-            y = self.shared_forward(flat, y)
+            y = self._routed._shared(flat, y)
         y = y.to(out_dtype).reshape(*orig[:-1], orig[-1])
         return (y, r) if return_router else y
 

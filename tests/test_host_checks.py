@@ -68,3 +68,28 @@ def test_shared_expert_refuses_matrices_that_do_not_match(monkeypatch, kw):
     if "up" in kw:
         assert "k3_act_rows" not in launches
     assert launches.count("k3_dense") <= 1
+
+
+@pytest.mark.parametrize("add", [torch.zeros(3, 15), torch.zeros(2, 16), torch.zeros(3, 16, dtype=BF16), torch.zeros(16)])
+def test_dense_refuses_an_added_matrix_of_another_form(add):
+    from k3hip import _blas
+    with pytest.raises(ValueError, match="add"):
+        _blas.dense(torch.zeros(3, 32), [torch.zeros(16, 32, dtype=BF16)], add)
+
+
+def test_dense_reads_an_added_view_at_its_own_strides(monkeypatch):
+    from k3hip import _blas, _lib
+    _no_device(monkeypatch, [])
+    seen = {}
+    monkeypatch.setattr(_lib, "lib", lambda: SimpleNamespace(k3_dense_workspace_size=lambda *a: 0))
+    monkeypatch.setattr(_lib, "call", lambda name, *a: seen.update(add=a[7]))
+    add = torch.arange(3 * 40, dtype=torch.float32).view(3, 40)[:, 1:17]
+    _blas.dense(torch.zeros(3, 32), [torch.zeros(16, 32, dtype=BF16)], add)
+    assert seen["add"] != add.data_ptr() and seen["add"] % 16 == 0
+
+
+def test_shared_forward_takes_the_hidden_state_alone():
+    import inspect
+    from k3hip.moe import LatentMoE, RoutedMoE
+    for cls in (RoutedMoE, LatentMoE):
+        assert list(inspect.signature(cls.shared_forward).parameters) == ["self", "x"]
