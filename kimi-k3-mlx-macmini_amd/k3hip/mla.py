@@ -196,9 +196,10 @@ def _rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
 def _rmsnorm_rows(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
     """_rmsnorm of the rows of an fp32 [M, K] device tensor in one launch."""
     M, K = x.shape
+    if tuple(w.shape) != (K,) or K % 4 or x.stride(1) != 1 or x.stride(0) % 4 or x.data_ptr() % 16 or M == 0:
+        return _rmsnorm(x, w, eps)   # (which refuses or broadcasts a w of another shape)
     w = T.contiguous_aligned(w.to(torch.float32))
-    if K % 4 or x.stride(1) != 1 or x.stride(0) % 4 or x.data_ptr() % 16 or M == 0:
-        return _rmsnorm(x, w, eps)
+    T.require_device(x, w)
     out = torch.empty((M, K), dtype=torch.float32, device=x.device)
     _lib.call("k3_rmsnorm_rows", T.ptr(x), x.stride(0) if M > 1 else K, T.ptr(w), float(eps), T.ptr(out), M, K, T.stream(x))
     return out

@@ -93,3 +93,18 @@ def test_shared_forward_takes_the_hidden_state_alone():
     from k3hip.moe import LatentMoE, RoutedMoE
     for cls in (RoutedMoE, LatentMoE):
         assert list(inspect.signature(cls.shared_forward).parameters) == ["self", "x"]
+
+
+@pytest.mark.parametrize("mod", ["mla", "moe"])
+def test_norm_of_rows_refuses_a_weight_of_another_length(monkeypatch, mod):
+    import importlib
+    m = importlib.import_module(f"k3hip.{mod}")
+    launches = []
+    _no_device(monkeypatch, launches)
+    x = torch.randn(3, 32)
+    with pytest.raises(RuntimeError):
+        m._rmsnorm_rows(x, torch.ones(16), 1e-5)
+    assert torch.equal(m._rmsnorm_rows(x, torch.full((1,), 2.0), 1e-5), m._rmsnorm_rows(x, torch.ones(1), 1e-5) * 2)
+    assert not launches
+    m._rmsnorm_rows(x, torch.ones(32), 1e-5)
+    assert launches == ["k3_rmsnorm_rows"]
