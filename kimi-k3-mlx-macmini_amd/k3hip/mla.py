@@ -305,7 +305,8 @@ class MLAAttention:
         B, Tn = q.shape[:2]
         if torch.is_grad_enabled() and (q.requires_grad or lat.requires_grad or self.kv_b.requires_grad):
             return False
-        return (B == 1 and Tn > 1 and q.is_cuda and q.dtype == torch.float32 and lat.dtype == rot.dtype
+        return (B == 1 and Tn > 1 and lat.shape[:2] == rot.shape[:2] and lat.shape[0] == 1
+                and q.is_cuda and q.dtype == torch.float32 and lat.dtype == rot.dtype
                 and lat.dtype in (torch.bfloat16, torch.float32) and self.kv_b.dtype == torch.bfloat16
                 and self.kv_b.is_contiguous() and self.kv_b.data_ptr() % 16 == 0
                 and (c.kv_lora_rank, c.qk_rope_head_dim, c.qk_nope_head_dim, c.v_head_dim) == (KV_LORA_RANK, ROPE_DIM, 128, 128)

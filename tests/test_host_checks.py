@@ -108,3 +108,39 @@ def test_norm_of_rows_refuses_a_weight_of_another_length(monkeypatch, mod):
     assert not launches
     m._rmsnorm_rows(x, torch.ones(32), 1e-5)
     assert launches == ["k3_rmsnorm_rows"]
+
+
+def _mla_stub(heads=4):
+    """MLAAttention's route, with tensors that claim to be on the device."""
+    from k3hip.mla import MLAAttention
+    attn = MLAAttention.__new__(MLAAttention)
+    attn.cfg = SimpleNamespace(num_attention_heads=heads, kv_lora_rank=512, qk_rope_head_dim=64, qk_nope_head_dim=128,
+                               v_head_dim=128, q_head_dim=192)
+    attn.kv_b = _dev(torch.zeros(1, 1, dtype=BF16))
+    return attn
+
+
+class _Dev:
+    """A CPU tensor that says it is a device tensor."""
+    def __init__(self, t, requires_grad=False):
+        self._t, self.is_cuda, self.requires_grad = t, True, requires_grad
+
+    def __getattr__(self, name):
+        return getattr(self._t, name)
+
+
+def _dev(t, **kw):
+    return _Dev(t, **kw)
+
+
+def _rows(B, Tk, width, **kw):
+    return _dev(torch.zeros(1, dtype=BF16).expand(B, Tk, width), **kw)
+
+
+def test_mla_prompt_takes_one_sequence_of_one_length():
+    attn = _mla_stub()
+    q = _dev(torch.zeros(1).expand(1, 20, 4, 192))
+    assert attn._expanded_ok(q, _rows(1, 20, 512), _rows(1, 20, 64))
+    assert not attn._expanded_ok(q, _rows(2, 20, 512), _rows(2, 20, 64))   # a cache of two sequences
+    assert not attn._expanded_ok(q, _rows(1, 20, 512), _rows(1, 19, 64))
+    assert not attn._expanded_ok(_dev(torch.zeros(1).expand(2, 20, 4, 192)), _rows(1, 20, 512), _rows(1, 20, 64))
