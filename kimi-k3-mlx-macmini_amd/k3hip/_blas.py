@@ -42,14 +42,13 @@ def _mm_bf16_f32(a2: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 def weights_ok(*ws: torch.Tensor) -> bool:
     """k3_dense takes these weights as they are: bf16 device matrices of whole 16-byte rows."""
-    return all(w.is_cuda and w.dim() == 2 and w.dtype == torch.bfloat16 and w.is_contiguous()
-               and w.data_ptr() % 16 == 0 and w.shape[1] % 8 == 0 and w.shape[0] > 0
-               and not (w.requires_grad and torch.is_grad_enabled()) for w in ws)
+    return not T.tracked(*ws) and all(w.is_cuda and w.dim() == 2 and w.dtype == torch.bfloat16 and w.is_contiguous()
+                                      and w.data_ptr() % 16 == 0 and w.shape[1] % 8 == 0 and w.shape[0] > 0 for w in ws)
 
 
 def dense_ok(a: torch.Tensor, *ws: torch.Tensor) -> bool:
     """k3_dense takes a against these weights as they are, and no gradient is asked for."""
-    return (a.is_cuda and a.dtype in (torch.float32, torch.bfloat16) and not (a.requires_grad and torch.is_grad_enabled())
+    return (a.is_cuda and a.dtype in (torch.float32, torch.bfloat16) and not T.tracked(a)
             and weights_ok(*ws) and all(w.shape[1] == a.shape[-1] and w.device == a.device for w in ws))
 
 

@@ -2,6 +2,7 @@
 from __future__ import annotations
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 
@@ -47,6 +48,14 @@ def require_device(*ts: torch.Tensor) -> None:
             dev, first = d, t
         elif d != dev:
             raise ValueError(f"tensors on different devices: {first.device} vs {t.device}")
+
+
+def tracked(*ts: torch.Tensor | None) -> bool:
+    """A gradient, or a forward-mode tangent, of one of these is asked for: the launches carry
+    neither, so such a call stays on the tensor operations that do."""
+    grad = torch.is_grad_enabled()
+    return any(t is not None and ((grad and t.requires_grad) or forward_ad.unpack_dual(t).tangent is not None)
+               for t in ts)
 
 
 def contiguous_aligned(t: torch.Tensor) -> torch.Tensor:

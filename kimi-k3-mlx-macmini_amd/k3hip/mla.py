@@ -196,7 +196,8 @@ def _rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
 def _rmsnorm_rows(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
     """_rmsnorm of the rows of an fp32 [M, K] device tensor in one launch."""
     M, K = x.shape
-    if tuple(w.shape) != (K,) or K % 4 or x.stride(1) != 1 or x.stride(0) % 4 or x.data_ptr() % 16 or M == 0:
+    if (tuple(w.shape) != (K,) or K % 4 or x.stride(1) != 1 or x.stride(0) % 4 or x.data_ptr() % 16 or M == 0
+            or T.tracked(x, w)):
         return _rmsnorm(x, w, eps)   # (which refuses or broadcasts a w of another shape)
     w = T.contiguous_aligned(w.to(torch.float32))
     T.require_device(x, w)
@@ -261,7 +262,10 @@ class MLAAttention:
         gated = bool(getattr(c, "mla_use_output_gate", False))
         mats = [self.q_a, self.kv_a] + ([self.g_w] if gated else [])
         xf = x.reshape(B * Tn, x.shape[-1])
-        if B * Tn > 1 and _blas.dense_ok(xf, *mats) and _blas.weights_ok(self.q_b, self.o_w):
+        # (a gradient or tangent of anything the call reads takes the tensor form throughout)
+        rest = [self.q_an, self.kv_an, self.kv_b] + ([] if cache is None else [cache.latent, cache.rot])
+        if (B * Tn > 1 and _blas.dense_ok(xf, *mats) and _blas.weights_ok(self.q_b, self.o_w)
+                and not T.tracked(*rest)):
             qa, ckv, *g = _blas.project(xf, mats)
             qa = _rmsnorm_rows(qa, self.q_an, eps)
             q = _blas.project(qa, [self.q_b])[0].reshape(B, Tn, nh, qhd)
@@ -287,7 +291,7 @@ class MLAAttention:
                                    (lat.dtype == torch.float32 and self.kv_b.dtype == torch.bfloat16)):
             o = mla_decode_absorbed(q[0, 0, :, :nope], q[0, 0, :, nope:], self.wk, self.wv,
                                     lat[0], rot[0], scale).reshape(1, 1, nh * vhd)
-        elif self._expanded_ok(q, lat, rot):
+        elif self._expanded_ok(q, lat, rot) and not T.tracked(gate):
             o, gate = self._expanded(q, lat[0], rot[0], scale, gate), None
         else:
             o = self._dense(q.transpose(1, 2), lat, rot, scale).transpose(1, 2).reshape(B, Tn, nh * vhd)
@@ -303,7 +307,7 @@ class MLAAttention:
     def _expanded_ok(self, q, lat, rot) -> bool:
         c = self.cfg
         B, Tn = q.shape[:2]
-        if torch.is_grad_enabled() and (q.requires_grad or lat.requires_grad or self.kv_b.requires_grad):
+        if T.tracked(q, lat, rot, self.kv_b):
             return False
         return (B == 1 and Tn > 1 and lat.shape[:2] == rot.shape[:2] and lat.shape[0] == 1
                 and q.is_cuda and q.dtype == torch.float32 and lat.dtype == rot.dtype

@@ -274,7 +274,7 @@ class RoutedMoE:
         flat = x.reshape(-1, x.shape[-1])
         # (gate and up rows that do not match go on to the tensor operations, which refuse them)
         if (self.fused and flat.shape[0] and self.sh_gate.shape == self.sh_up.shape and _blas.dense_ok(flat, *mats)
-                and _blas.weights_ok(self.sh_down)):
+                and _blas.weights_ok(self.sh_down) and not T.tracked(add)):
             g, u = _blas.project(flat, mats)
             _lib.call("k3_act_rows", T.ptr(g), T.ptr(u), T.ptr(g), g.numel(), _act_code(act), float(beta),
                       float(lb or 0.0), T.stream(g))
@@ -419,7 +419,7 @@ def _rmsnorm_rows(y: torch.Tensor, w32: torch.Tensor, eps: float) -> torch.Tenso
     """_rmsnorm32 of the contiguous rows of an fp32 [M, K] device tensor in one launch."""
     M, K = y.shape
     if (M == 0 or K % 4 or not y.is_contiguous() or y.data_ptr() % 16 or w32.data_ptr() % 16 or y.dtype != torch.float32
-            or tuple(w32.shape) != (K,)):
+            or tuple(w32.shape) != (K,) or T.tracked(y, w32)):
         return _rmsnorm32(y, w32, eps)
     T.require_device(y, w32)
     out = torch.empty_like(y)

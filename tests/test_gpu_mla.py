@@ -529,3 +529,31 @@ def test_mla_many_tokens_match_fp64(T, past, heads, cache, gate):
     c2.length = Tk - 1
     one, _ = attn(x[:, -1:], c2)
     assert float((one[0, 0] - out[0, -1]).norm() / out[0, -1].norm()) <= 2e-3
+
+
+@pytest.mark.parametrize("name", ["q_a_layernorm.weight", "kv_a_layernorm.weight", "g_proj.weight", "kv_b_proj.weight"])
+def test_mla_many_tokens_keep_a_weights_gradient(name):
+    """A weight that asks for its gradient gets the one the tensor form gives (a call whose input
+    asks for one too takes that form throughout)."""
+    from types import SimpleNamespace
+    from k3hip.mla import MLAAttention
+    g = torch.Generator(device=DEV)
+    g.manual_seed(3)
+    rn = lambda *s: torch.randn(*s, device=DEV, generator=g)  # noqa: E731
+    hid, ql, heads, T = 256, 512, 4, 20
+    lin = lambda o, i: (rn(o, i) * i ** -0.5).to(torch.bfloat16)  # noqa: E731
+    w = {"q_a_proj.weight": lin(ql, hid), "q_a_layernorm.weight": 1 + 0.1 * rn(ql), "q_b_proj.weight": lin(heads * 192, ql),
+         "kv_a_proj_with_mqa.weight": lin(576, hid), "kv_a_layernorm.weight": 1 + 0.1 * rn(512),
+         "kv_b_proj.weight": lin(heads * 256, 512), "g_proj.weight": lin(heads * 128, hid),
+         "o_proj.weight": lin(hid, heads * 128)}
+    cfg = SimpleNamespace(hidden_size=hid, num_attention_heads=heads, q_lora_rank=ql, kv_lora_rank=512, qk_nope_head_dim=128,
+                          qk_rope_head_dim=64, v_head_dim=128, q_head_dim=192, rms_norm_eps=1e-5, mla_use_output_gate=True,
+                          mla_cache_dtype=torch.float32)
+    x, up = rn(1, T, hid), rn(1, T, hid)
+    grads = []
+    for xi in (x, x.clone().requires_grad_()):
+        w[name] = w[name].detach().clone().requires_grad_()
+        out, _ = MLAAttention(cfg, w)(xi)
+        (out * up).sum().backward()
+        grads.append(w[name].grad.double())
+    assert float((grads[0] - grads[1]).norm()) <= 1e-5 * float(grads[1].norm()) and float(grads[1].norm()) > 0

@@ -144,3 +144,46 @@ def test_mla_prompt_takes_one_sequence_of_one_length():
     assert not attn._expanded_ok(q, _rows(2, 20, 512), _rows(2, 20, 64))   # a cache of two sequences
     assert not attn._expanded_ok(q, _rows(1, 20, 512), _rows(1, 19, 64))
     assert not attn._expanded_ok(_dev(torch.zeros(1).expand(2, 20, 4, 192)), _rows(1, 20, 512), _rows(1, 20, 64))
+
+
+@pytest.mark.parametrize("mod", ["mla", "moe"])
+def test_norm_of_rows_keeps_gradients_and_tangents(monkeypatch, mod):
+    import importlib
+    from torch.autograd import forward_ad
+    m = importlib.import_module(f"k3hip.{mod}")
+    launches = []
+    _no_device(monkeypatch, launches)
+    x, w = torch.randn(3, 32), torch.ones(32, requires_grad=True)
+    m._rmsnorm_rows(x, w, 1e-5).sum().backward()
+    assert w.grad is not None and torch.isfinite(w.grad).all()
+    with forward_ad.dual_level():
+        y = m._rmsnorm_rows(forward_ad.make_dual(x, torch.ones_like(x)), torch.ones(32), 1e-5)
+        assert forward_ad.unpack_dual(y).tangent is not None
+    assert not launches
+    with torch.no_grad():
+        m._rmsnorm_rows(x, w, 1e-5)
+    assert launches == ["k3_rmsnorm_rows"]
+
+
+def test_routes_leave_tracked_tensors_to_tensor_operations(monkeypatch):
+    from torch.autograd import forward_ad
+    from k3hip import _blas
+    from k3hip import _torch as T
+    attn = _mla_stub()
+    q, lat, rot = _dev(torch.zeros(1).expand(1, 20, 4, 192)), _rows(1, 20, 512), _rows(1, 20, 64)
+    for args in ((_dev(q._t, requires_grad=True), lat, rot), (q, _rows(1, 20, 512, requires_grad=True), rot),
+                 (q, lat, _rows(1, 20, 64, requires_grad=True))):
+        assert not attn._expanded_ok(*args)
+    w, v = torch.zeros(16, 32, dtype=BF16), torch.zeros(16, 32, dtype=BF16)
+    assert _blas.weights_ok(_dev(w)) and not _blas.weights_ok(_dev(w), _dev(v, requires_grad=True))
+    a = torch.zeros(3, 32)
+    with forward_ad.dual_level():
+        dual = forward_ad.make_dual(a, torch.ones_like(a))
+        assert T.tracked(None, dual) and not T.tracked(None, a)
+    # a gradient of what the shared expert is added to
+    _no_device(monkeypatch, [])
+    monkeypatch.setattr(_blas, "dense", lambda a, ws, add=None: pytest.fail("a launch cuts the gradient")
+                        if add is not None else [a @ w.float().t() for w in ws])
+    add = torch.zeros(3, 32, requires_grad=True)
+    y = _layer()._shared(torch.zeros(3, 32), add)
+    assert y.requires_grad
