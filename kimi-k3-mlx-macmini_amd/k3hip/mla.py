@@ -291,7 +291,8 @@ class MLAAttention:
                                    (lat.dtype == torch.float32 and self.kv_b.dtype == torch.bfloat16)):
             o = mla_decode_absorbed(q[0, 0, :, :nope], q[0, 0, :, nope:], self.wk, self.wv,
                                     lat[0], rot[0], scale).reshape(1, 1, nh * vhd)
-        elif self._expanded_ok(q, lat, rot) and not T.tracked(gate):
+        elif (self._expanded_ok(q, lat, rot) and not T.tracked(gate)
+              and self._expand_pays(Tn, lat.shape[1], lat.dtype == torch.float32)):
             o, gate = self._expanded(q, lat[0], rot[0], scale, gate), None
         else:
             o = self._dense(q.transpose(1, 2), lat, rot, scale).transpose(1, 2).reshape(B, Tn, nh * vhd)
@@ -299,10 +300,28 @@ class MLAAttention:
             o = o * torch.sigmoid(gate)
         return mm(o, self.o_w), cache
 
-    # The expanded form forms every head's keys and values of all Tk cached positions, the
-    # absorbed form 3.4 times the work per (query, position): with few queries over a long
-    # cache the latter is less.
-    EXPAND_QUERIES, EXPAND_POSITIONS = 16, 4096
+    def _expand_pays(self, Tn: int, Tk: int, f32: bool) -> bool:
+        """Whether the expanded form (k3_mla_prefill) takes less time than the masked form for Tn queries
+        over Tk cached positions, by what each was measured to cost in us:
+
+        * expanded: forming a position's keys and values costs 0.89 ns a head (fp32 cache 1.55), however
+          few the queries; then every head is a chain of Tk / 32 steps per 128 queries, 1.7 us a
+          step (1.75) where at most 64 of the 128 are there and 2.4 (2.6) else, 256 chains at a time, a
+          group of heads (what its scratch holds) after the other;
+        * masked (fp32 library products): its launches (205), the passes over
+          the cache (0.52 ns a head and position) or 28 ps a head, query and position, whichever is most.
+
+        64 heads, bf16 cache, masked / expanded: 16 queries over 1024 positions 220 / 115, 4096 247 / 443,
+        32,768 1488 / 8852; 128 queries over 4096 939 / 545, 16,384 3589 / 3366, 32,768 7678 / 11,984; 256
+        over 32,768 15,225 / 11,969.  fp32 cache: 2 queries over 2048 203 / 269, 128 over 4096 935 / 661.
+        16 heads: 128 queries over 4096 336 / 376, 256 558 / 376."""
+        heads = self.cfg.num_attention_heads
+        padded = _round_up(Tk, 32)
+        group = _lib.size("k3_mla_prefill_workspace_size", Tk, heads) // (padded * 2 * 3 * 2 * 128)
+        turns = -(-group * -(-Tn // 128) // 256) * -(-heads // group)
+        step = (1.75 if f32 else 1.7) if Tn <= 64 else (2.6 if f32 else 2.4)
+        expanded = (1.55e-3 if f32 else 8.9e-4) * Tk * heads + turns * padded / 32 * step
+        return expanded < max(205.0, 5.2e-4 * Tk * heads, 2.8e-5 * Tn * Tk * heads)
 
     def _expanded_ok(self, q, lat, rot) -> bool:
         c = self.cfg
@@ -314,8 +333,7 @@ class MLAAttention:
                 and lat.dtype in (torch.bfloat16, torch.float32) and self.kv_b.dtype == torch.bfloat16
                 and self.kv_b.is_contiguous() and self.kv_b.data_ptr() % 16 == 0
                 and (c.kv_lora_rank, c.qk_rope_head_dim, c.qk_nope_head_dim, c.v_head_dim) == (KV_LORA_RANK, ROPE_DIM, 128, 128)
-                and c.q_head_dim == 192
-                and (Tn >= self.EXPAND_QUERIES or lat.shape[1] <= self.EXPAND_POSITIONS))
+                and c.q_head_dim == 192)
 
     def _expanded(self, q, lat, rot, scale, gate):
         """Multi-token form (prefill) of one sequence through k3_mla_prefill: q [1, T, H, 192] fp32 over the

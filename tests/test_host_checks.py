@@ -187,3 +187,21 @@ def test_routes_leave_tracked_tensors_to_tensor_operations(monkeypatch):
     add = torch.zeros(3, 32, requires_grad=True)
     y = _layer()._shared(torch.zeros(3, 32), add)
     assert y.requires_grad
+
+
+# (heads, fp32 cache, cached positions, queries, masked form us, expanded form us)
+MLA_FORMS = [(64, False, 256, 2, 218, 51), (64, False, 1024, 16, 220, 115), (64, False, 1024, 128, 336, 138),
+             (64, False, 2048, 128, 531, 256), (64, False, 4096, 2, 224, 442), (64, False, 4096, 16, 247, 443),
+             (64, False, 4096, 128, 939, 545), (64, False, 8192, 16, 443, 860), (64, False, 8192, 128, 1791, 1065),
+             (64, False, 16384, 64, 1831, 2667), (64, False, 16384, 256, 7071, 3375), (64, False, 32768, 16, 1488, 8852),
+             (64, False, 32768, 96, 5782, 11407), (64, False, 32768, 256, 15225, 11969), (64, False, 65536, 16, 2982, 31724),
+             (64, False, 65536, 192, 32909, 44087), (64, True, 1024, 16, 203, 148), (64, True, 2048, 2, 203, 269),
+             (64, True, 4096, 16, 236, 544), (64, True, 4096, 128, 935, 661), (64, True, 32768, 48, 3361, 10594),
+             (16, False, 1024, 8, 214, 92), (16, False, 4096, 128, 336, 376), (16, False, 4096, 256, 558, 376),
+             (16, False, 32768, 16, 539, 2205), (16, False, 32768, 256, 3647, 2974)]
+
+
+@pytest.mark.parametrize("heads,f32,Tk,T,masked,expanded", MLA_FORMS)
+def test_mla_form_for_several_tokens_is_the_shorter_one(heads, f32, Tk, T, masked, expanded):
+    """Both forms were measured at each of these; the rule takes the one that was shorter."""
+    assert _mla_stub(heads)._expand_pays(T, Tk, f32) == (expanded < masked)
