@@ -67,6 +67,10 @@ int k3_scale_minmax(const void *scales, int64_t n, int32_t *minmax, void *stream
 int k3_mxfp4_matvec(const void *x, int x_dtype, const void *packed, const void *scales,
                     void *out, int out_dtype, int64_t M, int64_t N, int64_t K, void *stream);
 
+/* Kernel launches k3_mxfp4_matvec makes for these sizes (0 where it refuses them): one where the
+ * matrix-core form takes all M tokens, else one per token tile of the GEMV. */
+int64_t k3_mxfp4_matvec_launches(int64_t M, int64_t N, int64_t K, int x_dtype);
+
 /* ---- MoE expert FFN ---------------------------------------------------------------- */
 
 /* Workspace bytes k3_expert_ffn needs for intermediate size I (the fp32 act vector passed

@@ -212,18 +212,41 @@ int launch_tt(const GemvArgs &a, hipStream_t st) {
 
 }  // namespace
 
-// A few tokens of few weights finish sooner in GEMV launches of four tokens: the matmul stages
-// whole 16-token tiles and walks K in one chain of steps, whatever M and N.  Both sides as fits
-// in us of launches measured over M 5..32, N 300..8192, K 1024..7168 (GEMV / matmul): fp32 x,
-// K = 7168: 5 tokens of 300 rows 9.0 / 17.5, 8 of 1024 rows 13.1 / 17.7, 12 of 1024 rows 19.3 /
-// 17.4, 8 of 2048 rows 23.1 / 17.4; K = 1024: 5 of 300 rows 5.3 / 5.0.  bf16 x, K = 7168: 5 tokens
-// of 300 rows 6.9 / 8.1, 8 of 300 rows 8.9 / 8.1.
+// A few tokens of few weights finish sooner in GEMV launches: the matmul stages whole 16-token
+// tiles and walks K in one chain of steps, whatever M and N.  The costs are fits in us of launches
+// measured over M 5..37, N 64..8192, K 1024..32,704.
+// K below 8192 (GEMV / matmul): fp32 x, K = 7168: 5 tokens of 300 rows 9.0 / 17.5, 8 of 1024 rows
+// 13.1 / 17.7, 12 of 1024 rows 19.3 / 17.4, 8 of 2048 rows 23.1 / 17.4; K = 1024: 5 of 300 rows
+// 5.3 / 5.0.  bf16 x, K = 7168: 5 tokens of 300 rows 6.9 / 8.1, 8 of 300 rows 8.9 / 8.1.
+// From 8192 on a GEMV launch takes four tokens up to the K whose activations a block holds
+// (gemv_token_tile: fp32 8192, bf16 16,384), then one.  fp32 x: 8 tokens of 300 rows at K = 8192
+// 13.2 / 22, 5 tokens of 1024 rows at 12,288 20.3 / 31.2, of 4096 rows 37.6 / 32.7, 8 tokens of
+// 300 rows at 16,384 32.9 / 39.9, 12 tokens 48.6 / 40.0.  bf16 x: 5 tokens of 300 rows at 12,288
+// 10.0 / 15.3, 8 tokens 12.7 / 15.3, 12 tokens at 16,384 21.1 / 19.0, 5 of 2048 rows there 17.9 / 19.1.
+// Of 1195 measured points with K from 8192 on, every one is within 7% of its shorter form.
 static bool gemv_sooner(int64_t M, int64_t N, int64_t K, bool x_bf16) {
-    if (M > 20 || K < 2048 || K > 8192 || (x_bf16 && N > 4096)) return false;
-    const double k = static_cast<double>(K), w = static_cast<double>(N) * k, waves = static_cast<double>(cdiv(N, 16 * 256));
-    const double per = x_bf16 ? 0.8e-4 + w / 400e9 : 0.95e-4 + w / 95e9;   // of a GEMV, per token and element
-    const double step = (x_bf16 ? k / 1500 : k / 500) * static_cast<double>(cdiv(M, 16));
-    return 2.0 * static_cast<double>(cdiv(M, 4)) + static_cast<double>(M) * k * per < (3.2 + step) * waves;
+    if (M > 20 || K < 2048 || (N > 4096 && (x_bf16 || K >= 8192))) return false;
+    const double k = static_cast<double>(K);
+    if (K < 8192) {
+        const double w = static_cast<double>(N) * k, waves = static_cast<double>(cdiv(N, 16 * 256));
+        const double per = x_bf16 ? 0.8e-4 + w / 400e9 : 0.95e-4 + w / 95e9;   // of a GEMV, per token and element
+        const double step = (x_bf16 ? k / 1500 : k / 500) * static_cast<double>(cdiv(M, 16));
+        return 2.0 * static_cast<double>(cdiv(M, 4)) + static_cast<double>(M) * k * per < (3.2 + step) * waves;
+    }
+    // (rows of a multiple of 4096 elements meet the same memory channels)
+    double matmul = x_bf16 ? (4.4 + 0.7e-3 * k) * (K % 4096 ? 1.0 : 1.18) : 3.2 + k / 455;
+    if (M > 16) matmul *= x_bf16 ? 1.4 : 1.7;
+    const int rows = static_cast<int>(cdiv(N, 1024));       // a GEMV launch's cost steps with these
+    if (gemv_token_tile(K, x_bf16) == 1) {
+        const double one = x_bf16 ? 3 + 8.5e-5 * k : 3.45 + 4e-5 * k;
+        return static_cast<double>(M) * one * (rows == 1 ? 1.0 : rows == 2 ? 1.45 : 2.0) < matmul;
+    }
+    double four = x_bf16 ? (K == 8192 ? 4.8 : 5.4 + 9e-5 * k) : 6.5;     // a launch of four tokens, of one
+    double one = x_bf16 ? (K == 8192 ? 2.7 : 2.4 + 7.5e-5 * k) : 3.5;
+    if (rows > 1) four *= rows > 2 ? 2.4 : x_bf16 && K == 8192 ? 1.33 : 1.8, one *= 1.2;
+    const int64_t rest = M % 4;
+    const double gemv = static_cast<double>(M / 4) * four + (rest ? one + (four - one) * static_cast<double>(rest - 1) / 3 : 0);
+    return gemv < matmul;
 }
 
 bool mxfp4_gemm_takes(int64_t M, int64_t N, int64_t K, bool x_bf16) {

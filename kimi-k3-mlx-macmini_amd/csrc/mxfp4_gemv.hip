@@ -297,6 +297,13 @@ static int matvec_impl(const void *x, int x_dtype, const void *packed, const voi
     return K3_OK;
 }
 
+extern "C" int64_t k3_mxfp4_matvec_launches(int64_t M, int64_t N, int64_t K, int x_dtype) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % 32 || (x_dtype != K3_F32 && x_dtype != K3_BF16)) return 0;
+    const int mt = gemv_token_tile(K, x_dtype == K3_BF16);
+    if (mt == 0) return 0;
+    return mxfp4_gemm_takes(M, N, K, x_dtype == K3_BF16) ? 1 : cdiv(M, mt);
+}
+
 extern "C" int k3_mxfp4_matvec(const void *x, int x_dtype, const void *packed, const void *scales,
                                void *out, int out_dtype, int64_t M, int64_t N, int64_t K,
                                void *stream) {

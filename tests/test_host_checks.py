@@ -205,3 +205,29 @@ MLA_FORMS = [(64, False, 256, 2, 218, 51), (64, False, 1024, 16, 220, 115), (64,
 def test_mla_form_for_several_tokens_is_the_shorter_one(heads, f32, Tk, T, masked, expanded):
     """Both forms were measured at each of these; the rule takes the one that was shorter."""
     assert _mla_stub(heads)._expand_pays(T, Tk, f32) == (expanded < masked)
+
+
+# (bf16 x, K, N, tokens, GEMV launches us, one matmul us)
+MATVEC_FORMS = [(False, 7168, 300, 5, 9.0, 17.5), (False, 7168, 2048, 8, 23.1, 17.4), (False, 8192, 300, 8, 13.2, 22.0),
+                (False, 8192, 300, 16, 25.3, 21.9), (False, 8192, 2048, 8, 24.3, 22.6), (False, 12288, 64, 5, 19.1, 30.1),
+                (False, 12288, 1024, 5, 20.3, 31.2), (False, 12288, 2048, 5, 25.9, 31.4), (False, 12288, 4096, 5, 37.6, 32.7),
+                (False, 12288, 300, 12, 45.6, 30.9), (False, 16384, 300, 5, 20.8, 39.5), (False, 16384, 1024, 8, 33.9, 40.4),
+                (False, 16384, 1024, 12, 49.9, 40.2), (False, 16384, 4096, 8, 68.1, 41.1), (True, 8192, 1024, 8, 10.0, 11.5),
+                (True, 8192, 1024, 12, 14.6, 11.6), (True, 8192, 2048, 5, 9.5, 11.6), (True, 12288, 64, 8, 12.2, 14.9),
+                (True, 12288, 1024, 5, 10.5, 15.4), (True, 12288, 4096, 5, 21.7, 15.7), (True, 16384, 300, 8, 14.3, 18.8),
+                (True, 16384, 1024, 12, 22.0, 19.1), (True, 16384, 2048, 8, 26.3, 19.2), (True, 24576, 300, 5, 23.2, 26.3)]
+
+
+@pytest.mark.parametrize("bf,K,N,M,gemv,matmul", MATVEC_FORMS)
+def test_matvec_form_for_a_few_tokens_is_the_shorter_one(bf, K, N, M, gemv, matmul):
+    """Both forms were measured at each of these; k3_mxfp4_matvec takes the one that was shorter."""
+    from k3hip import _lib
+    n = _lib.lib().k3_mxfp4_matvec_launches(M, N, K, _lib.K3_BF16 if bf else _lib.K3_F32)
+    assert (n > 1) == (gemv < matmul)
+
+
+def test_matvec_launches_of_refused_sizes():
+    from k3hip import _lib
+    f = _lib.lib().k3_mxfp4_matvec_launches
+    assert f(1, 64, 4096, 0) == 1 and f(3, 64, 16384, 0) == 3 and f(4, 64, 16384, 1) == 1
+    assert [f(0, 64, 64, 0), f(1, 64, 48, 0), f(1, 64, 1 << 20, 0), f(1, 64, 64, 7)] == [0] * 4
