@@ -79,17 +79,25 @@ def dense(a: torch.Tensor, ws, add: torch.Tensor | None = None) -> list[torch.Te
     return outs
 
 
-def project(a: torch.Tensor, ws) -> list[torch.Tensor]:
-    """[a [M, K] @ w[N, K]^T in fp32 for w in ws], all against one activation.
+def one_launch(M: int, K: int, rows: list[int]) -> bool:
+    """Whether one k3_dense launch takes several bf16 matrices against M bf16 tokens (one matrix-core
+    pass) sooner than a library GEMM each.  Up to 64 tokens it does at every set measured, weights not
+    yet cached (library / k3_dense us): 1536 + 576 + 8192 rows of 7168 2 tokens 48.6 / 36.1, 64 tokens
+    64 / 41; 512 + 512 of 1024 11.2 / 10.5; 4 x 12,288 + 224 of 7168 163 / 130; at worst 6144 + 6144 of
+    7168, 2 tokens 40.2 / 42.0.  Beyond, its K split costs small sets more than the launches it saves:
+    512 + 512 of 1024, 256 tokens 15.9 / 21.6; 2048 + 2048 of 2048 (8.4 million weights) 23.5 / 29.2; but
+    three matrices, 768 + 576 + 2048 of 2048 (6.9 million), 33.5 / 29.7, 1536 + 576 of 7168 (15 million)
+    43.4 / 37.9, 2048 + 2048 of 7168, 700 tokens 82.7 / 66.9.  Beyond 1024 tokens neither leads throughout (1536 + 576 + 8192 of 7168, 1500
+    tokens 236 / 193, 2048 tokens 288 / 343)."""
+    return len(rows) > 1 and (M <= 64 or (M <= 1024 and len(rows) * sum(rows) * K >= 20_000_000))
 
-    fp32 a: one k3_dense launch.  bf16 a, which needs one matrix-core pass: k3_dense for several
-    matrices of up to 1024 tokens, where one launch replaces a library GEMM each (224 + 4 x
-    12,288 rows of 7168: 2 tokens 120 against 153 us, 256 tokens 217 against 349 us; 10,304 rows
-    in three matrices: 64 tokens 34 against 63 us, 1000 tokens 156 against 158 us), and for one
-    matrix of 65 to 256 tokens, where its K split fills the chip (256 x 7168 x 12288: 64 against
-    111 us); the library elsewhere (700 x 7168 x 2048: 48 against 28 us)."""
+
+def project(a: torch.Tensor, ws) -> list[torch.Tensor]:
+    """[a [M, K] @ w[N, K]^T in fp32 for w in ws], all against one activation: fp32 a in one k3_dense
+    launch (three library products a matrix were slower at every size measured, 2 to 2048 tokens of
+    64 to 12,288 rows); bf16 a where one_launch holds, on the library elsewhere."""
     M = a.shape[0]
-    if M and dense_ok(a, *ws) and (a.dtype == torch.float32 or (len(ws) > 1 and M <= 1024) or 64 < M <= 256):
+    if M and dense_ok(a, *ws) and (a.dtype == torch.float32 or one_launch(M, a.shape[1], [w.shape[0] for w in ws])):
         return dense(a, list(ws))
     return [mm_f32(a, w) for w in ws]
 

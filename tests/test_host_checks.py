@@ -231,3 +231,22 @@ def test_matvec_launches_of_refused_sizes():
     f = _lib.lib().k3_mxfp4_matvec_launches
     assert f(1, 64, 4096, 0) == 1 and f(3, 64, 16384, 0) == 3 and f(4, 64, 16384, 1) == 1
     assert [f(0, 64, 64, 0), f(1, 64, 48, 0), f(1, 64, 1 << 20, 0), f(1, 64, 64, 7)] == [0] * 4
+
+
+# (K, rows of each matrix, tokens, library us, one launch us), weights not yet cached
+PROJECTIONS = [(7168, [1536, 576, 8192], 2, 48.6, 36.1), (7168, [1536, 576, 8192], 700, 154.5, 126.9),
+               (7168, [1536, 576, 8192], 2048, 287.8, 343.3), (2048, [768, 576, 2048], 64, 33.0, 18.3),
+               (2048, [768, 576, 2048], 256, 33.5, 29.7), (7168, [12288] * 4, 1500, 963, 900), (1024, [512, 512], 24, 11.4, 11.0),
+               (1024, [512, 512], 256, 15.9, 21.6), (1024, [512, 512], 1000, 17.3, 28.2), (2048, [768, 576], 64, 15.9, 14.6),
+               (2048, [768, 576], 192, 16.4, 25.5), (2048, [2048, 2048], 32, 22.4, 15.5), (2048, [2048, 2048], 384, 25.8, 35.4),
+               (4096, [1024, 1024], 256, 25.0, 29.0), (7168, [1024, 1024], 256, 38.2, 36.4), (7168, [2048, 2048], 700, 82.7, 66.9),
+               (7168, [3072, 3072], 1000, 129.9, 117.1)]
+
+
+@pytest.mark.parametrize("K,rows,M,library,launch", PROJECTIONS)
+def test_projections_of_bf16_tokens_take_the_shorter_form(K, rows, M, library, launch):
+    """Both were measured at each of these; past 1024 tokens, where neither leads throughout, the
+    library is taken."""
+    from k3hip import _blas
+    assert not _blas.one_launch(M, K, rows[:1])
+    assert _blas.one_launch(M, K, rows) == (launch < library and M <= 1024)
