@@ -40,29 +40,36 @@ def _mm_bf16_f32(a2: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return torch.mm(a2, w.t(), out_dtype=torch.float32)
 
 
+def _rows_ok(w: torch.Tensor) -> bool:
+    return (w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() and w.data_ptr() % 16 == 0
+            and w.shape[1] % 8 == 0 and w.shape[0] > 0)
+
+
 def weights_ok(*ws: torch.Tensor) -> bool:
     """k3_dense takes these weights as they are: bf16 device matrices of whole 16-byte rows."""
-    return not T.tracked(*ws) and all(w.is_cuda and w.dim() == 2 and w.dtype == torch.bfloat16 and w.is_contiguous()
-                                      and w.data_ptr() % 16 == 0 and w.shape[1] % 8 == 0 and w.shape[0] > 0 for w in ws)
+    return not T.tracked(*ws) and all(map(_rows_ok, ws))
 
 
 def dense_ok(a: torch.Tensor, *ws: torch.Tensor) -> bool:
     """k3_dense takes a against these weights as they are, and no gradient is asked for."""
-    return (a.is_cuda and a.dtype in (torch.float32, torch.bfloat16) and not T.tracked(a)
-            and weights_ok(*ws) and all(w.shape[1] == a.shape[-1] and w.device == a.device for w in ws))
+    if not a.is_cuda or a.dtype not in (torch.float32, torch.bfloat16) or T.tracked(a, *ws):
+        return False
+    K, dev = a.shape[-1], a.get_device()
+    for w in ws:
+        if not _rows_ok(w) or w.shape[1] != K or w.get_device() != dev:
+            return False
+    return True
 
 
 def dense(a: torch.Tensor, ws, add: torch.Tensor | None = None) -> list[torch.Tensor]:
-    """[a [M, K] @ w[N, K]^T in fp32 for w in ws] (k3_dense; dtypes and alignment checked by dense_ok),
-    plus ``add`` [M, N] fp32 where one weight is given."""
+    """[a [M, K] @ w[N, K]^T in fp32 for w in ws] (k3_dense; a and ws checked by dense_ok), plus
+    ``add`` [M, N] fp32 where one weight is given."""
     M, K = a.shape
-    if any(w.shape[1] != K for w in ws):
-        raise ValueError(f"a is [{M}, {K}]; weights {[tuple(w.shape) for w in ws]}")
     if add is not None:
         if len(ws) != 1 or tuple(add.shape) != (M, ws[0].shape[0]) or add.dtype != torch.float32:
             raise ValueError(f"add must be float32 [{M}, N] beside one weight [N, {K}]; got {add.dtype} {tuple(add.shape)}")
+        T.require_device(a, add)
         add = T.contiguous_aligned(add)
-    T.require_device(a, add, *ws)
     if a.stride(1) != 1 or (a.stride(0) * a.element_size()) % 16 or a.stride(0) < K or a.data_ptr() % 16:
         a = T.contiguous_aligned(a)
     n = len(ws)

@@ -53,9 +53,14 @@ def require_device(*ts: torch.Tensor) -> None:
 def tracked(*ts: torch.Tensor | None) -> bool:
     """A gradient, or a forward-mode tangent, of one of these is asked for: the launches carry
     neither, so such a call stays on the tensor operations that do."""
-    grad = torch.is_grad_enabled()
-    return any(t is not None and ((grad and t.requires_grad) or forward_ad.unpack_dual(t).tangent is not None)
-               for t in ts)
+    if torch.is_grad_enabled():
+        for t in ts:
+            if t is not None and t.requires_grad:
+                return True
+    # (unpack_dual takes half a microsecond a tensor: only inside a dual level, or where torch no longer says)
+    if getattr(forward_ad, "_current_level", 0) >= 0:
+        return any(t is not None and forward_ad.unpack_dual(t).tangent is not None for t in ts)
+    return False
 
 
 def contiguous_aligned(t: torch.Tensor) -> torch.Tensor:

@@ -42,23 +42,33 @@ def kda_recurrent(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Te
     dt = torch.bfloat16 if all(t.dtype == torch.bfloat16 for t in (q, k, v, g, beta)) else torch.float32
     # time-major, so each step's [B, heads, dim] slice is contiguous
     q, k, v, g, beta = (t.to(dt).transpose(0, 1).contiguous() for t in (q, k, v, g, beta))
+    S = _state(state, (B, HV, K, V), q.device)
+    return _recurrent(q, k, v, g, beta, float(scale), S).transpose(0, 1), S
+
+
+def _state(state: torch.Tensor | None, shape: tuple, device) -> torch.Tensor:
+    """The state to update in place: the given one where the kernels can, else a copy, or zeros."""
     if state is None:
-        S = torch.zeros((B, HV, K, V), dtype=torch.float32, device=q.device)
-    elif tuple(state.shape) != (B, HV, K, V):
-        raise ValueError(f"state must be [{B}, {HV}, {K}, {V}]; got {tuple(state.shape)}")
-    elif state.dtype == torch.float32 and state.is_contiguous() and state.data_ptr() % 16 == 0:
-        S = state
-    else:
-        S = state.to(torch.float32).contiguous().clone()
+        return torch.zeros(shape, dtype=torch.float32, device=device)
+    if tuple(state.shape) != shape:
+        raise ValueError(f"state must be {list(shape)}; got {tuple(state.shape)}")
+    if state.dtype == torch.float32 and state.is_contiguous() and state.data_ptr() % 16 == 0:
+        return state
+    return state.to(torch.float32).contiguous().clone()
+
+
+def _recurrent(q, k, v, g, beta, scale: float, S: torch.Tensor) -> torch.Tensor:
+    """All tokens of contiguous time-major q, k [T, B, H, K], v [T, B, HV, V], g [T, B, HV, K], beta
+    [T, B, HV] on the state S in one launch -> o [T, B, HV, V] fp32."""
+    Tn, B, H, K = q.shape
+    HV, V = v.shape[2], v.shape[3]
     o = torch.empty((Tn, B, HV, V), dtype=torch.float32, device=q.device)
-    code = T.dtype_code(dt)
-    st = T.stream(q)
     # B sequences are B * HV independent heads: q/k head b * H + h serves value heads
     # (b * HV + h * G) .. + G, the same grouping as within one sequence; all tokens in one
     # launch, the state kept in registers between them
-    _lib.call("k3_kda_recurrent", T.ptr(q), T.ptr(k), T.ptr(v), T.ptr(g), T.ptr(beta), code, T.ptr(S), T.ptr(o),
-              _lib.K3_F32, Tn, B * H, B * HV, K, V, float(scale), st)
-    return o.transpose(0, 1), S
+    _lib.call("k3_kda_recurrent", T.ptr(q), T.ptr(k), T.ptr(v), T.ptr(g), T.ptr(beta), T.dtype_code(q.dtype), T.ptr(S),
+              T.ptr(o), _lib.K3_F32, Tn, B * H, B * HV, K, V, scale, T.stream(q))
+    return o
 
 
 class KDAAttention:
@@ -101,14 +111,15 @@ class KDAAttention:
 
     def _check_widths(self) -> None:
         """The launches of prefill read these weights at the layer's widths, whatever their shapes."""
-        P = self.H * self.D
-        for name, w, rows in (("q_proj", self.q_w, P), ("k_proj", self.k_w, P), ("v_proj", self.v_w, P),
-                              ("g_proj", self.g_w, P), ("f_b_proj", self.fb, P), ("b_proj", self.b_w, self.H)):
-            if w.dim() != 2 or w.shape[0] != rows:
-                raise ValueError(f"{name} must have {rows} rows; got {tuple(w.shape)}")
-        if self.dt_bias.numel() != P or self.o_norm_w.numel() != self.D or self.A_log.numel() < self.H:
-            raise ValueError(f"dt_bias [{P}], o_norm [{self.D}] and A_log for {self.H} heads expected; got "
-                             f"{self.dt_bias.numel()}, {self.o_norm_w.numel()} and {self.A_log.numel()} values")
+        H, D = self.H, self.D
+        P = H * D
+        if (self.q_w.shape[0] == self.k_w.shape[0] == self.v_w.shape[0] == self.g_w.shape[0] == self.fb.shape[0] == P
+                and self.b_w.shape[0] == H and self.dt_bias.numel() == P and self.o_norm_w.numel() == D
+                and self.A_log.numel() >= H):
+            return
+        raise ValueError(f"{H} heads of {D} do not match " + ", ".join(f"{n} {tuple(w.shape)}" for n, w in (
+            ("q_proj", self.q_w), ("k_proj", self.k_w), ("v_proj", self.v_w), ("g_proj", self.g_w), ("f_b_proj", self.fb),
+            ("b_proj", self.b_w), ("dt_bias", self.dt_bias), ("o_norm", self.o_norm_w), ("A_log", self.A_log))))
 
     def prefill(self, x: torch.Tensor, state: torch.Tensor | None = None, conv: tuple | None = None):
         """Many tokens (attention_kda.py:94-115): the projections of all tokens (each weight
@@ -143,8 +154,8 @@ class KDAAttention:
         _lib.call("k3_kda_prefill_inputs", *(T.ptr(t) for t in (yq, yk, yv, fb, br, self.qc, self.kc, self.vc, *wins,
                                                                 *states, self.A_log, self.dt_bias, q, k, v, g, beta)),
                   B, Tn, H, D, K, float(c.kda_gate_lower_bound), st)
-        o, state = kda_recurrent(*(t.transpose(0, 1) for t in (q, k, v, g, beta)), D ** -0.5, state)
-        o = o.transpose(0, 1)                     # [T, B, H, D], as the launch wrote it
+        state = _state(state, (B, H, D, D), dev)
+        o = _recurrent(q, k, v, g, beta, D ** -0.5, state)
         y = torch.empty((B * Tn, P), dtype=torch.float32, device=dev)
         _lib.call("k3_kda_gated_norm", T.ptr(o), T.ptr(og), T.ptr(self.o_norm_w), float(c.rms_norm_eps), T.ptr(y), B, Tn,
                   H, D, st)
@@ -157,12 +168,7 @@ class KDAAttention:
             return self.prefill(x, state, conv)
         H, D, K = self.H, self.D, self.K
         P = H * D
-        if state is None:
-            state = torch.zeros((B, H, D, D), dtype=torch.float32, device=x.device)
-        elif tuple(state.shape) != (B, H, D, D):
-            raise ValueError(f"state must be [{B}, {H}, {D}, {D}]; got {tuple(state.shape)}")
-        elif not (state.dtype == torch.float32 and state.is_contiguous() and state.data_ptr() % 16 == 0):
-            state = state.to(torch.float32).contiguous().clone()
+        state = _state(state, (B, H, D, D), x.device)
         # the windows of q, k and v in one buffer (one launch, or none where a caller passes back
         # the views a call returned); the step writes every element of the next ones
         fin = torch.empty((1, 3, K - 1, P), dtype=torch.float32, device=x.device)

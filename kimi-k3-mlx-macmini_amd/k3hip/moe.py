@@ -272,9 +272,10 @@ class RoutedMoE:
         act, beta, lb = self._act()
         mats = [self.sh_gate, self.sh_up]
         flat = x.reshape(-1, x.shape[-1])
-        # (gate and up rows that do not match go on to the tensor operations, which refuse them)
+        # (matrices that do not match go on to the tensor operations, which refuse them)
         if (self.fused and flat.shape[0] and self.sh_gate.shape == self.sh_up.shape and _blas.dense_ok(flat, *mats)
-                and _blas.weights_ok(self.sh_down) and not T.tracked(add)):
+                and _blas.weights_ok(self.sh_down) and self.sh_down.shape[1] == self.sh_gate.shape[0]
+                and self.sh_down.device == flat.device and not T.tracked(add)):
             g, u = _blas.project(flat, mats)
             _lib.call("k3_act_rows", T.ptr(g), T.ptr(u), T.ptr(g), g.numel(), _act_code(act), float(beta),
                       float(lb or 0.0), T.stream(g))

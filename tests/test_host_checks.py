@@ -53,7 +53,7 @@ def _no_device(monkeypatch, launches):
     monkeypatch.setattr(T, "require_device", lambda *ts: None)
     monkeypatch.setattr(T, "stream", lambda t: 0)
     monkeypatch.setattr(_blas, "weights_ok", lambda *ws: True)
-    monkeypatch.setattr(_blas, "dense_ok", lambda a, *ws: True)
+    monkeypatch.setattr(_blas, "dense_ok", lambda a, *ws: all(w.shape[1] == a.shape[-1] for w in ws))
     monkeypatch.setattr(_blas, "_mm_bf16_f32", lambda a, w: a.float() @ w.float().t())
     monkeypatch.setattr(_lib, "call", lambda name, *a: launches.append(name))
 
