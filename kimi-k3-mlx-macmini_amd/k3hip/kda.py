@@ -169,6 +169,10 @@ class KDAAttention:
         H, D, K = self.H, self.D, self.K
         P = H * D
         state = _state(state, (B, H, D, D), x.device)
+        if B * Tn == 0:      # nothing to do: the state and the windows as they came
+            wins = [torch.zeros((B, K - 1, P), dtype=torch.float32, device=x.device) if conv is None
+                    else conv[m].to(torch.float32).reshape(B, K - 1, P).clone() for m in range(3)]
+            return torch.empty((B, Tn, hid), dtype=torch.float32, device=x.device), state, tuple(wins)
         # the windows of q, k and v in one buffer (one launch, or none where a caller passes back
         # the views a call returned); the step writes every element of the next ones
         fin = torch.empty((1, 3, K - 1, P), dtype=torch.float32, device=x.device)

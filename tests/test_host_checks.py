@@ -250,3 +250,18 @@ def test_projections_of_bf16_tokens_take_the_shorter_form(K, rows, M, library, l
     from k3hip import _blas
     assert not _blas.one_launch(M, K, rows[:1])
     assert _blas.one_launch(M, K, rows) == (launch < library and M <= 1024)
+
+
+@pytest.mark.parametrize("B,T", [(1, 0), (2, 0), (0, 3)])
+def test_kda_without_tokens_returns_the_state_and_windows(monkeypatch, B, T):
+    launches = []
+    _no_device(monkeypatch, launches)
+    kda = _kda()
+    x = torch.zeros(B, T, 64)
+    out, state, conv = kda(x)
+    assert out.shape == (B, T, 64) and state.shape == (B, 2, 128, 128) and not state.any()
+    assert [tuple(c.shape) for c in conv] == [(B, 3, 256)] * 3 and not any(c.any() for c in conv)
+    S, wins = torch.randn(B, 2, 128, 128), tuple(torch.randn(B, 3, 256) for _ in range(3))
+    out, state, conv = kda(x, S, wins)
+    assert state is S and all(torch.equal(a, b) and a.dtype == torch.float32 for a, b in zip(conv, wins))
+    assert not launches
