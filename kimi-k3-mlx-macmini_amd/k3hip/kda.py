@@ -145,8 +145,8 @@ class KDAAttention:
             fa, br = (_blas.mm_f32(xf, w) for w in mats[4:])
         fb = _blas.project(fa, [self.fb])[0]
         wins = [None] * 3 if conv is None else [
-            T.contiguous_aligned(conv[m].detach().to(torch.float32).reshape(B, K - 1, P)) for m in range(3)]
-        T.require_device(x, state, *wins)
+            T.contiguous_aligned(conv[m].detach().to(dev, torch.float32).reshape(B, K - 1, P)) for m in range(3)]
+        T.require_device(x, state)
         states = tuple(torch.empty((B, K - 1, P), dtype=torch.float32, device=dev) for _ in range(3))
         q, k, v, g = (torch.empty((Tn, B, H, D), dtype=torch.float32, device=dev) for _ in range(4))
         beta = torch.empty((Tn, B, H), dtype=torch.float32, device=dev)
@@ -171,7 +171,7 @@ class KDAAttention:
         state = _state(state, (B, H, D, D), x.device)
         if B * Tn == 0:      # nothing to do: the state and the windows as they came
             wins = [torch.zeros((B, K - 1, P), dtype=torch.float32, device=x.device) if conv is None
-                    else conv[m].to(torch.float32).reshape(B, K - 1, P).clone() for m in range(3)]
+                    else conv[m].to(x.device, torch.float32).reshape(B, K - 1, P).clone() for m in range(3)]
             return torch.empty((B, Tn, hid), dtype=torch.float32, device=x.device), state, tuple(wins)
         # the windows of q, k and v in one buffer (one launch, or none where a caller passes back
         # the views a call returned); the step writes every element of the next ones
@@ -179,9 +179,8 @@ class KDAAttention:
         if conv is None:
             cin = torch.zeros((3, K - 1, P), dtype=torch.float32, device=x.device)
         else:
-            wins = [c.to(torch.float32).reshape(1, K - 1, P) for c in conv]
+            wins = [c.to(x.device, torch.float32).reshape(1, K - 1, P) for c in conv]
             step = (K - 1) * P * 4
-            T.require_device(x, *wins)
             if (all(c.is_contiguous() for c in wins) and wins[0].data_ptr() % 16 == 0
                     and all(wins[m].data_ptr() == wins[0].data_ptr() + m * step for m in (1, 2))):
                 cin = wins[0]

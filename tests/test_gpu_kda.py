@@ -242,3 +242,16 @@ def test_kda_prefill_windows_and_batches(B, Tn, conv):
     want, want_S, want_cv = okda.kda_layer(cfg, w, x, S0, cv0)
     assert om.normwise_rel(out.cpu().numpy(), want) <= 2e-5 and om.normwise_rel(S.cpu().numpy(), want_S) <= 2e-5
     assert max(om.normwise_rel(a.cpu().numpy(), b) for a, b in zip(cv, want_cv)) <= 2e-6
+
+
+@pytest.mark.parametrize("Tn", [1, 3, 12])
+def test_kda_windows_kept_on_the_host(Tn):
+    """Convolution windows that a program kept in host memory continue a sequence as the device
+    ones do, one token or several."""
+    cfg, w, attn, rng = _layer(41, 256, 2, scale=0.05)
+    x = torch.from_numpy(rng.standard_normal((1, Tn, 256)).astype(np.float32)).to(DEV)
+    wins = tuple(torch.from_numpy(rng.standard_normal((1, 3, 256)).astype(np.float32)) for _ in range(3))
+    out, S, conv = attn(x, conv=wins)
+    want = attn(x, conv=tuple(c.to(DEV) for c in wins))
+    assert torch.equal(out, want[0]) and torch.equal(S, want[1])
+    assert all(torch.equal(a, b) for a, b in zip(conv, want[2]))
