@@ -347,7 +347,9 @@ constexpr int kPrepTokens = 8;
 
 __global__ __launch_bounds__(128) void kda_prep_kernel(KdaPrepArgs a) {
     __shared__ float part[2][kPrepTokens][2];
-    const int c = threadIdx.x, h = blockIdx.x, t0 = blockIdx.y * kPrepTokens, b = blockIdx.z;
+    // blocks: head, then eight tokens, then sequence
+    const int nt = (a.T + kPrepTokens - 1) / kPrepTokens, tile = blockIdx.x / a.H;
+    const int c = threadIdx.x, h = blockIdx.x % a.H, t0 = tile % nt * kPrepTokens, b = tile / nt;
     const int P = a.H * kKdaK, ch = h * kKdaK + c, kc = a.kc, lane = c & 63, wave = c >> 6;
     const int64_t row0 = static_cast<int64_t>(b) * a.T;
     // input i of the padded sequence: the window, then the tokens
@@ -380,7 +382,7 @@ __global__ __launch_bounds__(128) void kda_prep_kernel(KdaPrepArgs a) {
         }
 #pragma unroll
         for (int i = 0; i < kPrepTokens; ++i) y[m][i] = y[m][i] / (1.0f + expf(-y[m][i]));
-        if (blockIdx.y == 0)
+        if (t0 == 0)
             for (int j = 0; j < kc - 1; ++j) a.win_out[m][(static_cast<int64_t>(b) * (kc - 1) + j) * P + ch] = xp(m, a.T + j);
     }
 #pragma unroll
@@ -593,13 +595,16 @@ extern "C" int k3_kda_prefill_inputs(const float *q_raw, const float *k_raw, con
                                      float *q, float *k, float *v, float *g, float *beta, int64_t B, int64_t T,
                                      int64_t heads, int64_t head_dim, int64_t conv_size, float gate_lower_bound,
                                      void *stream) {
-    if (!q_raw || !k_raw || !v_raw || !fb || !b_raw || !q_conv || !k_conv || !v_conv || !q_win_out || !k_win_out ||
-        !v_win_out || !A_log || !dt_bias || !q || !k || !v || !g || !beta || (!q_win != !k_win) || (!q_win != !v_win))
+    const bool windows = conv_size != 1;    // (one tap keeps no inputs: the windows are empty)
+    if (!q_raw || !k_raw || !v_raw || !fb || !b_raw || !q_conv || !k_conv || !v_conv ||
+        (windows && (!q_win_out || !k_win_out || !v_win_out)) || !A_log || !dt_bias || !q || !k || !v || !g || !beta || (!q_win != !k_win) || (!q_win != !v_win))
         return set_error(K3_ERR_NULL, "kda prefill inputs: null pointer");
     if (head_dim != kKdaK) return set_error(K3_ERR_SHAPE, "kda prefill inputs: head_dim=%lld; the kernels take %d",
                                             (long long)head_dim, kKdaK);
-    if (conv_size < 2 || conv_size > 8) return set_error(K3_ERR_SHAPE, "kda prefill inputs: conv_size=%lld", (long long)conv_size);
-    if (B <= 0 || T <= 0 || heads <= 0 || B > 65535 || T > 8 * 65535 || heads > (1 << 20))
+    if (conv_size < 1 || conv_size > (1 << 16))
+        return set_error(K3_ERR_SHAPE, "kda prefill inputs: conv_size=%lld", (long long)conv_size);
+    if (B <= 0 || T <= 0 || heads <= 0 || B > (1 << 24) || T > (1 << 24) || heads > (1 << 20) ||
+        B * cdiv(T, kPrepTokens) >= (1ll << 25) || B * cdiv(T, kPrepTokens) * heads >= (1ll << 25))
         return set_error(K3_ERR_SHAPE, "kda prefill inputs: B=%lld, T=%lld, heads=%lld", (long long)B, (long long)T,
                          (long long)heads);
     KdaPrepArgs a{};
@@ -610,8 +615,7 @@ extern "C" int k3_kda_prefill_inputs(const float *q_raw, const float *k_raw, con
     a.A_log = A_log, a.dt_bias = dt_bias, a.lower = gate_lower_bound;
     a.q = q, a.k = k, a.v = v, a.g = g, a.beta = beta;
     a.B = static_cast<int>(B), a.T = static_cast<int>(T), a.H = static_cast<int>(heads), a.kc = static_cast<int>(conv_size);
-    const dim3 grid(static_cast<unsigned>(heads), static_cast<unsigned>(cdiv(T, kPrepTokens)), static_cast<unsigned>(B));
-    kda_prep_kernel<<<grid, 128, 0, static_cast<hipStream_t>(stream)>>>(a);
+    kda_prep_kernel<<<dim3(static_cast<unsigned>(heads * cdiv(T, kPrepTokens) * B)), 128, 0, static_cast<hipStream_t>(stream)>>>(a);
     return check_hip(hipGetLastError(), "kda prefill inputs launch");
 }
 

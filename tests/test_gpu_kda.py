@@ -255,3 +255,55 @@ def test_kda_windows_kept_on_the_host(Tn):
     want = attn(x, conv=tuple(c.to(DEV) for c in wins))
     assert torch.equal(out, want[0]) and torch.equal(S, want[1])
     assert all(torch.equal(a, b) for a, b in zip(conv, want[2]))
+
+
+@pytest.mark.parametrize("conv", [1, 9, 12])
+def test_kda_many_tokens_of_other_convolution_sizes(conv):
+    """One tap (no windows) and more than eight, against the fp64 layer; then split in two with the
+    state and the windows carried."""
+    from k3hip.kda import KDAAttention
+    cfg = KdaCfg(256, 2)
+    cfg.kda_conv_size = conv
+    rng = np.random.default_rng(conv)
+    w = okda.random_kda_weights(rng, cfg, 0.05)
+    for n in ("q_proj", "k_proj", "v_proj", "g_proj", "o_proj", "f_a_proj", "f_b_proj", "b_proj"):
+        w[n + ".weight"] = om.bf16_round(w[n + ".weight"])
+    attn = KDAAttention(cfg, {n: torch.from_numpy(a).to(DEV) for n, a in w.items()})
+    x = om.bf16_round(rng.standard_normal((2, 19, 256)).astype(np.float32))
+    xd = torch.from_numpy(x).to(DEV).to(torch.bfloat16)
+    out, S, cv = attn(xd)
+    want, want_S, want_cv = okda.kda_layer(cfg, w, x)
+    assert om.normwise_rel(out.cpu().numpy(), want) <= 2e-5 and om.normwise_rel(S.cpu().numpy(), want_S) <= 2e-5
+    assert [tuple(c.shape) for c in cv] == [(2, conv - 1, 256)] * 3
+    if conv > 1:
+        assert max(om.normwise_rel(a.cpu().numpy(), b) for a, b in zip(cv, want_cv)) <= 2e-6
+    o1, S1, c1 = attn(xd[:, :10])
+    o2, S2, _ = attn(xd[:, 10:], S1, c1)
+    assert om.normwise_rel(torch.cat([o1, o2], 1).cpu().numpy(), want) <= 2e-5
+    assert om.normwise_rel(S2.cpu().numpy(), want_S) <= 2e-5
+
+
+def test_kda_more_sequences_than_a_grid_dimension():
+    """70,000 sequences of two tokens: each is the same sequence's result in a small batch."""
+    cfg, w, attn, rng = _layer(43, 64, 1, scale=0.05)
+    B = 70000
+    x = torch.randn(B, 2, 64, device=DEV, generator=torch.Generator(device=DEV).manual_seed(3)).to(torch.bfloat16)
+    out, S, cv = attn(x)
+    for b in (0, 65535, 65536, B - 3):
+        o, s, c = attn(x[b:b + 3])
+        for got, one in ((out, o), (S, s), (cv[0], c[0]), (cv[2], c[2])):
+            assert float((got[b:b + 3] - one).abs().max()) <= 2e-5 * float(one.abs().max())
+
+
+def test_kda_more_tokens_than_a_grid_dimension():
+    """A sequence of 8 x 65535 tokens and some ends in the state and windows of the same sequence in
+    two calls."""
+    cfg, w, attn, rng = _layer(44, 64, 1, scale=0.05)
+    T = 8 * 65535 + 21
+    x = torch.randn(1, T, 64, device=DEV, generator=torch.Generator(device=DEV).manual_seed(4)).to(torch.bfloat16)
+    out, S, cv = attn(x)
+    h = T // 2 + 3
+    o1, S1, c1 = attn(x[:, :h])
+    o2, S2, c2 = attn(x[:, h:], S1, c1)
+    for got, one in ((out[:, h:], o2), (S, S2), (cv[1], c2[1])):
+        assert float((got - one).abs().max()) <= 1e-4 * float(one.abs().max())
