@@ -250,7 +250,8 @@ static bool gemv_sooner(int64_t M, int64_t N, int64_t K, bool x_bf16) {
 }
 
 bool mxfp4_gemm_takes(int64_t M, int64_t N, int64_t K, bool x_bf16) {
-    return M > 4 && !gemv_sooner(M, N, K, x_bf16) && M <= 64 * 65535 && N < (1ll << 31) && 16 * (K / 32) + 32 <= kMaxScale && K * 64 * 4 < (1ll << 31);
+    return M > 4 && !gemv_sooner(M, N, K, x_bf16) && M <= 64 * 65535 && N <= (1ll << 26) &&   // (2^32 threads a grid dimension)
+           16 * (K / 32) + 32 <= kMaxScale && K * 64 * 4 < (1ll << 31);
 }
 
 int mxfp4_gemm_launch(const GemvArgs &a, hipStream_t st) {

@@ -40,9 +40,13 @@ def _mm_bf16_f32(a2: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return torch.mm(a2, w.t(), out_dtype=torch.float32)
 
 
+# what k3_dense takes: rows of a and of one weight matrix, and their width and pitch
+MAX_ROWS, MAX_WIDTH = 1 << 24, 1 << 20
+
+
 def _rows_ok(w: torch.Tensor) -> bool:
     return (w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() and w.data_ptr() % 16 == 0
-            and w.shape[1] % 8 == 0 and w.shape[0] > 0)
+            and w.shape[1] % 8 == 0 and w.shape[1] <= MAX_WIDTH and 0 < w.shape[0] <= MAX_ROWS)
 
 
 def weights_ok(*ws: torch.Tensor) -> bool:
@@ -55,6 +59,8 @@ def dense_ok(a: torch.Tensor, *ws: torch.Tensor) -> bool:
     if not a.is_cuda or a.dtype not in (torch.float32, torch.bfloat16) or T.tracked(a, *ws):
         return False
     K, dev = a.shape[-1], a.get_device()
+    if a.numel() > MAX_ROWS * K:
+        return False
     for w in ws:
         if not _rows_ok(w) or w.shape[1] != K or w.get_device() != dev:
             return False
@@ -70,7 +76,8 @@ def dense(a: torch.Tensor, ws, add: torch.Tensor | None = None) -> list[torch.Te
             raise ValueError(f"add must be float32 [{M}, N] beside one weight [N, {K}]; got {add.dtype} {tuple(add.shape)}")
         T.require_device(a, add)
         add = T.contiguous_aligned(add)
-    if a.stride(1) != 1 or (a.stride(0) * a.element_size()) % 16 or a.stride(0) < K or a.data_ptr() % 16:
+    if (a.stride(1) != 1 or (a.stride(0) * a.element_size()) % 16 or not K <= a.stride(0) <= MAX_WIDTH
+            or a.data_ptr() % 16):
         a = T.contiguous_aligned(a)
     n = len(ws)
     outs = [torch.empty((M, w.shape[0]), dtype=torch.float32, device=a.device) for w in ws]

@@ -196,7 +196,7 @@ def _rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
 def _rmsnorm_rows(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
     """_rmsnorm of the rows of an fp32 [M, K] device tensor in one launch."""
     M, K = x.shape
-    if (tuple(w.shape) != (K,) or K % 4 or x.stride(1) != 1 or x.stride(0) % 4 or x.data_ptr() % 16 or M == 0
+    if (tuple(w.shape) != (K,) or M > _blas.MAX_ROWS or K % 4 or x.stride(1) != 1 or x.stride(0) % 4 or x.data_ptr() % 16 or M == 0
             or T.tracked(x, w)):
         return _rmsnorm(x, w, eps)   # (which refuses or broadcasts a w of another shape)
     w = T.contiguous_aligned(w.to(torch.float32))
@@ -329,6 +329,7 @@ class MLAAttention:
         if T.tracked(q, lat, rot, self.kv_b):
             return False
         return (B == 1 and Tn > 1 and lat.shape[:2] == rot.shape[:2] and lat.shape[0] == 1
+                and lat.shape[1] <= 1 << 24 and c.num_attention_heads <= 4096 and lat.stride(1) <= 1 << 20
                 and q.is_cuda and q.dtype == torch.float32 and lat.dtype == rot.dtype
                 and lat.dtype in (torch.bfloat16, torch.float32) and self.kv_b.dtype == torch.bfloat16
                 and self.kv_b.is_contiguous() and self.kv_b.data_ptr() % 16 == 0

@@ -419,7 +419,7 @@ def _rmsnorm32(y: torch.Tensor, w32: torch.Tensor, eps: float) -> torch.Tensor:
 def _rmsnorm_rows(y: torch.Tensor, w32: torch.Tensor, eps: float) -> torch.Tensor:
     """_rmsnorm32 of the contiguous rows of an fp32 [M, K] device tensor in one launch."""
     M, K = y.shape
-    if (M == 0 or K % 4 or not y.is_contiguous() or y.data_ptr() % 16 or w32.data_ptr() % 16 or y.dtype != torch.float32
+    if (M == 0 or M > _blas.MAX_ROWS or K % 4 or not y.is_contiguous() or y.data_ptr() % 16 or w32.data_ptr() % 16 or y.dtype != torch.float32
             or tuple(w32.shape) != (K,) or T.tracked(y, w32)):
         return _rmsnorm32(y, w32, eps)
     T.require_device(y, w32)

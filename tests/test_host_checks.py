@@ -265,3 +265,35 @@ def test_kda_without_tokens_returns_the_state_and_windows(monkeypatch, B, T):
     out, state, conv = kda(x, S, wins)
     assert state is S and all(torch.equal(a, b) and a.dtype == torch.float32 for a, b in zip(conv, wins))
     assert not launches
+
+
+def test_sizes_beyond_a_launch_stay_where_they_ran(monkeypatch):
+    """More rows, wider rows or wider pitches than the launches take go the way they went before."""
+    from k3hip import _blas, _lib, mla
+    z = lambda *s, dt=torch.float32: _dev(torch.zeros((1,) * len(s), dtype=dt).expand(*s))  # noqa: E731
+    w = _dev(torch.zeros(16, 8, dtype=BF16))
+    assert _blas.dense_ok(z(1 << 24, 8), w) and not _blas.dense_ok(z((1 << 24) + 1, 8), w)
+    wide = _dev(torch.zeros(1, (1 << 20) + 8, dtype=BF16))
+    assert not _blas.weights_ok(wide) and not _blas.dense_ok(z(2, (1 << 20) + 8), wide)
+    attn = _mla_stub()
+    for heads, Tk, ok in ((4, 1 << 24, True), (4, (1 << 24) + 1, False), (4097, 64, False)):
+        attn.cfg.num_attention_heads = heads
+        assert attn._expanded_ok(z(1, 20, heads, 192), _rows(1, Tk, 512), _rows(1, Tk, 64)) == ok
+    launches = _lib.lib().k3_mxfp4_matvec_launches
+    assert launches(5, 1 << 26, 32, 0) == 1 and launches(5, 1 << 28, 32, 0) == 2
+    launched = []
+    _no_device(monkeypatch, launched)
+    x = z((1 << 24) + 1, 4)._t
+    monkeypatch.setattr(mla, "_rmsnorm", lambda *a: "tensor operations")
+    assert mla._rmsnorm_rows(x, torch.ones(4), 1e-5) == "tensor operations" and not launched
+
+
+def test_dense_copies_rows_of_a_pitch_it_does_not_take(monkeypatch):
+    from k3hip import _blas, _lib
+    _no_device(monkeypatch, [])
+    seen = {}
+    monkeypatch.setattr(_lib, "lib", lambda: SimpleNamespace(k3_dense_workspace_size=lambda *a: 0))
+    monkeypatch.setattr(_lib, "call", lambda name, *a: seen.update(ptr=a[0], lda=a[2]))
+    a = torch.zeros(3, (1 << 20) + 64)[:, :32]
+    _blas.dense(a, [torch.zeros(16, 32, dtype=BF16)])
+    assert seen["lda"] == 32 and seen["ptr"] != a.data_ptr()
