@@ -649,7 +649,9 @@ def moe_grouped_ffn(x: torch.Tensor, expert_indices: torch.Tensor, expert_weight
     if n_tok == 0:
         return out
     nbytes = _lib.size("k3_moe_grouped_workspace_size", n_tok, k, E, H, intermediate)
-    ws = _workspace.get(x.device, nbytes, "moe_grouped")
+    # the call's own: calls of several threads on one stream, and a captured graph whose call is
+    # followed by a larger one, must not meet in a kept buffer
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
     _lib.call("k3_moe_grouped_ffn", T.ptr(x), T.dtype_code(x.dtype), T.ptr(idx), T.ptr(w), T.ptr(table),
               T.ptr(out), T.dtype_code(out_dtype), n_tok, H, intermediate, E, k, _act_code(act), float(beta),
               float(linear_beta or 0.0), T.ptr(ws), ws.numel(), T.stream(x))

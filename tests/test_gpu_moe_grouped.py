@@ -249,3 +249,71 @@ def test_grouped_tile_edges(H, I, off, xdt):
     print(f"H={H} I={I} scale offset {off} {xdt}: {rel:.2e}")
     assert rel <= 2e-5
     assert torch.equal(got, moe_grouped_ffn(x, ids, w, table, I, "situ", 2.0, 3.0))
+
+
+def _prompts(E, H, I, k, sizes):
+    from k3hip.moe import moe_grouped_ffn
+    rng = np.random.default_rng(31)
+    _, ex_dev = make_experts(rng, 4, H, I)
+    table = table_of(ex_dev, E)
+    calls = []
+    for T in sizes:
+        idx, w = distinct_routing(rng, T, E, k)
+        args = [torch.from_numpy(om.bf16_round(rng.standard_normal((T, H)).astype(np.float32))).to(DEV).to(torch.bfloat16),
+                torch.from_numpy(idx).to(DEV), torch.from_numpy(w).to(DEV), table, I]
+        calls.append(lambda a=args: moe_grouped_ffn(*a, validate=False))
+    return calls, (ex_dev, table)
+
+
+def test_grouped_replay_after_larger_calls():
+    """A captured prompt keeps its own scratch: later, larger prompts on its stream and whatever takes
+    the memory they free leave its replays as the eager result."""
+    (small, big, bigger), keep = _prompts(16, 256, 128, 4, (20, 150, 700))
+    want = small().clone()
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        small()
+    torch.cuda.current_stream().wait_stream(stream)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        out = small()
+    for call in (big, bigger, small):
+        with torch.cuda.stream(stream):
+            call()
+            junk = [torch.full((n,), 0x7f, dtype=torch.uint8, device=DEV) for n in (1 << 17, 1 << 19, 1 << 21, 1 << 23)]
+        torch.cuda.synchronize()
+        del junk
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(small(), want)
+
+
+def test_grouped_threads_on_one_stream():
+    """Two threads run prompts of different sizes on one stream, their launches in any order."""
+    import threading
+    calls, keep = _prompts(16, 256, 128, 4, (40, 150))
+    want = [c().clone() for c in calls]
+    torch.cuda.synchronize()
+    stream, got, errors = torch.cuda.Stream(), [[], []], []
+    start = threading.Barrier(2)
+
+    def work(i):
+        try:
+            start.wait()
+            with torch.cuda.stream(stream):
+                for _ in range(40):
+                    got[i].append(calls[i]())
+        except Exception as e:  # reported below
+            errors.append(repr(e))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(timeout=60)
+    stream.synchronize()
+    assert not errors and not any(t.is_alive() for t in threads)
+    for i in range(2):
+        assert len(got[i]) == 40 and all(torch.equal(y, want[i]) for y in got[i])

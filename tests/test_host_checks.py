@@ -297,3 +297,16 @@ def test_dense_copies_rows_of_a_pitch_it_does_not_take(monkeypatch):
     a = torch.zeros(3, (1 << 20) + 64)[:, :32]
     _blas.dense(a, [torch.zeros(16, 32, dtype=BF16)])
     assert seen["lda"] == 32 and seen["ptr"] != a.data_ptr()
+
+
+def test_grouped_prompts_do_not_share_scratch(monkeypatch):
+    """Every prompt through the grouped experts brings scratch of its own (a captured graph and a later
+    call, or two threads on one stream, would meet in a kept buffer)."""
+    from k3hip import _lib, _workspace, moe
+    seen = []
+    _no_device(monkeypatch, [])
+    monkeypatch.setattr(_lib, "call", lambda name, *a: seen.append((name, a[-3])))
+    monkeypatch.setattr(_workspace, "get", lambda *a: pytest.fail("a kept buffer"))
+    x, idx, w = torch.zeros(9, 64), torch.zeros(9, 2, dtype=torch.int64), torch.zeros(9, 2)
+    moe.moe_grouped_ffn(x, idx, w, torch.zeros(4, 6, dtype=torch.int64), 64, validate=False)
+    assert [n for n, _ in seen] == ["k3_moe_grouped_ffn"] and seen[0][1]
