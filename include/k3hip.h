@@ -48,6 +48,10 @@ extern "C" {
 const char *k3_last_error(void);
 const char *k3_version(void);
 
+/* A number that differs between captures if the stream is being captured into a graph, else 0.  A
+ * caller that keeps workspaces gives each capture one of its own. */
+int64_t k3_stream_capture_id(void *stream);
+
 /* Bit-exact dequantisation to fp32 (out_dtype K3_F32) or bf16 (K3_BF16), [N, K].
  * Replaces decode_mxfp4_mlx (air_llm/models/kimi_k3/mxfp4.py:68-81) with the values of
  * k3ref.weights.decode_mxfp4 (k3ref/weights.py:29-37) for every code and scale byte. */

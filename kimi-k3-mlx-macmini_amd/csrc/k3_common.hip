@@ -26,3 +26,13 @@ int check_hip(hipError_t e, const char *what) {
 extern "C" const char *k3_last_error(void) { return k3::g_err; }
 
 extern "C" const char *k3_version(void) { return "k3hip 0.1 gfx950"; }
+
+extern "C" int64_t k3_stream_capture_id(void *stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(static_cast<hipStream_t>(stream), &status, &id) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    return status == hipStreamCaptureStatusNone ? 0 : static_cast<int64_t>(id) + 1;
+}

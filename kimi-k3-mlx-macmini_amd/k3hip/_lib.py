@@ -34,6 +34,7 @@ SIGNATURES: dict[str, list] = {
     "k3_mxfp4_decode": [_P, _P, _P, _I32, _I64, _I64, _P],
     "k3_scale_minmax": [_P, _I64, _P, _P],
     "k3_mxfp4_matvec": [_P, _I32, _P, _P, _P, _I32, _I64, _I64, _I64, _P],
+    "k3_stream_capture_id": [_P],
     "k3_mxfp4_matvec_launches": [_I64, _I64, _I64, _I32],
     "k3_expert_ffn_workspace_size": [_I64],
     "k3_expert_ffn": [_P, _I32, _P, _P, _P, _P, _P, _P, _P, _I32, _I64, _I64, _I32, _F32, _F32,
@@ -95,6 +96,7 @@ _RESTYPE = {"k3_last_error": ctypes.c_char_p, "k3_version": ctypes.c_char_p,
             "k3_mla_step_workspace_size": ctypes.c_int64,
             "k3_kda_step_workspace_size": ctypes.c_int64,
             "k3_mxfp4_matvec_launches": ctypes.c_int64,
+            "k3_stream_capture_id": ctypes.c_int64,
             "k3_dense_workspace_size": ctypes.c_int64,
             "k3_mla_prefill_workspace_size": ctypes.c_int64,
             "k3_moe_grouped_workspace_size": ctypes.c_int64,

@@ -283,3 +283,38 @@ def test_route_only_with_garbage_counter(router):
         assert np.allclose(got_w, wts[0], rtol=1e-5, atol=1e-7)
         assert np.allclose(got_raw, raw[0], rtol=1e-4, atol=1e-7)
         assert int(ws[:4].view(torch.int32).item()) == 0
+
+
+def test_workspaces_of_graphs_that_were_captured_cold_or_outgrown():
+    """Two graphs captured with no eager call on their stream before (one token each, and two tokens):
+    an eager call there, then the second graph, then the first, then both again after larger calls and
+    after whatever takes freed memory, all give the eager results."""
+    from k3hip.moe import RoutedMoE
+    cfg, w, source, *_ = make_layer(7, 1024, 256, 32, 4, 256)
+    moe = RoutedMoE(cfg, 0, w, source)
+    g = torch.Generator(device=DEV).manual_seed(8)
+    xs = [torch.randn(n, 1024, device=DEV, generator=g).to(torch.bfloat16) for n in (1, 2, 8)]
+    want = [moe(x).clone() for x in xs]
+    stream = torch.cuda.Stream()
+    graphs, outs = [], []
+    torch.cuda.synchronize()
+    for order in ((0, 1), (1, 0)):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            out = {i: moe(xs[i]) for i in order}
+        graphs.append(graph)
+        outs.append(out)
+    with torch.cuda.stream(stream):
+        assert torch.equal(moe(xs[0]), want[0])
+    for turn in range(3):
+        for graph, out in list(zip(graphs, outs))[::-1 if turn == 0 else 1]:
+            for o in out.values():
+                o.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert all(torch.equal(o, want[i]) for i, o in out.items())
+        with torch.cuda.stream(stream):
+            assert torch.equal(moe(xs[2]), want[2]) and torch.equal(moe(xs[1]), want[1])
+            junk = [torch.full((n,), 0x7f, dtype=torch.uint8, device=DEV) for n in (1 << 14, 1 << 17, 1 << 20, 1 << 22)]
+        torch.cuda.synchronize()
+        del junk

@@ -310,3 +310,42 @@ def test_grouped_prompts_do_not_share_scratch(monkeypatch):
     x, idx, w = torch.zeros(9, 64), torch.zeros(9, 2, dtype=torch.int64), torch.zeros(9, 2)
     moe.moe_grouped_ffn(x, idx, w, torch.zeros(4, 6, dtype=torch.int64), 64, validate=False)
     assert [n for n, _ in seen] == ["k3_moe_grouped_ffn"] and seen[0][1]
+
+
+@pytest.fixture
+def workspaces(monkeypatch):
+    """k3hip._workspace on the host: one stream, and a capture that the test opens and closes."""
+    from k3hip import _lib, _workspace
+    from k3hip import _torch as T
+    state = SimpleNamespace(capture=0, get=lambda n, tag="t": _workspace.get(torch.device("cpu"), n, tag), mod=_workspace)
+    monkeypatch.setattr(T, "stream_of", lambda device: 7)
+    monkeypatch.setattr(_lib, "lib", lambda: SimpleNamespace(k3_stream_capture_id=lambda stream: state.capture))
+    for name in ("_cache", "_captured", "_outgrown"):
+        monkeypatch.setattr(_workspace, name, type(getattr(_workspace, name, {}))())
+    return state
+
+
+def test_an_outgrown_workspace_stays(workspaces):
+    """A captured graph may go on writing it.  All outgrown ones together are smaller than the one in use."""
+    import weakref
+    sizes = [5000, 9000, 9001, 30000, 200000]
+    seen = [weakref.ref(workspaces.get(n)) for n in sizes]
+    assert all(r() is not None for r in seen)
+    kept = workspaces.mod._outgrown
+    assert sum(b.numel() for b in kept) < workspaces.get(1).numel() and not workspaces.get(1).any()
+    del kept
+    workspaces.mod.clear()
+    assert all(r() is None for r in seen)
+
+
+def test_a_workspace_made_in_a_capture_is_that_captures_own(workspaces):
+    workspaces.capture = 3
+    a = workspaces.get(5000)
+    assert workspaces.get(4000).data_ptr() == a.data_ptr() and not a[:4096].any()
+    workspaces.capture = 4                  # another graph, which may replay before the first ever does
+    b = workspaces.get(5000)
+    workspaces.capture = 0                  # an eager call, the same
+    c = workspaces.get(5000)
+    assert len({a.data_ptr(), b.data_ptr(), c.data_ptr()}) == 3 and not c.any()
+    workspaces.capture = 5                  # a buffer in use outside is taken by captures too, as it is
+    assert workspaces.get(5000).data_ptr() == c.data_ptr()
