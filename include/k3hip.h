@@ -79,7 +79,7 @@ int64_t k3_mxfp4_matvec_launches(int64_t M, int64_t N, int64_t K, int x_dtype);
 
 /* Workspace bytes k3_expert_ffn needs for intermediate size I (the fp32 act vector passed
  * between its two launches).  Needs no initialisation.  Calls that share a workspace must
- * not overlap (calls on one stream never do). */
+ * not overlap (those that one thread makes on one stream never do). */
 int64_t k3_expert_ffn_workspace_size(int64_t I);
 
 /* One routed expert at batch 1, two stream-ordered launches (gate/up + act, then the down
@@ -113,7 +113,7 @@ int k3_expert_ffn_noalloc(const void *x, int x_dtype, const void *gate_packed, c
  * shared expert).  Its first 4096 bytes hold arrival counters (finished router blocks,
  * finished blocks of each range of output rows; at that place for every shape): zero-fill
  * them before the first call; every call returns them to zero.  The rest is rewritten by every call.  Calls that share a workspace must not
- * overlap (calls on one stream never do). */
+ * overlap (those that one thread makes on one stream never do). */
 int64_t k3_moe_layer_workspace_size(int64_t H, int64_t I, int64_t shared_I, int64_t n_experts,
                                     int64_t top_k);
 

@@ -3,7 +3,9 @@
 The C-ABI allocates nothing.  Intermediate records (the expert's act vector, router
 records, split-T partials, grouping lists) live in a workspace the caller passes in.
 Concurrent launches must not share a workspace, so workspaces are kept per (device,
-stream, user).  (The prompt paths allocate theirs per call instead.)
+stream, user, thread): the launches of two threads' calls may interleave on one stream.  (A
+later thread may get an ended one's number, and with it its buffers; on one stream that is
+in order.  The prompt paths allocate their scratch per call instead.)
 
 A captured graph goes on using the buffer its capture was given.  So a buffer that a later call
 outgrows is kept beside its successor, which is at least twice as large, so all of one key's outgrown
@@ -30,9 +32,9 @@ _captured: dict[tuple, tuple[int, torch.Tensor]] = {}    # (capture, its buffer)
 
 
 def get(device: torch.device, nbytes: int, tag: str = "") -> torch.Tensor:
-    """A uint8 device buffer of at least nbytes for the current stream, zero when made (inside a
-    capture: its first COUNTERS bytes)."""
-    key = (device.index, T.stream_of(device), tag)
+    """A uint8 device buffer of at least nbytes for the current stream and thread, zero when made
+    (inside a capture: its first COUNTERS bytes)."""
+    key = (device.index, T.stream_of(device), tag, threading.get_ident())
     buf = _cache.get(key)
     if buf is None or buf.numel() < nbytes:
         buf = _make(device, nbytes, key)

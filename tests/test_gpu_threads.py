@@ -132,3 +132,46 @@ def test_moe_layer_from_threads_matches_one_thread():
     assert not errors, errors
     for t in range(3):
         assert len(results[t]) == rounds and all(torch.equal(y, want[t]) for y in results[t])
+
+
+def test_threads_on_one_stream_match_one_thread():
+    """Three threads decode through one expert and one RoutedMoE (one token, and three) on one shared
+    stream: each call is several launches, and theirs interleave; every output and every router
+    record equals the single-threaded one."""
+    from k3hip.moe import RoutedMoE, expert_ffn_fused
+    from test_gpu_moe_layer import make_layer
+    cfg, w, source, *_ = make_layer(9, 1024, 256, 64, 8, 512)
+    moe = RoutedMoE(cfg, 0, w, source)
+    expert = tuple(source(0, 3, n) for n in ("w1", "w3", "w2"))
+    g = torch.Generator(device=DEV).manual_seed(10)
+    xs = [torch.randn(4, 1024, device=DEV, generator=g).to(torch.bfloat16) for _ in range(3)]
+
+    def calls(x):
+        y, r = moe(x[:1], return_router=True)
+        return [expert_ffn_fused(x[:1], *expert), y, r.expert_indices, r.expert_weights, moe(x[1:])]
+
+    want = [calls(x) for x in xs]
+    torch.cuda.synchronize()
+    stream, results, errors = torch.cuda.Stream(), {}, []
+    start = threading.Barrier(3)
+
+    def worker(t):
+        try:
+            start.wait()
+            with torch.cuda.stream(stream):
+                results[t] = [calls(xs[t]) for _ in range(30)]
+        except Exception as e:  # reported below with the thread's index
+            errors.append(f"thread {t}: {e!r}")
+
+    threads = [threading.Thread(target=worker, args=(t,)) for t in range(3)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join(timeout=120)
+    stream.synchronize()
+    assert not any(th.is_alive() for th in threads), "a thread did not finish"
+    assert not errors, errors
+    for t in range(3):
+        assert len(results[t]) == 30
+        for got in results[t]:
+            assert all(torch.equal(a, b) for a, b in zip(got, want[t]))

@@ -349,3 +349,20 @@ def test_a_workspace_made_in_a_capture_is_that_captures_own(workspaces):
     assert len({a.data_ptr(), b.data_ptr(), c.data_ptr()}) == 3 and not c.any()
     workspaces.capture = 5                  # a buffer in use outside is taken by captures too, as it is
     assert workspaces.get(5000).data_ptr() == c.data_ptr()
+
+
+def test_threads_on_one_stream_have_workspaces_of_their_own(workspaces):
+    import threading
+    got, both = {}, threading.Barrier(2)
+
+    def work(i):
+        got[i] = workspaces.get(5000)
+        both.wait()                        # both threads are alive: their numbers differ
+        assert workspaces.get(5000).data_ptr() == got[i].data_ptr()
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert got[0].data_ptr() != got[1].data_ptr()
