@@ -21,9 +21,13 @@ def ptr(t: torch.Tensor | None) -> int:
     return 0 if t is None else t.data_ptr()
 
 
+def _stream_handle(device_index: int) -> int:
+    return torch.cuda.current_stream(device_index).cuda_stream
+
+
 # The raw handle of the current stream, without the Stream object that
-# torch.cuda.current_stream builds around it (about 1 us per call).
-_raw_stream = torch._C._cuda_getCurrentRawStream
+# torch.cuda.current_stream builds around it (about 1 us per call) where torch offers it.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", _stream_handle)
 
 
 def stream(t: torch.Tensor) -> int:

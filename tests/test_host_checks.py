@@ -366,3 +366,16 @@ def test_threads_on_one_stream_have_workspaces_of_their_own(workspaces):
     for t in threads:
         t.join()
     assert got[0].data_ptr() != got[1].data_ptr()
+
+
+def test_import_without_the_raw_stream_getter(monkeypatch):
+    """A torch that lacks it imports the package and takes the handle from its Stream objects."""
+    import importlib.util
+    from k3hip import _torch as T
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: SimpleNamespace(cuda_stream=1000 + device))
+    spec = importlib.util.spec_from_file_location("k3hip._torch_again", T.__file__)
+    again = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(again)
+    assert again.stream_of(torch.device("cuda", 3)) == 1003
+    assert again.stream(SimpleNamespace(get_device=lambda: 2)) == 1002
