@@ -263,7 +263,7 @@ __global__ __launch_bounds__(kThreads, 2) void dense_kernel(DenseArgs a) {
                 for (int j = 0; j < NT; ++j) {
                     uint32_t t[3][4];
 #pragma unroll
-                    for (int x = 0; x < 4; ++x) split3(acc[j][i][x], t[0][x], t[1][x], t[2][x]);
+                    for (int x = 0; x < 4; ++x) split3_near(acc[j][i][x], t[0][x], t[1][x], t[2][x]);
 #pragma unroll
                     for (int x = 0; x < 3; ++x) {
                         uint16_t *dst = wn ? a.vt + mla_v_index(ntile, a.tpad, x, 16 * j + r16, mt0) + q * 8

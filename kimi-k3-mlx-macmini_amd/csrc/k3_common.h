@@ -66,6 +66,20 @@ __device__ __forceinline__ void split3(float v, uint32_t &t1, uint32_t &t2, uint
     t3 = __float_as_uint(r - __uint_as_float(t2));
     if ((u & 0x7fffffffu) > 0x7f800000u) t1 |= 0x00400000u;  // a NaN whose payload is cut stays one
 }
+// The same with the first two terms rounded to nearest (cut where that would overflow), for
+// products of two split values that leave the small term products out: a rounded term is at most
+// half a unit of the one before it and has either sign, so what is left out is small and
+// does not lean to one side.  SMALL: v is known to be far from overflow (or NaN, which the
+// remainders carry).
+template <bool SMALL = false>
+__device__ __forceinline__ void split3_near(float v, uint32_t &t1, uint32_t &t2, uint32_t &t3) {
+    const uint32_t u = __float_as_uint(v), a = u & 0x7fffffffu;
+    t1 = (SMALL || a < 0x7f7f8000u ? u + 0x8000u : u) & 0xffff0000u;
+    const float r = !SMALL && a >= 0x7f800000u ? 0.f : v - __uint_as_float(t1);
+    t2 = (__float_as_uint(r) + 0x8000u) & 0xffff0000u;
+    t3 = __float_as_uint(r - __uint_as_float(t2));
+    if (!SMALL && a > 0x7f800000u) t1 |= 0x00400000u;
+}
 __device__ __forceinline__ uint32_t hi16x2(uint32_t a, uint32_t b) {  // (a >> 16) | (b & 0xffff0000)
     return __builtin_amdgcn_perm(b, a, 0x07060302u);
 }

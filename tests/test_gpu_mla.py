@@ -479,8 +479,8 @@ def test_mla_fused_decode_step_other_shapes(hidden, heads, q_lora, gate):
 def test_mla_many_tokens_match_fp64(T, past, heads, cache, gate):
     """k3_mla_prefill (query tiles of 128, 16 per wave, steps of 32 cached tokens, both cache
     dtypes, past lengths that leave part steps) against the masked form in fp64 over the same
-    cache rows.  Six products of three-term operands leave 2^-24 of a product, so the error is
-    that of fp32 sums of 192 and 128 (context of up to 4217) products: 1e-5 normwise."""
+    cache rows.  The products of three-term operands that are left out are below fp32's rounding of a
+    product (0.1 x 2^-24 rms, 2^-23 at most), so the error is that of fp32 sums of 192 and 128 (context of up to 4217) products: 1e-5 normwise."""
     from types import SimpleNamespace
     from k3hip.mla import MLAAttention, new_cache
     g = torch.Generator(device=DEV)
@@ -557,3 +557,46 @@ def test_mla_many_tokens_keep_a_weights_gradient(name):
         (out * up).sum().backward()
         grads.append(w[name].grad.double())
     assert float((grads[0] - grads[1]).norm()) <= 1e-5 * float(grads[1].norm()) and float(grads[1].norm()) > 0
+
+
+def _expanded_layer(heads, cache, kv_b):
+    from types import SimpleNamespace
+    from k3hip.mla import MLAAttention
+    hid, ql = 64, 64
+    z = lambda o, i: torch.zeros(o, i, device=DEV, dtype=torch.bfloat16)  # noqa: E731
+    w = {"q_a_proj.weight": z(ql, hid), "q_a_layernorm.weight": torch.ones(ql, device=DEV), "q_b_proj.weight": z(heads * 192, ql),
+         "kv_a_proj_with_mqa.weight": z(576, hid), "kv_a_layernorm.weight": torch.ones(512, device=DEV), "kv_b_proj.weight": kv_b,
+         "o_proj.weight": z(hid, heads * 128)}
+    cfg = SimpleNamespace(hidden_size=hid, num_attention_heads=heads, q_lora_rank=ql, kv_lora_rank=512, qk_nope_head_dim=128,
+                          qk_rope_head_dim=64, v_head_dim=128, q_head_dim=192, rms_norm_eps=1e-5, mla_use_output_gate=False,
+                          mla_cache_dtype=cache)
+    return MLAAttention(cfg, w)
+
+
+@pytest.mark.parametrize("where", ["rotary", "key"])
+def test_mla_many_tokens_scores_keep_their_products(where):
+    """A score of one product whose small term products matter most (both factors just below 1 + 2^-7:
+    cut into terms they would lose 6.9 to 7.8 x 2^-24 of it, always downwards) against a score that is that
+    product rounded to fp32.  A score of S carries two fp32 roundings (2^-24 S each) and the left-out
+    products; the log of the two probabilities' ratio is off by at most 6 x 2^-24 S and by less than
+    2 x 2^-24 S on average over 64 queries."""
+    T, A = 64, 2.0 ** 15
+    v0 = np.float32(1 + 2 ** -7 - 2 ** -23)
+    vt = np.float32(1 + 2 ** -7) - np.float32(2 ** -23) * np.arange(1, T + 1).astype(np.float32)
+    kv_b = torch.zeros(256, 512, device=DEV, dtype=torch.bfloat16)
+    kv_b[0, 1] = kv_b[1, 2] = kv_b[128, 0] = 1          # key columns 0, 1 and value column 0
+    attn = _expanded_layer(1, torch.float32, kv_b)
+    q = torch.zeros(1, T, 1, 192, device=DEV)
+    lat, rot = torch.zeros(1, T + 2, 512, device=DEV), torch.zeros(1, T + 2, 64, device=DEV)
+    lat[0, 0, 0], lat[0, 1, 0] = 1, -1
+    qc, keys = (q[..., 128:], rot) if where == "rotary" else (q, lat[..., 1:])
+    prod = (np.float32(A) * vt * v0).astype(np.float32)
+    qc[0, :, 0, 0], qc[0, :, 0, 1] = torch.from_numpy(np.float32(A) * vt).to(DEV), torch.from_numpy(prod).to(DEV)
+    keys[0, 0, 0], keys[0, 1, 1] = float(v0), 1
+    scale = 192 ** -0.5
+    assert attn._expanded_ok(q, lat, rot)
+    out = attn._expanded(q, lat[0], rot[0], scale, None)[0, :, 0].double().cpu().numpy()
+    exact = A * vt.astype(np.float64) * v0
+    off = (2 * np.arctanh(out) - scale * (exact - prod)) / (scale * exact * 2.0 ** -24)
+    print(f"{where}: off by {off.mean():.2f} on average, {abs(off).max():.2f} at most (2^-24 of the score)")
+    assert abs(off).max() <= 6 and abs(off.mean()) <= 2
