@@ -197,7 +197,8 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
         for (int h = 0; h < 2; ++h)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                float z = (hi[h][v] + lo[h][v]) * a.c;
+                // (an infinite score stands in hi alone: infinity times a zero or negative term is in lo)
+                float z = (__builtin_isinf(hi[h][v]) ? hi[h][v] : hi[h][v] + lo[h][v]) * a.c;
                 if (edge && 16 * h + 4 * q + v > seen) z = -INFINITY;
                 p[4 * h + v] = z;
             }
@@ -205,12 +206,14 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
         for (int i = 0; i < 8; ++i) mx = fmaxf(mx, p[i]);
         mx = fmaxf(mx, __shfl_xor(mx, 16));
         mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float al = __builtin_amdgcn_exp2f(m - mx);
+        // (every score so far -infinity: weights of zero, not of -infinity - -infinity)
+        const float ref = mx == -INFINITY ? 0.f : mx;
+        const float al = __builtin_amdgcn_exp2f(m - ref);
         m = mx;
         l *= al;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            p[i] = __builtin_amdgcn_exp2f(p[i] - mx);
+            p[i] = __builtin_amdgcn_exp2f(p[i] - ref);
             l += p[i];
         }
 #pragma unroll

@@ -600,3 +600,47 @@ def test_mla_many_tokens_scores_keep_their_products(where):
     off = (2 * np.arctanh(out) - scale * (exact - prod)) / (scale * exact * 2.0 ** -24)
     print(f"{where}: off by {off.mean():.2f} on average, {abs(off).max():.2f} at most (2^-24 of the score)")
     assert abs(off).max() <= 6 and abs(off.mean()) <= 2
+
+
+@pytest.mark.parametrize("cache", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("case", ["overflow", "far overflow", "infinite row", "large"])
+def test_mla_many_tokens_extreme_scores(case, cache):
+    """Scores past fp32's range and infinite ones, of some positions (the whole first steps among
+    them) or of one query: the weights are those of a softmax over the same fp32 scores, so a
+    position at -infinity has none, and a query with a score of +infinity is NaN alone."""
+    heads, T, past = 2, 20, 50
+    g = torch.Generator(device=DEV).manual_seed(12)
+    Tk = past + T
+    kv_b = (torch.randn(heads * 256, 512, device=DEV, generator=g) * 512 ** -0.5).to(torch.bfloat16)
+    attn = _expanded_layer(heads, cache, kv_b)
+    q = torch.randn(1, T, heads, 192, device=DEV, generator=g)
+    lat, rot = (torch.randn(1, Tk, n, device=DEV, generator=g).to(cache) for n in (512, 64))
+    q[..., 128:], q[..., 130] = 0, 1.25 if case != "large" else 3.0
+    first = 40                                             # more than one step of 32 positions
+    if case == "overflow":
+        q[..., 128], rot[:, :first, 0] = 1e20, -3e19       # -3e39 each
+    elif case == "far overflow":
+        q[..., 128], rot[:, :first, 0] = 1.2345e35, -3.21e30
+    elif case == "infinite row":
+        rot[:, :first, 2] = float("-inf")
+        q[:, 7, 1, 130] = -1.25                            # query 7 of head 1: +infinity
+    else:
+        q, rot = q * 300, rot * 3                          # scores of about +-1e4
+    rot[:, first:, 0] = 0
+    got = attn._expanded(q, lat[0], rot[0], 192 ** -0.5, None)[0].view(T, heads, 128)
+    kb = kv_b.double().view(heads, 256, 512).cpu()
+    ld, rd, qd = lat[0].double().cpu(), rot[0].double().cpu(), q[0].double().cpu()
+    keys, values = torch.matmul(ld, kb[:, :128].transpose(1, 2)), torch.matmul(ld, kb[:, 128:].transpose(1, 2))   # [H, Tk, 128]
+    qh = qd.transpose(0, 1)
+    s = (torch.matmul(qh[..., :128], keys.transpose(1, 2)) + qh[..., 128:] @ rd.T).float().double()
+    mask = torch.arange(Tk)[None] > torch.arange(past, Tk)[:, None]
+    p = torch.softmax((s * 192 ** -0.5).masked_fill(mask, float("-inf")), -1)
+    want = torch.matmul(p, values).transpose(0, 1)
+    bad = torch.isnan(want).all(-1)
+    assert bad.sum() == (1 if case == "infinite row" else 0) and torch.isnan(want).any(-1).equal(bad)
+    got = got.double().cpu()
+    assert torch.isnan(got).all(-1).equal(bad) and torch.isfinite(got[~bad]).all()
+    # fp32 scores of S are off by a few 2^-24 S of their largest partial sums (S up to 2e4 in "large"), and so
+    # are the logarithms of the weights
+    tol = 2e-2 if case == "large" else 1e-4
+    assert float((got - want)[~bad].abs().max()) <= tol * float(want[~bad].abs().max())
