@@ -896,7 +896,7 @@ def main():
             "pct_hbm_peak": round(100 * pbytes / pst / 1e9 / HBM_PEAK_GBS, 1), "bytes": pbytes,
             "useful_TFLOP/s": round(PF_FLOPS / pst / 1e12, 1),
             "mfma": "v_mfma_f32_16x16x32_bf16 (MXFP4 decoded to bf16 in registers; act as two bf16 terms)",
-            "pct_fp8_mfma_peak": round(100 * PF_FLOPS / pst / 5.0e15, 1),
+            "pct_bf16_mfma_peak": round(100 * PF_FLOPS / pst / 2.5e15, 1),
             "tokens": PF_T, "top_k": PF_K, "experts": E_LAYER, "routing": "zipf(1.1), seeded",
             "expert_load": {"max": int(counts.max()), "mean": round(float(counts.mean()), 1),
                             "empty": int((counts == 0).sum())},

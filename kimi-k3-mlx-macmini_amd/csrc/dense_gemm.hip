@@ -19,7 +19,8 @@
 // 400 -> 314 us (1.12 PFLOP/s executed), 256 x 7168 x 12288 347 -> 141 us, 16 x 7168 x 8192 104 -> 33 us;
 // bf16 a, six matrices of 49,376 rows in all at K 7168: 2 tokens 153 -> 120 us (5.9 TB/s), 256 tokens
 // 349 -> 217 us.  What bounds it: the matrix cores at the clock they hold under load (46% busy by
-// counter, LDS 24%, no bank conflicts) and, at few tokens, HBM.
+// counter, LDS 24%, no bank conflicts), CUs without a tile where the tiles are more than half the
+// CUs and no multiple of them (make_plan) and, at few tokens, HBM.
 #include <algorithm>
 #include <type_traits>
 
@@ -327,7 +328,9 @@ struct Plan {
     int bm, mt, ksplit, ksteps;
 };
 // BM: the smallest tile that takes M in one, 128 (bf16 a: 256) above.  ksplit: enough blocks
-// for every CU, in pieces of at least four steps.
+// for every CU, in pieces of at least four steps.  A tile is never shared by two blocks once there
+// are more than 128, so 1000 tokens against 8192 + 1536 + 576 rows are 164 blocks (64% of the CUs),
+// 700 against 7168 168, 256 against 4 x 12,288 192, 1000 against 12,288 384 in two turns (75%).
 Plan make_plan(int64_t M, int64_t K, int nt, bool f32) {
     Plan p{};
     p.bm = M <= 32 ? 32 : (M <= 64 ? 64 : (M <= 128 || f32 ? 128 : 256));

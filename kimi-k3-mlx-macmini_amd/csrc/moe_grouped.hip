@@ -1,6 +1,8 @@
 // Grouped routed-expert FFN for many tokens (prefill): every routed (token, slot) pair is
 // grouped by expert and each expert runs as a GEMM with M = its token count on the bf16
-// matrix cores, so each expert's MXFP4 weights stream from HBM once.
+// matrix cores.  Each expert's MXFP4 weights are read once per 64-token tile; the tiles of an expert
+// run side by side on one XCD, so most repeats come from its L2 (2048 tokens over 896 experts, 520
+// of them reached, in 845 tiles: 7.0 GB fetched for gate and up, of 6.1 GB of weights).
 //
 // Reference: LatentMoE.__call__ (air_llm/models/kimi_k3/moe.py:110-132; k3ref
 // k3ref/layers.py:241-261): for each distinct routed expert, gather its tokens, run
@@ -132,8 +134,9 @@ __device__ __forceinline__ void bf16_split2(float v, uint16_t &hi, uint16_t &lo)
 }
 
 // The activation of moe_common.h's act_fn in straight-line code on the hardware's exp2 and
-// reciprocal (each within one unit in the last place): about 1e-6 relative, against the 2^-17
-// its two-term storage keeps.
+// reciprocal (each within one unit in the last place).  The exponent's rounding enters the result
+// by its size: about 1e-6 relative up to |x| of 20, 4e-6 at 80, against the 2^-17 (7.6e-6) that the
+// two-term storage keeps.
 __device__ __forceinline__ float fast_sigmoid(float x) {
     return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * x));
 }

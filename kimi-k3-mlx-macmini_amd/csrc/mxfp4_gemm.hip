@@ -60,12 +60,12 @@ __global__ __launch_bounds__(kThreads, 2) void mxfp4_gemm_kernel(GemvArgs a) {
     const int nrows = static_cast<int>(a.N - n0 < Sh::R ? a.N - n0 : Sh::R), mrows = min(16 * TT, a.M - m0);
 
     // ---- loads.  x: KC * element size bytes per row and step, 16-byte chunks
-    constexpr int ES = TERMS == 1 ? 2 : 4, XC = KC * ES / 16;        // chunks per x row: 32
+    constexpr int ES = TERMS == 1 ? 2 : 4, XC = KC * ES / 16;        // chunks per x row: 32 to 128
     constexpr int XR = kThreads / XC, NX = 16 * TT / XR;             // rows per pass, passes
     const int xc = tid % XC, xr = tid / XC;
     const auto rx = make_rsrc(static_cast<const char *>(a.x) + static_cast<int64_t>(m0) * a.ldx * ES,
                               static_cast<uint32_t>(static_cast<int64_t>(mrows) * a.ldx * ES));
-    constexpr int WC = KC / 32;                                      // 16-byte chunks per weight row: 8 or 4
+    constexpr int WC = KC / 32;                                      // 16-byte chunks per weight row: 4 to 32
     const int wc = tid % WC, wrow = tid / WC;                        // rows past R: no load
     const uint32_t row_bytes = static_cast<uint32_t>(K >> 1);
     const auto rw = make_rsrc(static_cast<const char *>(a.packed) + n0 * row_bytes, static_cast<uint32_t>(nrows) * row_bytes);

@@ -322,7 +322,7 @@ def test_latent_moe_unfused_bf16_matches_fused():
 def test_latent_moe_fp32_hidden_states(T):
     """fp32 x that is not bf16-exact: the decode kernel (T <= 8) routes on x and keeps the
     latent state in fp32; the grouped path (T = 12) routes on the unrounded x and feeds
-    the fp32 latent state to the MFMA GEMM as three E4M3 terms."""
+    the fp32 latent state to the MFMA GEMM as two bf16 terms."""
     from k3hip.moe import LatentMoE
     cfg = K3Cfg()
     w, source, args = make_latent(70 + T, cfg)

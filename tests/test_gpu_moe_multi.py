@@ -240,7 +240,9 @@ def test_routed_moe_few_tokens_and_prefill_dispatch(router, xdt, Is):
     which = {"w1": 0, "w3": 1, "w2": 2}
     moe = RoutedMoE(cfg, 0, w, lambda L, e, wh: ex_dev[e][which[wh]])
     experts = {e: ex_np[e] for e in range(E)}
-    for T, tol in ((1, TOL), (2, TOL), (4, TOL), (8, TOL), (12, 5e-4)):
+    # the grouped path (12 tokens) keeps 16 bits of an fp32 x: 2^-17 of a value, which SiTU's exponential
+    # multiplies by the size of its argument (4.1e-5 observed; 2.9e-6 for bf16 x)
+    for T, tol in ((1, TOL), (2, TOL), (4, TOL), (8, TOL), (12, TOL if xdt == torch.bfloat16 else 1e-4)):
         x32 = rng.standard_normal((T, H)).astype(np.float32)
         if xdt == torch.bfloat16:
             x32 = om.bf16_round(x32)
