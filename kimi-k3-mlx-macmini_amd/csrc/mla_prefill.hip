@@ -24,8 +24,8 @@
 //              softmax in the very order the context product takes them.
 // What bounds it: the six-fold products (1.3e11 at 1000 tokens and 64 heads, about 100 us of the
 // matrix cores) beside LDS reads of 52 KB per wave and step, with two waves per SIMD to overlap
-// a step's scores, softmax and context.  Measured at 1000 tokens, 64 heads: attention 141 us,
-// expansion 57 us; the fp32 absorbed form in library products took 1.9 ms with its passes.
+// a step's scores, softmax and context.  Measured at 1000 tokens, 64 heads: attention 147 us,
+// expansion 59 us; the fp32 absorbed form in library products took 1.9 ms with its passes.
 #include <algorithm>
 
 #include "k3_common.h"

@@ -219,8 +219,8 @@ struct GemmArgs {
 // reads what another one does.  Weights become bf16 in registers (4 v_cvt per 8 values of
 // a row, reused by the tile's column groups and both terms).
 // Measured (2048 tokens, 896 experts top-16, latent 3584 / 3072; the former form fed the scaled
-// FP4 x FP8 MFMA in operand order): gate/up 4470 -> 2840 us, down 2366 -> 1930 us; 700 tokens over
-// 384 experts: 1850 -> 1270 and 1208 -> 860 us.  What bounds it now: a step costs a barrier, the
+// FP4 x FP8 MFMA in operand order): gate/up 4470 -> 2790 us, down 2366 -> 1970 us; 700 tokens over
+// 384 experts: 1850 -> 1340 and 1208 -> 960 us under the profiler.  What bounds it now: a step costs a barrier, the
 // LDS round trip and the products in turn, 1.2 us at one column group (its weights take 1.2 us
 // of HBM), 1.6 at three, 1.9 at four (matrix cores busy 28% in gate/up, 39% in down).  Measured
 // and not kept: the two wave groups half a beat apart (gate/up 3030 -> 3940 us: too little work

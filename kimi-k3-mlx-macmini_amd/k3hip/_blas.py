@@ -95,15 +95,25 @@ def dense(a: torch.Tensor, ws, add: torch.Tensor | None = None) -> list[torch.Te
 
 def one_launch(M: int, K: int, rows: list[int]) -> bool:
     """Whether one k3_dense launch takes several bf16 matrices against M bf16 tokens (one matrix-core
-    pass) sooner than a library GEMM each.  Up to 64 tokens it does at every set measured, weights not
-    yet cached (library / k3_dense us): 1536 + 576 + 8192 rows of 7168 2 tokens 48.6 / 36.1, 64 tokens
-    64 / 41; 512 + 512 of 1024 11.2 / 10.5; 4 x 12,288 + 224 of 7168 163 / 130; at worst 6144 + 6144 of
-    7168, 2 tokens 40.2 / 42.0.  Beyond, its K split costs small sets more than the launches it saves:
-    512 + 512 of 1024, 256 tokens 15.9 / 21.6; 2048 + 2048 of 2048 (8.4 million weights) 23.5 / 29.2; but
-    three matrices, 768 + 576 + 2048 of 2048 (6.9 million), 33.5 / 29.7, 1536 + 576 of 7168 (15 million)
-    43.4 / 37.9, 2048 + 2048 of 7168, 700 tokens 82.7 / 66.9.  Beyond 1024 tokens neither leads throughout (1536 + 576 + 8192 of 7168, 1500
-    tokens 236 / 193, 2048 tokens 288 / 343)."""
-    return len(rows) > 1 and (M <= 64 or (M <= 1024 and len(rows) * sum(rows) * K >= 20_000_000))
+    pass) sooner than a library GEMM each.  Measured at 559 points, weights not yet cached (M 2..1100, K
+    1024..7168, 2 to 4 matrices of 512 to 12,288 rows), it picks the sooner one within 11%
+    (library / k3_dense us):
+
+    * up to 64 tokens it does throughout: 1536 + 576 + 8192 rows of 7168 at 2 tokens 48.6 / 36.1, 512 + 512 of
+      1024 11.2 / 10.5; at worst 6144 + 6144 of 7168 at 2 tokens 40.2 / 42.0;
+    * to 1024 tokens for three matrices or more, whose launches add up (768 + 576 + 2048 of 2048 at 256 tokens
+      33.5 / 29.7), and for long rows, whose K it splits over blocks (2048 + 2048 of 7168 at 700 tokens 82.7 /
+      66.9); two matrices of short rows are shorter on the library (2048 + 2048 of 2048 at 256 tokens 23.5 /
+      29.2, 5632 + 5632 of 2048 35.0 / 48.8);
+    * between, for wide matrices to 256 tokens (4096 + 4096 of 4096 at 192 tokens 66.4 / 43.0; at 384 51.4 /
+      55.4) and any but the smallest to 128 (3200 + 3200 of 2560 at 102 tokens 29.2 / 24.7; 768 + 576 of 2048
+      at 128 16.3 / 18.4);
+    * beyond 1024 tokens neither leads (1536 + 576 + 8192 of 7168 at 1500 tokens 236 / 193, at 2048 288 / 343)."""
+    if len(rows) < 2 or M > 1024:
+        return False
+    widest = max(rows)
+    return (M <= 64 or len(rows) > 2 or K >= 4800 or (M <= 256 and 3000 <= K <= 1.25 * widest)
+            or (M <= 128 and sum(rows) * K >= 4_000_000 and widest <= 2 * K))
 
 
 def project(a: torch.Tensor, ws) -> list[torch.Tensor]:

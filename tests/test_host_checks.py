@@ -240,7 +240,10 @@ PROJECTIONS = [(7168, [1536, 576, 8192], 2, 48.6, 36.1), (7168, [1536, 576, 8192
                (1024, [512, 512], 256, 15.9, 21.6), (1024, [512, 512], 1000, 17.3, 28.2), (2048, [768, 576], 64, 15.9, 14.6),
                (2048, [768, 576], 192, 16.4, 25.5), (2048, [2048, 2048], 32, 22.4, 15.5), (2048, [2048, 2048], 384, 25.8, 35.4),
                (4096, [1024, 1024], 256, 25.0, 29.0), (7168, [1024, 1024], 256, 38.2, 36.4), (7168, [2048, 2048], 700, 82.7, 66.9),
-               (7168, [3072, 3072], 1000, 129.9, 117.1)]
+               (7168, [3072, 3072], 1000, 129.9, 117.1), (2048, [5632, 5632], 274, 35.0, 48.8), (1536, [3328, 3328], 172, 22.4, 29.9),
+               (1280, [5248, 5248], 95, 19.4, 23.5), (2560, [3200, 3200], 102, 29.2, 24.7), (4096, [4096, 4096], 192, 66.4, 43.0),
+               (4096, [4096, 4096], 384, 51.4, 55.4), (3328, [640, 640], 167, 19.8, 28.0), (5888, [768, 768], 1000, 56.7, 43.4),
+               (2048, [768, 576], 128, 16.3, 18.4)]
 
 
 @pytest.mark.parametrize("K,rows,M,library,launch", PROJECTIONS)
