@@ -308,20 +308,26 @@ class MLAAttention:
           few the queries; then every head is a chain of Tk / 32 steps per 128 queries, 1.7 us a
           step (1.75) where at most 64 of the 128 are there and 2.4 (2.6) else, 256 chains at a time, a
           group of heads (what its scratch holds) after the other;
-        * masked (fp32 library products): its launches (205), the passes over
-          the cache (0.52 ns a head and position) or 28 ps a head, query and position, whichever is most.
+        * masked (fp32 library products): 205 of launches, or the passes over the cache (0.33 ns a head and
+          position and 68 us of launches, for every chunk of queries whose scores fit) and 23 ps a head, query
+          and position, fitted over even and odd sizes.
 
         64 heads, bf16 cache, masked / expanded: 16 queries over 1024 positions 220 / 115, 4096 247 / 443,
         32,768 1488 / 8852; 128 queries over 4096 939 / 545, 16,384 3589 / 3366, 32,768 7678 / 11,984; 256
-        over 32,768 15,225 / 11,969.  fp32 cache: 2 queries over 2048 203 / 269, 128 over 4096 935 / 661.
-        16 heads: 128 queries over 4096 336 / 376, 256 558 / 376."""
+        over 32,768 15,225 / 11,969.  fp32 cache: 2 queries over 2048 203 / 269, 128 over 4096 935 / 661; 96
+        heads, 70 over 918 448 / 189.  16 heads: 128 queries over 4096 336 / 376, 256 558 / 376.  At 396 of
+        397 measured points the form it picks is within 9% of the shorter one (192 queries over 32,768
+        positions of an fp32 cache: 13,865 for 11,501)."""
         heads = self.cfg.num_attention_heads
         padded = _round_up(Tk, 32)
         group = _lib.size("k3_mla_prefill_workspace_size", Tk, heads) // (padded * 2 * 3 * 2 * 128)
         turns = -(-group * -(-Tn // 128) // 256) * -(-heads // group)
         step = (1.75 if f32 else 1.7) if Tn <= 64 else (2.6 if f32 else 2.4)
         expanded = (1.55e-3 if f32 else 8.9e-4) * Tk * heads + turns * padded / 32 * step
-        return expanded < max(205.0, 5.2e-4 * Tk * heads, 2.8e-5 * Tn * Tk * heads)
+        chunks = -(-Tn // max(1, self.DENSE_SCORE_BYTES // (heads * Tk * 4)))
+        masked = (chunks * (68 + 3.27e-4 * Tk * heads) + 2.25e-5 * Tn * Tk * heads + 0.0144 * Tn * heads
+                  + 0.0065 * Tk)
+        return expanded < (masked ** 4 + 205 ** 4) ** 0.25
 
     def _expanded_ok(self, q, lat, rot) -> bool:
         c = self.cfg

@@ -198,7 +198,9 @@ MLA_FORMS = [(64, False, 256, 2, 218, 51), (64, False, 1024, 16, 220, 115), (64,
              (64, False, 65536, 192, 32909, 44087), (64, True, 1024, 16, 203, 148), (64, True, 2048, 2, 203, 269),
              (64, True, 4096, 16, 236, 544), (64, True, 4096, 128, 935, 661), (64, True, 32768, 48, 3361, 10594),
              (16, False, 1024, 8, 214, 92), (16, False, 4096, 128, 336, 376), (16, False, 4096, 256, 558, 376),
-             (16, False, 32768, 16, 539, 2205), (16, False, 32768, 256, 3647, 2974)]
+             (16, False, 32768, 16, 539, 2205), (16, False, 32768, 256, 3647, 2974), (96, True, 918, 70, 448, 189),
+             (96, False, 2904, 50, 614, 380), (64, True, 1637, 60, 344, 256), (8, False, 2784, 256, 318, 249),
+             (64, False, 44255, 337, 35996, 29605), (48, False, 37410, 119, 8902, 10215), (96, False, 6172, 5, 437, 777)]
 
 
 @pytest.mark.parametrize("heads,f32,Tk,T,masked,expanded", MLA_FORMS)
