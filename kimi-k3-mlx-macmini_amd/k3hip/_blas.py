@@ -51,7 +51,10 @@ def _rows_ok(w: torch.Tensor) -> bool:
 
 def weights_ok(*ws: torch.Tensor) -> bool:
     """k3_dense takes these weights as they are: bf16 device matrices of whole 16-byte rows."""
-    return not T.tracked(*ws) and all(map(_rows_ok, ws))
+    for w in ws:
+        if not _rows_ok(w):
+            return False
+    return not T.tracked(*ws)
 
 
 def dense_ok(a: torch.Tensor, *ws: torch.Tensor) -> bool:
@@ -93,36 +96,33 @@ def dense(a: torch.Tensor, ws, add: torch.Tensor | None = None) -> list[torch.Te
     return outs
 
 
-def one_launch(M: int, K: int, rows: list[int]) -> bool:
-    """Whether one k3_dense launch takes several bf16 matrices against M bf16 tokens (one matrix-core
-    pass) sooner than a library GEMM each.  Measured at 559 points, weights not yet cached (M 2..1100, K
-    1024..7168, 2 to 4 matrices of 512 to 12,288 rows), it picks the sooner one within 11%
-    (library / k3_dense us):
+def one_launch(M: int, n: int) -> bool:
+    """Whether one k3_dense launch takes n bf16 matrices against M bf16 tokens (one matrix-core pass)
+    instead of a library GEMM each.
 
-    * up to 64 tokens it does throughout: 1536 + 576 + 8192 rows of 7168 at 2 tokens 48.6 / 36.1, 512 + 512 of
-      1024 11.2 / 10.5; at worst 6144 + 6144 of 7168 at 2 tokens 40.2 / 42.0;
-    * to 1024 tokens for three matrices or more, whose launches add up (768 + 576 + 2048 of 2048 at 256 tokens
-      33.5 / 29.7), and for long rows, whose K it splits over blocks (2048 + 2048 of 7168 at 700 tokens 82.7 /
-      66.9); two matrices of short rows are shorter on the library (2048 + 2048 of 2048 at 256 tokens 23.5 /
-      29.2, 5632 + 5632 of 2048 35.0 / 48.8);
-    * between, for wide matrices to 256 tokens (4096 + 4096 of 4096 at 192 tokens 66.4 / 43.0; at 384 51.4 /
-      55.4) and any but the smallest to 128 (3200 + 3200 of 2560 at 102 tokens 29.2 / 24.7; 768 + 576 of 2048
-      at 128 16.3 / 18.4);
-    * beyond 1024 tokens neither leads (1536 + 576 + 8192 of 7168 at 1500 tokens 236 / 193, at 2048 288 / 343)."""
-    if len(rows) < 2 or M > 1024:
-        return False
-    widest = max(rows)
-    return (M <= 64 or len(rows) > 2 or K >= 4800 or (M <= 256 and 3000 <= K <= 1.25 * widest)
-            or (M <= 128 and sum(rows) * K >= 4_000_000 and widest <= 2 * K))
+    On the device (weights not yet cached, library / k3_dense us) it is shorter up to 64 tokens (1536 +
+    576 + 8192 rows of 7168 at 2 tokens 48.6 / 36.1, at 64 64 / 41; 512 + 512 of 1024 11.2 / 10.5; at worst
+    6144 + 6144 of 7168 at 2 tokens 40.2 / 42.0), for three matrices or more (768 + 576 + 2048 of 2048 at 256
+    tokens 33.5 / 29.7) and for long rows, whose K it splits over blocks (2048 + 2048 of 7168 at 700 tokens
+    82.7 / 66.9).  Two matrices of short rows are shorter on the library beyond 64 tokens, by 14 us
+    at most of 559 measured points (512 + 512 of 1024 at 1000 tokens 17.3 / 28.2, 5632 + 5632 of 2048 at 274
+    35.0 / 48.8).  But every library call costs the host more than that, and a layer of such sizes
+    waits for the host: 162 tokens through a layer with 1024 + 1024 rows of 1792 140.5 us with one
+    launch, 166.7 with two library calls.  Beyond 1024 tokens neither leads (1536 + 576 + 8192 of 7168 at 1500
+    tokens 236 / 193, at 2048 288 / 343) and the library stays."""
+    return n > 1 and M <= 1024
 
 
-def project(a: torch.Tensor, ws) -> list[torch.Tensor]:
+def project(a: torch.Tensor, ws, checked: bool = False) -> list[torch.Tensor]:
     """[a [M, K] @ w[N, K]^T in fp32 for w in ws], all against one activation: fp32 a in one k3_dense
     launch (three library products a matrix were slower at every size measured, 2 to 2048 tokens of
-    64 to 12,288 rows); bf16 a where one_launch holds, on the library elsewhere."""
-    M = a.shape[0]
-    if M and dense_ok(a, *ws) and (a.dtype == torch.float32 or one_launch(M, a.shape[1], [w.shape[0] for w in ws])):
-        return dense(a, list(ws))
+    64 to 12,288 rows); bf16 a where one_launch holds, on the library elsewhere.  checked: weights_ok
+    holds for ws, and a is a device tensor of either type that nothing is asked of (tracked)."""
+    M, K = a.shape
+    if M and (a.dtype == torch.float32 or one_launch(M, len(ws))):
+        dev = a.get_device()
+        if all(w.shape[1] == K and w.get_device() == dev for w in ws) if checked else dense_ok(a, *ws):
+            return dense(a, list(ws))
     return [mm_f32(a, w) for w in ws]
 
 

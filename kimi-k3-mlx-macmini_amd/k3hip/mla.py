@@ -196,11 +196,10 @@ def _rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
 def _rmsnorm_rows(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
     """_rmsnorm of the rows of an fp32 [M, K] device tensor in one launch."""
     M, K = x.shape
-    if (tuple(w.shape) != (K,) or M > _blas.MAX_ROWS or K % 4 or x.stride(1) != 1 or x.stride(0) % 4 or x.data_ptr() % 16 or M == 0
-            or T.tracked(x, w)):
+    if (w.shape != (K,) or w.get_device() != x.get_device() or not 0 < M <= _blas.MAX_ROWS or K % 4 or x.stride(1) != 1
+            or x.stride(0) % 4 or x.data_ptr() % 16 or T.tracked(x, w)):
         return _rmsnorm(x, w, eps)   # (which refuses or broadcasts a w of another shape)
     w = T.contiguous_aligned(w.to(torch.float32))
-    T.require_device(x, w)
     out = torch.empty((M, K), dtype=torch.float32, device=x.device)
     _lib.call("k3_rmsnorm_rows", T.ptr(x), x.stride(0) if M > 1 else K, T.ptr(w), float(eps), T.ptr(out), M, K, T.stream(x))
     return out
@@ -266,9 +265,9 @@ class MLAAttention:
         rest = [self.q_an, self.kv_an, self.kv_b] + ([] if cache is None else [cache.latent, cache.rot])
         if (B * Tn > 1 and _blas.dense_ok(xf, *mats) and _blas.weights_ok(self.q_b, self.o_w)
                 and not T.tracked(*rest)):
-            qa, ckv, *g = _blas.project(xf, mats)
+            qa, ckv, *g = _blas.project(xf, mats, checked=True)
             qa = _rmsnorm_rows(qa, self.q_an, eps)
-            q = _blas.project(qa, [self.q_b])[0].reshape(B, Tn, nh, qhd)
+            q = _blas.project(qa, [self.q_b], checked=True)[0].reshape(B, Tn, nh, qhd)
             c_new = _rmsnorm_rows(ckv[:, :klr], self.kv_an, eps).reshape(B, Tn, klr)
             r_new = ckv[:, klr:].reshape(B, Tn, -1)
             gate = g[0].reshape(B, Tn, nh * vhd) if gated else None
@@ -319,6 +318,8 @@ class MLAAttention:
         397 measured points the form it picks is within 9% of the shorter one (192 queries over 32,768
         positions of an fp32 cache: 13,865 for 11,501)."""
         heads = self.cfg.num_attention_heads
+        if Tk <= 512 and Tk * heads <= 1 << 15:     # (expanded: 93 at most)
+            return True
         padded = _round_up(Tk, 32)
         group = _lib.size("k3_mla_prefill_workspace_size", Tk, heads) // (padded * 2 * 3 * 2 * 128)
         turns = -(-group * -(-Tn // 128) // 256) * -(-heads // group)
@@ -353,7 +354,7 @@ class MLAAttention:
         q = T.contiguous_aligned(q)
         gate = None if gate is None else T.contiguous_aligned(gate)
         out = torch.empty((1, Tn, nh * vhd), dtype=torch.float32, device=q.device)
-        nbytes = int(_lib.lib().k3_mla_prefill_workspace_size(lat.shape[0], nh))
+        nbytes = _lib.size("k3_mla_prefill_workspace_size", lat.shape[0], nh)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)   # the call's own, as the scores of _dense
         _lib.call("k3_mla_prefill", T.ptr(q), nh * c.q_head_dim, T.ptr(self.kv_b), T.ptr(lat), lat.stride(0), T.ptr(rot),
                   rot.stride(0), T.dtype_code(lat.dtype), T.ptr(gate), T.ptr(out), Tn, lat.shape[0], nh, c.kv_lora_rank,

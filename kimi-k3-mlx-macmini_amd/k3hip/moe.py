@@ -276,7 +276,7 @@ class RoutedMoE:
         if (self.fused and flat.shape[0] and self.sh_gate.shape == self.sh_up.shape and _blas.dense_ok(flat, *mats)
                 and _blas.weights_ok(self.sh_down) and self.sh_down.shape[1] == self.sh_gate.shape[0]
                 and self.sh_down.device == flat.device and not T.tracked(add)):
-            g, u = _blas.project(flat, mats)
+            g, u = _blas.project(flat, mats, checked=True)
             _lib.call("k3_act_rows", T.ptr(g), T.ptr(u), T.ptr(g), g.numel(), _act_code(act), float(beta),
                       float(lb or 0.0), T.stream(g))
             return _blas.dense(g, [self.sh_down], add)[0].reshape(x.shape)
@@ -419,10 +419,10 @@ def _rmsnorm32(y: torch.Tensor, w32: torch.Tensor, eps: float) -> torch.Tensor:
 def _rmsnorm_rows(y: torch.Tensor, w32: torch.Tensor, eps: float) -> torch.Tensor:
     """_rmsnorm32 of the contiguous rows of an fp32 [M, K] device tensor in one launch."""
     M, K = y.shape
-    if (M == 0 or M > _blas.MAX_ROWS or K % 4 or not y.is_contiguous() or y.data_ptr() % 16 or w32.data_ptr() % 16 or y.dtype != torch.float32
-            or tuple(w32.shape) != (K,) or T.tracked(y, w32)):
+    if (w32.shape != (K,) or w32.get_device() != y.get_device() or not 0 < M <= _blas.MAX_ROWS or K % 4
+            or not y.is_contiguous() or y.data_ptr() % 16 or w32.data_ptr() % 16 or y.dtype != torch.float32
+            or T.tracked(y, w32)):
         return _rmsnorm32(y, w32, eps)
-    T.require_device(y, w32)
     out = torch.empty_like(y)
     _lib.call("k3_rmsnorm_rows", T.ptr(y), K, T.ptr(w32), eps, T.ptr(out), M, K, T.stream(y))
     return out

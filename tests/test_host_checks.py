@@ -235,26 +235,26 @@ def test_matvec_launches_of_refused_sizes():
     assert [f(0, 64, 64, 0), f(1, 64, 48, 0), f(1, 64, 1 << 20, 0), f(1, 64, 64, 7)] == [0] * 4
 
 
-# (K, rows of each matrix, tokens, library us, one launch us), weights not yet cached
-PROJECTIONS = [(7168, [1536, 576, 8192], 2, 48.6, 36.1), (7168, [1536, 576, 8192], 700, 154.5, 126.9),
-               (7168, [1536, 576, 8192], 2048, 287.8, 343.3), (2048, [768, 576, 2048], 64, 33.0, 18.3),
-               (2048, [768, 576, 2048], 256, 33.5, 29.7), (7168, [12288] * 4, 1500, 963, 900), (1024, [512, 512], 24, 11.4, 11.0),
-               (1024, [512, 512], 256, 15.9, 21.6), (1024, [512, 512], 1000, 17.3, 28.2), (2048, [768, 576], 64, 15.9, 14.6),
-               (2048, [768, 576], 192, 16.4, 25.5), (2048, [2048, 2048], 32, 22.4, 15.5), (2048, [2048, 2048], 384, 25.8, 35.4),
-               (4096, [1024, 1024], 256, 25.0, 29.0), (7168, [1024, 1024], 256, 38.2, 36.4), (7168, [2048, 2048], 700, 82.7, 66.9),
-               (7168, [3072, 3072], 1000, 129.9, 117.1), (2048, [5632, 5632], 274, 35.0, 48.8), (1536, [3328, 3328], 172, 22.4, 29.9),
-               (1280, [5248, 5248], 95, 19.4, 23.5), (2560, [3200, 3200], 102, 29.2, 24.7), (4096, [4096, 4096], 192, 66.4, 43.0),
-               (4096, [4096, 4096], 384, 51.4, 55.4), (3328, [640, 640], 167, 19.8, 28.0), (5888, [768, 768], 1000, 56.7, 43.4),
-               (2048, [768, 576], 128, 16.3, 18.4)]
-
-
-@pytest.mark.parametrize("K,rows,M,library,launch", PROJECTIONS)
-def test_projections_of_bf16_tokens_take_the_shorter_form(K, rows, M, library, launch):
-    """Both were measured at each of these; past 1024 tokens, where neither leads throughout, the
-    library is taken."""
+def test_projections_of_bf16_tokens(monkeypatch):
+    """Several matrices in one launch up to 1024 tokens; one matrix, and more tokens, on the library;
+    fp32 tokens in one launch always; and operands that do not match never reach the launch."""
     from k3hip import _blas
-    assert not _blas.one_launch(M, K, rows[:1])
-    assert _blas.one_launch(M, K, rows) == (launch < library and M <= 1024)
+    _no_device(monkeypatch, [])
+    took = []
+    monkeypatch.setattr(_blas, "dense", lambda a, ws, add=None: took.append("launch") or [a.float() @ w.float().t() for w in ws])
+    monkeypatch.setattr(_blas, "mm_f32", lambda a, w: took.append("library") or a.float() @ w.float().t())
+    w = [torch.zeros(16, 32, dtype=BF16)] * 2
+    for M, dt, ws, want in ((2, BF16, w, ["launch"]), (1024, BF16, w, ["launch"]), (1025, BF16, w, ["library"] * 2),
+                            (200, BF16, w[:1], ["library"]), (2000, torch.float32, w, ["launch"]),
+                            (7, torch.float32, w[:1], ["launch"])):
+        for checked in (False, True):
+            took.clear()
+            _blas.project(torch.zeros(M, 32, dtype=dt), ws, checked)
+            assert took == want
+    took.clear()
+    with pytest.raises(RuntimeError):
+        _blas.project(torch.zeros(3, 24), w, True)
+    assert "launch" not in took
 
 
 @pytest.mark.parametrize("B,T", [(1, 0), (2, 0), (0, 3)])
