@@ -182,6 +182,7 @@ int64_t k3_mla_prefill_workspace_size(int64_t Tk, int64_t heads);
  *   multiplies the result; out [T, heads * 128] fp32.
  * fp32 operands enter the bf16 matrix cores as three terms each, of whose nine products the three
  * smallest are left out (at most 2^-23 of a product, of either sign; 0.1 x 2^-24 rms); sums are fp32.
+ * A score of -infinity has weight zero; an infinite value that a query sees makes its result NaN.
  * Replaces the multi-token branch of MLAAttention.__call__ (attention_mla.py:193-214). */
 int k3_mla_prefill(const float *q, int64_t ldq, const void *kv_b, const void *lat, int64_t ld_lat,
                    const void *rot, int64_t ld_rot, int cache_dtype, const float *gate, float *out, int64_t T,

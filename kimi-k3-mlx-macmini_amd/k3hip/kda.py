@@ -6,7 +6,8 @@
 sequence is one ``k3_kda_step_decode`` (projections, short convolutions, norms, gate,
 recurrence, gated RMSNorm, o_proj in four launches); more take ``prefill``, which reads every
 weight once for all tokens: the projections (``_blas.project``), ``k3_kda_prefill_inputs``,
-one ``k3_kda_recurrent`` launch and ``k3_kda_gated_norm``.  The recurrent state is fp32
+one ``k3_kda_recurrent`` launch and ``k3_kda_gated_norm``.  For inference: no gradient passes
+through the recurrence, and the output carries none.  The recurrent state is fp32
 [B, H, 128, 128], updated in place; the convolution states come back as fp32 [B, k-1, C].
 
 ``kda_recurrent(q, k, v, g, beta, scale, state)`` takes the reference's tensors

@@ -19,8 +19,9 @@ bf16 projection weights (the checkpoint dtype) the decode step (one token, batch
 gate and o_proj in seven HIP launches.  With other weight dtypes the projections are torch
 fp32 matmuls around the HIP core.  Prefill (T > 1) runs the projections of all tokens
 (``_blas.project``) and the causal attention over keys and values expanded from the cache
-(``k3_mla_prefill``); fp32 weights, batches and other widths keep the reference's dense
-masked form in torch.
+(``k3_mla_prefill``); fp32 weights, batches, other widths, a few queries over a long cache
+(``_expand_pays``) and calls that a gradient or tangent is asked of keep the reference's
+dense masked form in torch.
 
 The cache defaults to bf16 (``cfg.mla_cache_dtype``), which the HIP core reads in place; the
 reference's default is an fp32 cache (``attention_mla.py:164``), which it calls lossless.
